@@ -182,8 +182,9 @@ def c3_run(ctx, max_passes=40):
             dt = time.perf_counter() - t0
         out[prec] = (rc, e, ks.result, dt)
     # the FP32 cell kernel on C3's operator at the filter's width with M^-1
-    # folded in (the degree loop's apply), 20 eager applies profiled per
-    # colour step (the solves above replay graphs, which are not profiled)
+    # folded in (the degree loop's apply), 20 eager applies profiled (the
+    # solves above replay graphs, which are not profiled): one record per
+    # apply on the slot path, per colour step on the colour path
     info = H.info()
     X = dfx.MultiVector(ctx, N, n, dfx.F32)
     X.fill_random(3, -1.0, 1.0)
@@ -197,14 +198,15 @@ def c3_run(ctx, max_passes=40):
     pr = H.profile(reset=True)
     H.set_profiling(False)
     nrows = len(prob.get("rows"))
-    fl = 2.0 * n * info["sumNe2"] / info["nColors"]
+    units = max(pr["launches"], 1) / 20
+    fl = 2.0 * n * info["sumNe2"] / units
     by = (4.0 * info["sumNe2"] + 4.0 * (info["sumNe"] + info["nCells"]) + 2.0 * 4 * N * n +
-          4.0 * 2 * nrows + 4.0 * nrows * n) / info["nColors"]
+          4.0 * 2 * nrows + 4.0 * nrows * n) / units
     ms = pr["kernelMs"] / max(pr["launches"], 1)
     t_m, t_h = fl / (PEAK_FP32_MFMA * 1e12), by / (PEAK_HBM * 1e9)
     ach = fl / (ms * 1e-3) / 1e12 if ms else 0.0
     c3_roof = {"bound": "mfma" if t_m > t_h else "hbm", "kernel": "cellApplyBufK<float> "
-               "(M^-1 folded), one colour step per launch unit",
+               "(M^-1 folded) and its row sums, %g launch units per apply" % units,
                "achieved_tflops": ach, "frac_of_fp32_mfma_peak": ach / PEAK_FP32_MFMA,
                "achieved_gbps": by / (ms * 1e-3) / 1e9 if ms else 0.0,
                "frac_of_hbm_peak": (by / (ms * 1e-3) / 1e9 / PEAK_HBM) if ms else 0.0,

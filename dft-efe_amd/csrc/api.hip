@@ -47,11 +47,82 @@ namespace dfx
   // rf (with dsc): the residual Chebyshev step fused in; Y then holds
   // partial sums on the rows the cells finish, and res is complete on
   // return (the listed remaining rows by a separate step)
+  // Whether an apply of B columns takes the slot path (all cells of a size
+  // class in one launch, their products to map slots, then the row sums)
+  // rather than one launch per colour and class.  The slot path writes and
+  // reads every cell's product once through memory where the colour path adds
+  // to Y in place; it pays for that by filling the GPU with one or two launches
+  // instead of eight or more.  The line lies where the slots' traffic wins
+  // that back.  Measured, slot against colour path (us per apply): 12^3 cells
+  // at p = 3, FP64, 1 / 64 / 200 columns (1 / 64 / 201 MiB of slots) 34 / 79 /
+  // 273 against 89 / 133 / 311; 24^3 cells at p = 4, FP64, 64 / 128 / 200
+  // columns (0.9 / 1.7 / 2.7 GiB) 1071 / 2011 / 3486 against 1263 / 2075 / 3366;
+  // FP32, 64 / 128 / 200 columns (0.4 / 0.9 / 1.3 GiB) 548 / 995 / 1853 against
+  // 619 / 997 / 1799; per degree step of the residual filter 24^3 at p = 4
+  // FP32 72 / 128 columns 1071 / 1633 against 1216 / 1596.  Both paths give the
+  // same bits
+  template <class T>
+  bool slotPath(const dfx_op *op, View<const T> X)
+  {
+    const u64 bytes = op->sumNe * X.B * sizeof(T);
+    return op->slotsOk && bytes <= SLOT_BYTES && k::slotAddressable<T>(op, X);
+  }
+
+  template <class T>
+  void applySlots(dfx_op *op, View<T> X, View<T> Y, const double *dsc, const T *xe, bool skipP2C,
+                  const k::ResFuse<T> *rf)
+  {
+    hipStream_t s = op->ctx->stream;
+    // rows held at zero are masked in the gather and cleared in X and Y by
+    // the row sums; other constraints take launches of their own
+    const bool mask = op->zeroRows && !skipP2C;
+    if (!dsc && !skipP2C && !op->zeroRows)
+      k::p2c<T>(s, op->cons, X);
+    if (op->yE.ensure((size_t)op->sumNe * X.B * sizeof(T)))
+      ++op->gen;
+    T            *slots = op->yE.as<T>();
+    const T      *frag  = fragOf<T>(op);
+    View<const T> Xc{X.p, X.N, X.B, X.ld};
+    const bool    prof = op->profiling && (op->profMask & (sizeof(T) == 8 ? 1 : 2)) &&
+                      (op->profApplies++ % op->profEvery) == 0;
+    ProfRec r{};
+    auto    event = [&] {
+      hipEvent_t e = nullptr;
+      DFX_HIP(hipEventCreate(&e));
+      op->profEvents.push_back(e);
+      DFX_HIP(hipEventRecord(e, s));
+      return e;
+    };
+    if (prof)
+      r.a = event();
+    for (const Launch &l : sizeof(T) == 8 ? op->slotLaunches64 : op->slotLaunches32)
+      {
+        k::cellSlots<T>(s, op, l, frag, Xc, slots, dsc, xe, mask);
+        const double B = X.B, sz = sizeof(T);
+        // cell matrices and the map once, rows of X gathered, slots written
+        // and read back, Y written
+        r.flops += 2.0 * B * (double)l.sumN2;
+        r.bytes += sz * (double)l.sumN2 + 4.0 * (double)l.sumN + 3.0 * sz * B * (double)l.sumN +
+                   (dsc ? 8.0 * (double)l.sumNc : 0.0);
+      }
+    r.bytes += sizeof(T) * (double)X.B * op->nDofs;
+    k::slotSum<T>(s, op, slots, X, Y, mask && !rf, rf);
+    if (prof) // one record per apply
+      {
+        r.b = event();
+        op->prof.push_back(r);
+      }
+    if (!rf && !op->zeroRows)
+      k::c2p<T>(s, op->cons, Y);
+  }
+
   template <class T>
   void applyCellwise(dfx_op *op, View<T> X, View<T> Y, const double *dsc = nullptr,
                      const T *xe = nullptr, bool skipP2C = false, T *yEOverride = nullptr,
                      const k::ResFuse<T> *rf = nullptr)
   {
+    if (!yEOverride && slotPath<T>(op, View<const T>{X.p, X.N, X.B, X.ld}))
+      return applySlots<T>(op, X, Y, dsc, xe, skipP2C, rf);
     hipStream_t s = op->ctx->stream;
     if (!dsc && !skipP2C)
       k::p2c<T>(s, op->cons, X);
@@ -167,28 +238,32 @@ namespace dfx
   // launches (all colours, one stream) per candidate width on zeroed scratch
   // multivectors and keep the fastest.  Candidates: 1, 2, 4, 8 tiles of 16
   // columns up to twice the columns there are, 5 for FP32 with 65..80
-  // columns, and only tiles that fit the LDS of a CU.  Per-column results do
+  // columns, 3 for slot launches of 33..48, and only tiles that fit the LDS of
+  // a CU; the launches timed are those of the path such an apply takes.  Per-column results do
   // not depend on the width (same K order per column), only the time does.
   template <class T>
   std::vector<std::pair<u32, int>> autotune(dfx_op *op, u32 B, u32 reps)
   {
     hipStream_t s    = op->ctx->stream;
-    const auto &L    = sizeof(T) == 8 ? op->launches64 : op->launches32;
     const T    *frag = fragOf<T>(op);
     const u32   N    = op->nDofs;
     DevBuf xb((size_t)N * B * sizeof(T)), yb((size_t)N * B * sizeof(T));
     DFX_HIP(hipMemsetAsync(xb.p, 0, xb.bytes, s));
     DFX_HIP(hipMemsetAsync(yb.p, 0, yb.bytes, s));
+    View<const T> X{xb.as<T>(), N, B, B};
+    View<T>       Y{yb.as<T>(), N, B, B};
+    const bool    buf   = k::cellBufferPath<T>(op, X, View<const T>{Y.p, N, B, B});
+    const bool    slots = slotPath<T>(op, X);
+    const auto   &L     = slots ? (sizeof(T) == 8 ? op->slotLaunches64 : op->slotLaunches32)
+                                : (sizeof(T) == 8 ? op->launches64 : op->launches32);
     T *yE = nullptr;
-    if (op->nEnrSlots)
+    if (op->nEnrSlots || slots)
       {
-        if (op->yE.ensure((size_t)op->nEnrSlots * B * sizeof(double)))
+        if (op->yE.ensure(slots ? (size_t)op->sumNe * B * sizeof(T)
+                                : (size_t)op->nEnrSlots * B * sizeof(double)))
           ++op->gen;
         yE = op->yE.as<T>();
       }
-    View<const T> X{xb.as<T>(), N, B, B};
-    View<T>       Y{yb.as<T>(), N, B, B};
-    const bool    buf = k::cellBufferPath<T>(op, X, View<const T>{Y.p, N, B, B});
     std::vector<u32> classes;
     for (const Launch &l : L)
       if (std::find(classes.begin(), classes.end(), l.mtw) == classes.end())
@@ -210,12 +285,15 @@ namespace dfx
             for (const Launch &l : L)
               if (l.mtw == c)
                 kpad = std::max(kpad, l.kpadMax);
-            const u32 rows = buf ? 64 * c : kpad; // K rows of the LDS tile
+            const u32 rows = buf || slots ? 64 * c : kpad; // K rows of the LDS tile
             int       best = 0;
             float     bestMs = 0.f;
-            for (int nt : {1, 2, 4, 5, 8})
+            for (int nt : {1, 2, 3, 4, 5, 8})
               {
                 if (nt == 5 && !(sizeof(T) == 4 && B > 64 && B <= 80))
+                  continue;
+                // three tiles: slot launches of 33..48 columns; eight: colour launches
+                if ((nt == 3 && !(slots && B > 32 && B <= 48)) || (nt == 8 && slots))
                   continue;
                 if (nt > 1 && 16u * nt > 2 * B)
                   continue;
@@ -223,7 +301,9 @@ namespace dfx
                   continue;
                 auto pass = [&] {
                   for (const Launch &l : L)
-                    if (l.mtw == c)
+                    if (l.mtw == c && slots)
+                      k::cellSlots<T>(s, op, l, frag, X, yE, nullptr, nullptr, op->zeroRows, nt);
+                    else if (l.mtw == c)
                       k::cellApply<T>(s, op, l, frag, X, Y, yE, nullptr, nullptr, nt);
                 };
                 pass(); // first launch: kernel attributes, instruction cache
@@ -238,7 +318,7 @@ namespace dfx
                   best = nt, bestMs = ms;
               }
             if (!best)
-              best = k::builtinNT<T>(B, kpad);
+              best = slots ? k::slotNT<T>(B, kpad) : k::builtinNT<T>(B, kpad);
             op->tuned.push_back(dfx_op::Tuned{(u32)sizeof(T), B, c, best});
             out.emplace_back(c, best);
           }
@@ -284,9 +364,10 @@ namespace dfx
     if ((sizeof(T) == 4 && !A->hasF32) || X.N != A->nDofs || Y.N != A->nDofs ||
         S1.N != A->nDofs || S1.ld != X.ld || X.B != Y.B || S1.B != X.B)
       return false;
-    if (!k::cellBufferPath<T>(A, View<const T>{X.p, X.N, X.B, X.ld},
-                              View<const T>{Y.p, Y.N, Y.B, Y.ld}) ||
-        (reinterpret_cast<uintptr_t>(S1.p) & 15) != 0)
+    const bool slots = slotPath<T>(A, View<const T>{X.p, X.N, X.B, X.ld});
+    if (!slots && (!k::cellBufferPath<T>(A, View<const T>{X.p, X.N, X.B, X.ld},
+                                         View<const T>{Y.p, Y.N, Y.B, Y.ld}) ||
+                   (reinterpret_cast<uintptr_t>(S1.p) & 15) != 0))
       return false;
     hipStream_t s = A->ctx->stream;
     if (A->foldedUid != Dinv->uid)
@@ -299,7 +380,8 @@ namespace dfx
         A->foldedUid = Dinv->uid;
         ++A->gen;
       }
-    if (!rf)
+    // (the slot path takes X's constrained rows as 0 and clears them itself)
+    if (!rf && !(A->zeroRows && slots))
       k::p2c<T>(s, Dinv->cons, X);
     if (Dinv->nEnriched)
       k::enrichedBlock<T>(s, S1, Dinv->enrBlock.as<double>(),

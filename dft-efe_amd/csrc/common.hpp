@@ -254,6 +254,20 @@ namespace dfx
     u32 color    = 0; // launches of one colour touch disjoint classical dofs
   };
 
+  // a row that a gather takes as 0 (never a dof: nDofs <= 2^32 - 2)
+  constexpr u32 ROW_NONE = 0xffffffffu;
+
+  // a classical row's slots for the row sums of the slot apply: the first
+  // slot, and (count << 27) | offset of the others in slotRest; ROW_ZERO as
+  // the count: the row is held at zero
+  struct RowHead
+  {
+    u32 slot0, rest;
+  };
+  constexpr u32 ROW_ZERO = 31, ROW_COUNT_SHIFT = 27;
+  // slot bytes up to which an apply takes the slot path (see slotPath)
+  constexpr u64 SLOT_BYTES = 1ull << 30;
+
   // one profiled kernel launch
   struct ProfRec
   {
@@ -307,7 +321,14 @@ struct dfx_op
   // enriched partial reduction
   dfx::u32 nEnrSlots = 0;
   dfx::DevBuf enrSlotOffsets, enrSlots; // CSR over enriched dofs -> yE rows
-  dfx::DevBuf yE;                       // scratch, grows with B
+  dfx::DevBuf yE; // enriched partial rows or all slots of an apply, grows with B
+  // ----- slot apply: cells by (size class, caller order), all of a class in
+  // one launch; the map with the rows held at zero masked (zeroRows: the
+  // constraints are homogeneous Dirichlet ones on classical rows); per
+  // classical row its slots in launch order; the enriched dofs' map slots
+  bool slotsOk = false, zeroRows = false;
+  std::vector<dfx::Launch> slotLaunches64, slotLaunches32;
+  dfx::DevBuf metaSlots, slotMap, rowHeads, slotRest, enrMapSlots;
   // standalone gather / scatter (dof -> slots CSR, slots in cell order)
   dfx::DevBuf dofSlotOffsets, dofSlots;
   // ----- diagonal

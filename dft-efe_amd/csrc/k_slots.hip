@@ -1,0 +1,173 @@
+// The row sums of the slot apply: every cell's product lies in its map slots'
+// rows (cellSlots), and each dof's row is the sum of its slots' rows in a
+// fixed order, with the step that follows the apply formed in the same launch.
+#include "enr_reduce.hpp"
+#include "kernels.hpp"
+#include "res_update.hpp"
+
+namespace dfx
+{
+  namespace k
+  {
+    namespace
+    {
+      template <class T, int V>
+      struct Vec
+      {
+        typedef T type __attribute__((ext_vector_type(V)));
+      };
+      template <class T>
+      struct Vec<T, 1>
+      {
+        typedef T type;
+      };
+      __device__ inline double at(double v, int) { return v; }
+      __device__ inline float  at(float v, int) { return v; }
+      template <class VT>
+      __device__ inline auto at(VT v, int e)
+      {
+        return v[e];
+      }
+      template <class T>
+      __device__ inline void put(T &v, int, T s)
+      {
+        v = s;
+      }
+      template <class VT, class T>
+      __device__ inline void put(VT &v, int e, T s)
+      {
+        v[e] = s;
+      }
+
+      // Blocks below nE * ceil(B / 16): one enriched dof and 16 columns each
+      // (EnrReduce; first, as they run longest).  The others: one thread per
+      // classical row and V columns (V: one 16-byte vector where widths and
+      // addresses allow).  A row's first slot sits in its head, so that slot's
+      // load does not wait for the list of the others; most rows (a cell's
+      // interior) have no others.  Bound by memory: B values read per slot,
+      // written per row (p = 4, 32^3 cells, FP32, 128 columns: 3.3 GB in 645 us;
+      // p = 3, 16^3 cells, 40 columns, FP32: 68 MB in 14 us)
+      template <class T, int V, bool RES>
+      __global__ __launch_bounds__(256) void slotSumK(
+        const RowHead *__restrict__ heads, const u32 *__restrict__ rest,
+        const u32 *__restrict__ enrOff, const u32 *__restrict__ enrSlots, u32 nC, u32 nE,
+        const T *__restrict__ slots, u32 B, T *x, u32 ldx, T *y, u32 ldy, int zeroX,
+        ResFuse<T> rf)
+      {
+        using vt = typename Vec<T, V>::type;
+        __shared__ EnrReduce<T> red;
+        const u32 nb = (B + EnrReduce<T>::CB - 1) / EnrReduce<T>::CB;
+        if (blockIdx.x < nE * nb)
+          {
+            const u32 g = blockIdx.x / nb;
+            const u32 j = (blockIdx.x % nb) * EnrReduce<T>::CB + threadIdx.x % EnrReduce<T>::CB;
+            const T   s = red.sum(enrSlots, enrOff[g], enrOff[g + 1], slots, B, j);
+            if (threadIdx.x < EnrReduce<T>::CB && j < B)
+              {
+                if constexpr (RES)
+                  {
+                    const u64 o = (u64)(nC + g) * ldx + j;
+                    rf.res[o]   = resUpdate<T>(s, x[o], rf.res[o], rf.r0[o], rf.mu[j],
+                                               (T)rf.coef[0], (T)rf.coef[1], (T)rf.coef[2]);
+                  }
+                else
+                  y[(u64)(nC + g) * ldy + j] = s;
+              }
+            return;
+          }
+        const u32 nv = B / V;
+        const u64 t  = (u64)(blockIdx.x - nE * nb) * 256 + threadIdx.x;
+        if (t >= (u64)nC * nv)
+          return;
+        u32 row, j;
+        if ((t >> 32) == 0)
+          row = (u32)t / nv, j = ((u32)t - row * nv) * V;
+        else
+          row = (u32)(t / nv), j = (u32)(t - (u64)row * nv) * V;
+        const RowHead h   = heads[row];
+        const u32     cnt = h.rest >> ROW_COUNT_SHIFT;
+        if (cnt == ROW_ZERO)
+          {
+            if constexpr (!RES)
+              {
+                *reinterpret_cast<vt *>(y + (u64)row * ldy + j) = vt{};
+                if (zeroX)
+                  *reinterpret_cast<vt *>(x + (u64)row * ldx + j) = vt{};
+              }
+            return;
+          }
+        const u64 o = (u64)row * ldx + j;
+        vt        xv{}, rv{}, zv{};
+        if constexpr (RES)
+          {
+            xv = *reinterpret_cast<const vt *>(x + o);
+            rv = *reinterpret_cast<const vt *>(rf.res + o);
+            zv = *reinterpret_cast<const vt *>(rf.r0 + o);
+          }
+        vt s{};
+        if (cnt)
+          s += *reinterpret_cast<const vt *>(slots + (u64)h.slot0 * B + j);
+        if (cnt > 1)
+          {
+            const u32 *q = rest + (h.rest & ((1u << ROW_COUNT_SHIFT) - 1));
+            for (u32 e = 0; e + 1 < cnt; e += 4)
+              {
+                vt v[4];
+#pragma unroll
+                for (u32 k = 0; k < 4; ++k)
+                  if (e + k + 1 < cnt)
+                    v[k] = *reinterpret_cast<const vt *>(slots + (u64)q[e + k] * B + j);
+#pragma unroll
+                for (u32 k = 0; k < 4; ++k)
+                  if (e + k + 1 < cnt)
+                    s += v[k];
+              }
+          }
+        if constexpr (RES)
+          {
+            const T a1 = (T)rf.coef[0], a2 = (T)rf.coef[1], c = (T)rf.coef[2];
+            vt      out{};
+#pragma unroll
+            for (int e = 0; e < V; ++e)
+              put(out, e, resUpdate<T>(at(s, e), at(xv, e), at(rv, e), at(zv, e), rf.mu[j + e],
+                                       a1, a2, c));
+            *reinterpret_cast<vt *>(rf.res + o) = out;
+          }
+        else
+          *reinterpret_cast<vt *>(y + (u64)row * ldy + j) = s;
+      }
+    } // namespace
+
+    template <class T>
+    void slotSum(hipStream_t s, const dfx_op *op, const T *slots, View<T> x, View<T> y,
+                 bool zeroX, const ResFuse<T> *rf)
+    {
+      const u32 nC = op->nClassical, nE = op->nDofs - nC, B = y.B;
+      if (!B || !op->nDofs)
+        return;
+      constexpr u32 V = 16 / sizeof(T);
+      auto aligned    = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+      const bool vec  = B % V == 0 && x.ld % V == 0 && y.ld % V == 0 && aligned(slots) &&
+                       aligned(x.p) && aligned(y.p) &&
+                       (!rf || (aligned(rf->res) && aligned(rf->r0)));
+      const u64 grid = (u64)nE * ((B + EnrReduce<T>::CB - 1) / EnrReduce<T>::CB) +
+                       ((u64)nC * (vec ? B / V : B) + 255) / 256;
+      DFX_REQUIRE(grid < (1ull << 31), "too many columns for the row sums");
+      auto go = [&](auto kern) {
+        kern<<<(unsigned)grid, 256, 0, s>>>(
+          op->rowHeads.as<RowHead>(), op->slotRest.as<u32>(), op->enrSlotOffsets.as<u32>(),
+          op->enrMapSlots.as<u32>(), nC, nE, slots, B, x.p, x.ld, y.p, y.ld, zeroX ? 1 : 0,
+          rf ? *rf : ResFuse<T>{});
+      };
+      if (rf)
+        vec ? go(slotSumK<T, (int)V, true>) : go(slotSumK<T, 1, true>);
+      else
+        vec ? go(slotSumK<T, (int)V, false>) : go(slotSumK<T, 1, false>);
+      checkLaunch("slotSum");
+    }
+    template void slotSum<double>(hipStream_t, const dfx_op *, const double *, View<double>,
+                                  View<double>, bool, const ResFuse<double> *);
+    template void slotSum<float>(hipStream_t, const dfx_op *, const float *, View<float>,
+                                 View<float>, bool, const ResFuse<float> *);
+  } // namespace k
+} // namespace dfx

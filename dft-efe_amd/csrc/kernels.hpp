@@ -151,6 +151,28 @@ namespace dfx
     // up to kpadMax
     template <class T>
     int builtinNT(u32 B, u32 kpadMax);
+    // the products of one size class's cells (a launch of the slot order), each
+    // row stored to its map slot's row of `slots` (sum n_e x B); mask: rows
+    // the operator's constraints hold at zero are taken as 0.  dsc, xe, nt as
+    // in cellApply
+    template <class T>
+    void cellSlots(hipStream_t s, const dfx_op *op, const Launch &L, const T *frag,
+                   View<const T> x, T *slots, const double *dsc, const T *xe, bool mask,
+                   int nt = 0);
+    template <class T>
+    int slotNT(u32 B, u32 kpadMax);
+    // whether the slot kernel reaches x's rows with 32-bit offsets (any width
+    // and alignment)
+    template <class T>
+    bool slotAddressable(const dfx_op *op, View<const T> x);
+    // Y from the slots, row by row (classical rows in launch order of their
+    // cells, enriched ones as enrichedReduce: the bits of the colour-by-colour
+    // apply); with zeroRows the rows held at zero are cleared in Y and, unless
+    // null, in X.  rf: the residual step on every row but those (x: its rn)
+    // instead of storing Y
+    template <class T>
+    void slotSum(hipStream_t s, const dfx_op *op, const T *slots, View<T> x, View<T> y,
+                 bool zeroX, const ResFuse<T> *rf);
     // out[s] = d[map[s]] (map[s] < nC) else 1, for every slot of a cell->dof map
     void gatherDiag(hipStream_t s, const double *d, const u32 *map, u64 n, u32 nC,
                     double *out);

@@ -45,6 +45,117 @@ namespace dfx
                          View<const float>{(const float *)Y->d, Y->N, Y->B, Y->B}, out);
   }
 
+  namespace
+  {
+    u32 mtwOf(u32 n) { return (((n + 15) / 16) + 3) / 4; }
+
+    // The slot apply's tables: launch records and cell metadata by (size
+    // class, caller order), so that neighbours follow each other; the masked
+    // map; per classical row its slots in launch order (the order in which
+    // the colour-by-colour apply adds); the enriched dofs' slots in cell
+    // order (eOff: their offsets).  Not built (slotsOk false) for rows of
+    // more than 30 cells or more than 2^27 shared slots
+    void buildSlots(dfx_op *op, const u32 *map, const std::vector<u32> &nc,
+                    const std::vector<u32> &eOff, bool merge)
+    {
+      const u32   nCells = op->nCells, nClassical = op->nClassical;
+      const auto &nd = op->hCellNdofs, &off = op->hMapOffset;
+      hipStream_t st = op->ctx->stream;
+      // slots per classical row; the first one is known from a row's head
+      std::vector<unsigned char> cnt(nClassical, 0);
+      u64                        others = 0;
+      for (u32 e = 0; e < nCells; ++e)
+        for (u32 s = off[e]; s < off[e] + nc[e]; ++s)
+          {
+            if (cnt[map[s]] == ROW_ZERO - 1)
+              return;
+            others += cnt[map[s]]++ != 0;
+          }
+      if (others >= (1ull << ROW_COUNT_SHIFT))
+        return;
+      const dfx_constraints *cons = op->cons;
+      op->zeroRows = cons && cons->homDirichlet && !cons->hRows.empty() &&
+                     *std::max_element(cons->hRows.begin(), cons->hRows.end()) < nClassical;
+      std::vector<RowHead> heads(nClassical);
+      std::vector<u32>     rest(others);
+      u32                  pos = 0;
+      for (u32 d = 0; d < nClassical; ++d)
+        {
+          heads[d] = {0u, ((u32)cnt[d] << ROW_COUNT_SHIFT) | pos};
+          pos += cnt[d] ? cnt[d] - 1u : 0u;
+        }
+      std::vector<unsigned char> seen(nClassical, 0);
+      for (u32 q = 0; q < nCells; ++q)
+        {
+          const u32 e = op->hOrder[q];
+          for (u32 s = off[e]; s < off[e] + nc[e]; ++s)
+            {
+              RowHead       &h = heads[map[s]];
+              unsigned char &k = seen[map[s]];
+              if (k == 0)
+                h.slot0 = s;
+              else
+                rest[(h.rest & ((1u << ROW_COUNT_SHIFT) - 1)) + k - 1] = s;
+              ++k;
+            }
+        }
+      if (op->zeroRows)
+        {
+          std::vector<u32> masked(map, map + op->sumNe);
+          for (u32 r : cons->hRows)
+            heads[r] = {0u, ROW_ZERO << ROW_COUNT_SHIFT};
+          for (u32 e = 0; e < nCells; ++e)
+            for (u32 s = off[e]; s < off[e] + nc[e]; ++s)
+              if (heads[map[s]].rest >> ROW_COUNT_SHIFT == ROW_ZERO)
+                masked[s] = ROW_NONE;
+          upload(op->slotMap, masked, st);
+        }
+      // enriched dofs: the same lists as the colour apply's, as map slots
+      std::vector<u32> eSlots(op->nEnrSlots), fp(eOff.begin(), eOff.end() - 1);
+      for (u32 e = 0; e < nCells; ++e)
+        for (u32 s = off[e] + nc[e]; s < off[e + 1]; ++s)
+          eSlots[fp[map[s] - nClassical]++] = s;
+      // launch order
+      std::vector<u32> place(nCells), at(nCells);
+      for (u32 q = 0; q < nCells; ++q)
+        place[op->hOrder[q]] = q;
+      std::iota(at.begin(), at.end(), 0u);
+      std::stable_sort(at.begin(), at.end(),
+                       [&](u32 a, u32 b) { return mtwOf(nd[a]) > mtwOf(nd[b]); });
+      std::vector<CellMeta> meta(nCells);
+      for (u32 q = 0; q < nCells; ++q)
+        meta[q] = op->hMeta[place[at[q]]];
+      for (int f64 = 0; f64 < 2; ++f64)
+        {
+          auto &out = f64 ? op->slotLaunches64 : op->slotLaunches32;
+          out.clear();
+          for (u32 q = 0; q < nCells;)
+            {
+              Launch l{};
+              l.begin = q;
+              l.mtw   = mtwOf(nd[at[q]]);
+              for (; q < nCells && (merge || mtwOf(nd[at[q]]) == l.mtw); ++q)
+                {
+                  const u32 n = nd[at[q]];
+                  l.kpadMax   = std::max(l.kpadMax, f64 ? 8 * ((n + 7) / 8) : 16 * ((n + 15) / 16));
+                  l.sumN2 += (u64)n * n;
+                  l.sumN += n;
+                  l.sumNc += nc[at[q]];
+                }
+              l.end = q;
+              out.push_back(l);
+            }
+        }
+      upload(op->metaSlots, meta, st);
+      upload(op->rowHeads, heads, st);
+      if (!rest.empty())
+        upload(op->slotRest, rest, st);
+      if (!eSlots.empty())
+        upload(op->enrMapSlots, eSlots, st);
+      op->slotsOk = true;
+    }
+  } // namespace
+
   void buildCellwise(dfx_ctx *ctx, dfx_op *op, u32 nCells, const u32 *cellNdofs,
                      const u32 *map, u32 nDofs, u32 nClassical, dfx_constraints *cons,
                      u32 flags)
@@ -150,7 +261,6 @@ namespace dfx
     op->nColors = (u32)nColors;
 
     // ---- launch order: (colour, M-tile class, cell)
-    auto mtwOf = [](u32 n) { return (((n + 15) / 16) + 3) / 4; };
     op->hOrder.resize(nCells);
     std::iota(op->hOrder.begin(), op->hOrder.end(), 0u);
     std::stable_sort(op->hOrder.begin(), op->hOrder.end(), [&](u32 a, u32 b) {
@@ -332,6 +442,7 @@ namespace dfx
     hipStream_t st = ctx->stream;
     upload(op->map, map, sumNe, st);
     upload(op->meta, op->hMeta, st);
+    buildSlots(op, map, nc, eOff, mergeEnv ? merge64 : nCells < 1024u);
     upload(op->first, hFirst, st);
     upload(op->last, hLast, st);
     if (!hResRows.empty())

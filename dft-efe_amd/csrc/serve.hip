@@ -101,7 +101,9 @@ namespace dfx
       // N x n FP64 arrays: subspaces, filter and CholGS / RR work, and the
       // H X, M X the solver keeps of its eigenvectors
       const u64 vecs  = 18 * N * (u64)r.numStates * 8;
-      return (mats + setup + vecs) * 5 / 4 + (64ull << 20);
+      // the slots of H's and M's applies
+      const u64 slots = 2 * std::min<u64>(SLOT_BYTES, sumN * r.numStates * 8);
+      return (mats + setup + vecs + slots) * 5 / 4 + (64ull << 20);
     }
 
     struct Shared

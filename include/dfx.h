@@ -228,7 +228,9 @@ int dfx_op_export_map(const dfx_op *op, uint32_t *cellNdofs, uint32_t *cellDofMa
  * by HIP events on the context's stream.  get_profile synchronizes, and
  * reports the colour steps ("launches"), their summed time, and the
  * algorithmic flops (2 B sum n_e^2) and bytes (matrices + map + gathered X +
- * scattered Y) of their cells. */
+ * scattered Y) of their cells.  An apply that sends its products through map
+ * slots (small and middle sizes) is one "launch": its cell kernels and row
+ * sums. */
 typedef struct dfx_op_profile
 {
   uint64_t launches;

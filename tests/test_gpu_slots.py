@@ -1,0 +1,128 @@
+"""The slot path of the cell-wise apply (every cell's product to its map
+slots, then row sums) against the colour-by-colour path, which
+dfx_op_apply_noalloc takes at any size: bit for bit, over column counts at the
+edges of the column tiles and 16-byte vectors, both precisions, constraints
+with and without parents, enriched rows and every size class."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import dfx
+import oracle as O
+from gpu_helpers import Ops
+from problems import c1_like, enriched, guess, hanging
+
+pytestmark = pytest.mark.gpu
+
+
+def mv(ctx, a, dtype=dfx.F64):
+    return dfx.MultiVector.from_numpy(ctx, a, dtype)
+
+
+@pytest.fixture(scope="module")
+def probs():
+    atoms = [(-1.0, 0.5, 0.2, 1), (1.2, -0.8, 0.6, 6), (0.3, 1.4, -1.1, 8)]
+    return {"c1": c1_like(n=3), "hang3": hanging(p=3), "enr": enriched(p=2, n=4),
+            "wide": O.Problem.build(p=4, n=(3, 3, 3), lo=(-12.,) * 3, hi=(12.,) * 3, atoms=atoms,
+                                    enrich=True, nq_enr=6)}
+
+
+@pytest.mark.parametrize("name", ["c1", "hang3", "enr", "wide"])
+@pytest.mark.parametrize("dtype", [dfx.F64, dfx.F32])
+def test_slot_apply_equals_colour_apply(ctx, probs, name, dtype):
+    P = probs[name]
+    ops = Ops(ctx, P)
+    npd = np.float64 if dtype == dfx.F64 else np.float32
+    for B in (1, 2, 3, 5, 16, 17, 31, 33, 40, 48, 49, 64, 66, 72, 80, 81, 101, 130):
+        X = O.rng_uniform(B, -1, 1, P.nDofs * B).reshape(P.nDofs, B).astype(npd)
+        Xa, Xb = mv(ctx, X, dtype), mv(ctx, X, dtype)
+        Ya, Yb = (dfx.MultiVector(ctx, P.nDofs, B, dtype) for _ in range(2))
+        ops.H.apply(Xa, Ya)
+        ops.H.apply_noalloc(Xb, Yb)
+        assert np.array_equal(Ya.to_numpy(), Yb.to_numpy()), (name, B)
+        assert np.array_equal(Xa.to_numpy(), Xb.to_numpy()), (name, B)   # the same P2C on X
+
+
+@pytest.mark.parametrize("name", ["c1", "hang3", "wide"])
+@pytest.mark.parametrize("dtype", [dfx.F64, dfx.F32])
+def test_folded_inverse_equals_the_two_applies_at_any_width(ctx, probs, name, dtype):
+    """M^-1 folded into the gather against M^-1's apply then H's colour path
+    (X gets the same parent->child update)."""
+    P = probs[name]
+    ops = Ops(ctx, P)
+    npd = np.float64 if dtype == dfx.F64 else np.float32
+    for B in (1, 3, 13, 40, 72):
+        X = O.rng_uniform(B, -1, 1, P.nDofs * B).reshape(P.nDofs, B).astype(npd)
+        Xa, Xb = mv(ctx, X, dtype), mv(ctx, X, dtype)
+        Ya, Yb, Z = (dfx.MultiVector(ctx, P.nDofs, B, dtype) for _ in range(3))
+        ops.H.apply_after_inverse(ops.Minv, Xa, Ya)
+        ops.Minv.apply(Xb, Z)
+        ops.H.apply_noalloc(Z, Yb)
+        assert np.array_equal(Ya.to_numpy(), Yb.to_numpy()), (name, B)
+        assert np.array_equal(Xa.to_numpy(), Xb.to_numpy()), (name, B)
+
+
+@pytest.mark.parametrize("B", [3, 13, 40])
+@pytest.mark.parametrize("prec", [dfx.PREC_FP64, dfx.PREC_MIXED])
+def test_residual_step_in_the_row_sums_is_bit_identical(ctx, probs, B, prec, monkeypatch):
+    P = probs["wide"]
+    ops = Ops(ctx, P)
+    X = guess(P, B, seed=B)
+    lo, hi, beta = P.lanczos(O.rng_uniform(2, -1, 1, P.nDofs))
+    a, c = lo, hi + beta / 10
+    b = a + 0.05 * (c - a)
+    outs = []
+    for fuse in ("1", "0"):
+        monkeypatch.setenv("DFX_FUSE_RES", fuse)
+        G, V = mv(ctx, X), dfx.MultiVector(ctx, P.nDofs, B)
+        s = dfx.ChebyshevFilteredEigenSolver(ctx, a, b, c, 7, 1e-14, G, True, 0, prec)
+        eig = np.linspace(a, b, B)
+        assert s.solve(ops.H, eig, V, True, ops.M, ops.Minv) == 0
+        outs.append((eig, V.to_numpy()))
+    assert np.array_equal(outs[0][0], outs[1][0]) and np.array_equal(outs[0][1], outs[1][1])
+
+
+@pytest.mark.parametrize("dtype", [dfx.F64, dfx.F32])
+@pytest.mark.parametrize("B", [4, 5])
+def test_addresses_of_one_value_alignment(ctx, probs, dtype, B):
+    """Caller-owned memory that starts one value past a 16-byte boundary."""
+    P = probs["enr"]
+    ops = Ops(ctx, P)
+    npd = np.float64 if dtype == dfx.F64 else np.float32
+    X = O.rng_uniform(B, -1, 1, P.nDofs * B).reshape(P.nDofs, B).astype(npd)
+    want = dfx.MultiVector(ctx, P.nDofs, B, dtype)
+    ops.H.apply(mv(ctx, X, dtype), want)
+
+    def shifted():
+        own = dfx.MultiVector(ctx, P.nDofs * B + 8, 1, dtype)
+        m = dfx.MultiVector.__new__(dfx.MultiVector)
+        m.ctx, m.N, m.B, m.dtype, m.h, m.own = ctx, P.nDofs, B, dtype, C.c_void_p(), own
+        ctx.check(dfx._lib.dfx_mv_wrap(ctx.h, own.device_ptr + np.dtype(npd).itemsize, P.nDofs, B,
+                                       dtype, C.byref(m.h)))
+        return m
+
+    Xs, Ys = shifted(), shifted()
+    Xs.upload(X)
+    ops.H.apply(Xs, Ys)
+    assert np.array_equal(Ys.to_numpy(), want.to_numpy())
+
+
+@pytest.mark.parametrize("cells", [30, 31, 40])
+def test_rows_of_many_cells_and_of_none(ctx, cells):
+    """Cells that all share one dof (a row of up to 30 cells has slot lists,
+    more fall back to one launch per colour) and a dof in no cell."""
+    n = cells + 2                                   # dof cells + 1: in no cell
+    cmap = np.stack([np.zeros(cells, int), np.arange(1, cells + 1)], axis=1)
+    A = O.rng_uniform(cells, -1, 1, cells * 4).reshape(cells, 2, 2)
+    op = dfx.CellOperator(ctx, np.full(cells, 2), cmap.ravel(), A.ravel(), n)
+    X = O.rng_uniform(3, -1, 1, n * 6).reshape(n, 6)
+    Y = dfx.MultiVector(ctx, n, 6)
+    Y.set(7.0)
+    op.apply(mv(ctx, X), Y)
+    ref = np.zeros_like(X)
+    for e in range(cells):
+        # y_cell = x_cell A (column-major blocks, both stored row by row here)
+        ref[cmap[e]] += A[e] @ X[cmap[e]]
+    # sums of at most `cells` + 2 products per entry
+    assert np.abs(Y.to_numpy() - ref).max() <= (cells + 2) * 2.0 ** -52 * cells
