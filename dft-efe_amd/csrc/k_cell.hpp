@@ -153,20 +153,29 @@ namespace dfx
           __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, off, 0, 0);
         }
         // the first `live` (<= 0: none, >= 4: all) of four consecutive values
-        // at off (4-byte aligned), 0 elsewhere; a vector is cut off only when
-        // `ragged` (uniform), and then loaded value by value
-        __device__ static f4_t part(rsrc_t r, u32 off, int live, bool ragged)
+        // at off (4-byte aligned), in two steps so that nothing waits between
+        // a load and its use: a vector that the row cuts off arrives as the
+        // end of a load that starts earlier in the row (part), and is shifted
+        // when used (whole).  `lead` false (uniform: nothing lies before it):
+        // loaded value by value
+        __device__ static f4_t part(rsrc_t r, u32 off, int live, bool lead)
         {
-          f4_t v = load4(r, live >= 4 ? off : OFF_NONE);
-          if (ragged)
+          if (!lead)
+            {
+              f4_t v{};
 #pragma unroll
-            for (int e = 0; e < 3; ++e)
-              {
-                const bool  one = live < 4 && live > e;
-                const float s   = load(r, one ? off + 4 * e : OFF_NONE);
-                v[e]            = one ? s : v[e];
-              }
-          return v;
+              for (int e = 0; e < 3; ++e)
+                v[e] = load(r, live > e ? off + 4 * e : OFF_NONE);
+              return v;
+            }
+          return load4(r, live > 0 ? off - (live < 4 ? 16 - 4 * live : 0) : OFF_NONE);
+        }
+        __device__ static f4_t whole(f4_t u, int live, bool lead)
+        {
+          return !lead || live >= 4 ? u
+                 : live == 3        ? f4_t{u[1], u[2], u[3], 0.f}
+                 : live == 2        ? f4_t{u[2], u[3], 0.f, 0.f}
+                                    : f4_t{u[3], 0.f, 0.f, 0.f};
         }
       };
       template <>
@@ -184,16 +193,15 @@ namespace dfx
         {
           __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2_t, v), r, off, 0, 0);
         }
-        // the first `live` of two consecutive values at off, 0 elsewhere
-        __device__ static d2_t part(rsrc_t r, u32 off, int live, bool ragged)
+        __device__ static d2_t part(rsrc_t r, u32 off, int live, bool lead)
         {
-          d2_t v = load4(r, live >= 2 ? off : OFF_NONE);
-          if (ragged)
-            {
-              const double s = load(r, live == 1 ? off : OFF_NONE);
-              v[0]           = live == 1 ? s : v[0];
-            }
-          return v;
+          if (!lead)
+            return d2_t{load(r, live > 0 ? off : OFF_NONE), 0.0};
+          return load4(r, live > 0 ? off - (live == 1 ? 8 : 0) : OFF_NONE);
+        }
+        __device__ static d2_t whole(d2_t u, int live, bool lead)
+        {
+          return lead && live == 1 ? d2_t{u[1], 0.0} : u;
         }
       };
 
@@ -392,11 +400,11 @@ namespace dfx
             // ---- gather.  A unit is G rows x G columns: G 16-byte loads,
             // transposed in registers into G 16-byte LDS stores (one per
             // column, holding G consecutive K values), at the swizzled column
-            // position swz().  SLOT takes any column count: a last vector of
-            // columns that the chunk cuts off is loaded value by value (the
-            // others are launched with whole vectors only: that test costs
-            // them 0.5 %)
+            // position swz().  SLOT takes any column count, with a last vector
+            // of columns that the chunk cuts off (the others are launched with
+            // whole vectors only: the test costs them 0.5 %)
             const bool ragged = SLOT && bw % G != 0;
+            const bool lead   = B >= (u32)G; // a cut-off vector has a whole one before it
             vec_t v[UPT][G];
             // the rows a wave gathers for unit u form one contiguous block
             // [kLo, kHi] (wave-uniform): wholly classical blocks read rX,
@@ -427,7 +435,7 @@ namespace dfx
                                         !(SLOT && m == ROW_NONE) & (c < bw))
                                          ? (SLOT ? bw - c : G)
                                          : 0,
-                                       ragged);
+                                       !SLOT || lead);
                   }
               }
             if (!oneX)
@@ -449,7 +457,7 @@ namespace dfx
                     const u32 m  = sMap[liveS ? kk : 0];
                     e[r] = BF::part(rXE, ((m - nC) * ldx + c0 + cS) * S,
                                     (liveS & (kk >= nc) & (kk < n) & (cS < bw)) ? (SLOT ? bw - cS : G) : 0,
-                                    ragged);
+                                    !SLOT || lead);
                   }
 #pragma unroll
                 for (int u = 0; u < UPT; ++u)
@@ -460,6 +468,15 @@ namespace dfx
                       v[u][r] = (u == uS & q * G + r >= nc) ? e[r] : v[u][r];
                   }
               }
+            if (SLOT && ragged) // uniform
+#pragma unroll
+              for (int u = 0; u < UPT; ++u)
+                {
+                  const int t = tx + u * 256, c = (t % VCL) * G;
+#pragma unroll
+                  for (int r = 0; r < G; ++r)
+                    v[u][r] = BF::whole(v[u][r], bw - c, lead);
+                }
 #pragma unroll
             for (int u = 0; u < UPT; ++u)
               {
