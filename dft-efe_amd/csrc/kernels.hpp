@@ -192,15 +192,19 @@ namespace dfx
 
     // --------------------------------------------------------- dense
     // S (n x n, column-major, FP64) = X^T Y over all N rows; deterministic
-    template <class T>
-    void gram(hipStream_t s, View<const T> X, View<const T> Y, double *partials,
+    void gram(hipStream_t s, View<const double> X, View<const double> Y, double *partials,
               size_t partialsCap, double *S);
-    // Xo = X Q  (Q n x n column-major FP64, device); Xo must not alias X;
-    // qrScratch holds n * 16 * ceil(n / 16) doubles.  With a rocBLAS handle
-    // (bound to stream s) an FP64 rotation is one library GEMM
-    template <class T>
-    void rotate(hipStream_t s, View<const T> X, const double *Q, View<T> Xo,
-                double *qrScratch, rocblas_handle blas = nullptr);
-    size_t gramPartialsNeeded(u32 N, u32 n);
+    // Xo = X Q  (Q n x n column-major FP64, device); Xo must not alias X; qf
+    // holds rotateScratch(n) doubles.  n > 256, or `library`: one rocBLAS GEMM
+    // (handle bound to stream s)
+    void rotate(hipStream_t s, View<const double> X, const double *Q, View<double> Xo, double *qf,
+                rocblas_handle blas, bool library);
+    inline size_t rotateScratch(u32 n)
+    {
+      const size_t m = (n + 15) / 16 * 16;
+      return m * m;
+    }
+    // partial sums of gram (ld: the larger leading dimension)
+    size_t gramPartialsNeeded(u32 N, u32 n, u32 ld);
   } // namespace k
 } // namespace dfx

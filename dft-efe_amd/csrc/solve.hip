@@ -406,12 +406,11 @@ namespace dfx
     }
 
     // ------------------------------------------------ subspace rotations
-    // Xo = X Q (N x n row-major, Q n x n column-major FP64) as one hipBLASLt
-    // matmul in column-major terms, Xo^T = Q^T X^T, with the first algorithm
-    // of the library's heuristic for the shape (a fixed choice, so results do
-    // not depend on timing); C4 (N = 2.1 M, n = 200): 3.2 ms against 3.7 for
-    // the rocBLAS DGEMM, which remains the fallback when hipBLASLt offers no
-    // algorithm
+    // Xo = X Q (N x n row-major, Q n x n column-major FP64): the hand-written
+    // kernel up to 256 columns.  Wider subspaces: one hipBLASLt matmul in
+    // column-major terms, Xo^T = Q^T X^T, with the first algorithm of the
+    // library's heuristic for the shape (a fixed choice, so results do not
+    // depend on timing), or the rocBLAS DGEMM when hipBLASLt offers none
     struct LtState
     {
       hipblasLtHandle_t h = nullptr;
@@ -456,9 +455,10 @@ namespace dfx
       DFX_REQUIRE(Xo.B == n && Xo.N == N, "rotate: shape mismatch");
       // DFX_ROTATE_LT=0: the rocBLAS DGEMM (read on every call)
       const char *env = getenv("DFX_ROTATE_LT");
-      if (env && atoi(env) == 0)
+      const bool  lib = env && atoi(env) == 0;
+      if (n <= 256 || lib)
         {
-          k::rotate<double>(ctx->stream, X, Q, Xo, qr, ctx->blas);
+          k::rotate(ctx->stream, X, Q, Xo, qr, ctx->blas, lib);
           return;
         }
       CaptureLock lk(captureMutex());
@@ -524,7 +524,7 @@ namespace dfx
             return;
           throw Error(DFX_E_HIP, "hipblasLtMatmul (rotation) failed");
         }
-      k::rotate<double>(ctx->stream, X, Q, Xo, qr, ctx->blas);
+      k::rotate(ctx->stream, X, Q, Xo, qr, ctx->blas, true);
     }
 
     // --------------------------------------------------- CholGS and RR
@@ -537,8 +537,8 @@ namespace dfx
       View<double> MX = workView<double>(ctx, "cg.mx", N, n);
       applyOp<double>(Bop, X, MX);
       double *S    = workDoubles(ctx, "cg.S", (size_t)n * n);
-      double *part = workDoubles(ctx, "gram.part", k::gramPartialsNeeded(N, n));
-      k::gram<double>(s, cv(X), cv(MX), part, k::gramPartialsNeeded(N, n), S);
+      double *part = workDoubles(ctx, "gram.part", k::gramPartialsNeeded(N, n, X.ld));
+      k::gram(s, cv(X), cv(MX), part, k::gramPartialsNeeded(N, n, X.ld), S);
       int *info = work(ctx, "info", 64).as<int>();
       rocblas_status st;
       {
@@ -583,7 +583,7 @@ namespace dfx
         for (u32 i = j; i < n; ++i)
           hQ[j + (size_t)n * i] = hS[i + (size_t)n * j];
       toDevice(ctx, Q, hQ.data(), hQ.size());
-      double *qr = workDoubles(ctx, "rot.qr", (size_t)n * 16 * ((n + 15) / 16));
+      double *qr = workDoubles(ctx, "rot.qr", k::rotateScratch(n));
       rotate64(ctx, cv(X), Q, Xo, qr);
       return 0;
     }
@@ -598,8 +598,8 @@ namespace dfx
       View<double> HX = workView<double>(ctx, hxName, N, n);
       applyOp<double>(A, X, HX);
       double *S    = workDoubles(ctx, "rr.S", (size_t)n * n);
-      double *part = workDoubles(ctx, "gram.part", k::gramPartialsNeeded(N, n));
-      k::gram<double>(s, cv(X), cv(HX), part, k::gramPartialsNeeded(N, n), S);
+      double *part = workDoubles(ctx, "gram.part", k::gramPartialsNeeded(N, n, X.ld));
+      k::gram(s, cv(X), cv(HX), part, k::gramPartialsNeeded(N, n, X.ld), S);
       double *D    = workDoubles(ctx, "rr.D", 2 * (size_t)n);
       int    *info = work(ctx, "info", 64).as<int>();
       rocblas_status st;
@@ -616,7 +616,7 @@ namespace dfx
       DFX_HIP(hipStreamSynchronize(s));
       if (hinfo != 0)
         return DFX_EIG_LAPACK_ERROR;
-      double *qr = workDoubles(ctx, "rot.qr", (size_t)n * 16 * ((n + 15) / 16));
+      double *qr = workDoubles(ctx, "rot.qr", k::rotateScratch(n));
       rotate64(ctx, cv(X), S, Xo, qr);
       return 0;
     }
@@ -823,7 +823,7 @@ namespace dfx
           const u32    N    = XV.N;
           const size_t by   = (size_t)N * n * sizeof(double);
           double      *S    = workDoubles(ctx, "rr.S", (size_t)n * n);
-          double      *qr   = workDoubles(ctx, "rot.qr", (size_t)n * 16 * ((n + 15) / 16));
+          double      *qr   = workDoubles(ctx, "rot.qr", k::rotateScratch(n));
           cs->kpHX.ensure(by);
           cs->kpMX.ensure(by);
           rotate64(ctx, cv(workView<double>(ctx, "rr.hx", N, n)), S,

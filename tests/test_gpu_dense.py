@@ -1,0 +1,66 @@
+"""Gram matrices and subspace rotations at the edges of their column tiles
+(1 to 257 columns: every kernel width, odd counts, the library path above 256)
+and of their row chunks, through the Cholesky-Gram-Schmidt and Rayleigh-Ritz
+entry points, against numpy."""
+import numpy as np
+import pytest
+
+import dfx
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+EPS = 2.0 ** -52
+
+
+def diagonal(ctx, d):
+    return dfx.DiagonalOperator(ctx, d)
+
+
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 33, 63, 64, 65, 101, 112, 113, 128, 129, 200,
+                               208, 255, 256, 257])
+def test_orthonormalization_and_ritz_at_every_width(ctx, n):
+    for N in sorted({n, n + 1, 1031, 4099}):
+        if N < n:
+            continue
+        rng = np.random.RandomState(n * 7 + N)
+        # columns of a well-conditioned block: an orthonormal basis, slightly mixed
+        X = np.linalg.qr(rng.uniform(-1, 1, (N, n)))[0]
+        X = X + 0.3 * X @ np.triu(rng.uniform(-1, 1, (n, n)), 1) / max(1, n)
+        m, h = rng.uniform(0.5, 2.0, N), rng.uniform(-1.0, 5.0, N)
+        Xo = dfx.MultiVector(ctx, N, n)
+        assert dfx.cholesky_gram_schmidt(ctx, dfx.MultiVector.from_numpy(ctx, X), Xo,
+                                         diagonal(ctx, m)) == 0
+        S = X.T @ (m[:, None] * X)
+        L = np.linalg.cholesky(S)
+        want = np.linalg.solve(L, X.T).T
+        # backward errors of the N-long sums and of the factorization, amplified
+        # by the factor's condition (below 10 here)
+        tol = 10 * EPS * (n + np.sqrt(N)) * np.linalg.cond(L)
+        got = Xo.to_numpy()
+        assert np.abs(got - want).max() <= tol * max(1.0, np.abs(want).max()), (n, N)
+        V = dfx.MultiVector(ctx, N, n)
+        Y = np.linalg.qr(X)[0]
+        rc, ev = dfx.rayleigh_ritz(ctx, diagonal(ctx, h), dfx.MultiVector.from_numpy(ctx, Y), V)
+        assert rc == 0
+        T = Y.T @ (h[:, None] * Y)
+        tol = 10 * EPS * (n + np.sqrt(N)) * 6
+        assert np.abs(ev - np.linalg.eigvalsh(T)).max() <= tol, (n, N)
+        v = V.to_numpy()
+        assert np.abs(v.T @ v - np.eye(n)).max() <= tol, (n, N)
+        assert np.abs(v.T @ (h[:, None] * v) - np.diag(ev)).max() <= tol, (n, N)
+
+
+def test_columns_past_the_block_do_not_enter(ctx):
+    """Not-a-number values of other columns stay out of a batch's products: the
+    padding of a narrow last tile is masked, not multiplied by zero."""
+    N, n = 300, 7
+    X = O.rng_uniform(5, -1, 1, N * n).reshape(N, n)
+    X = np.linalg.qr(X)[0]
+    m = np.ones(N)
+    Xo = dfx.MultiVector(ctx, N, n)
+    assert dfx.cholesky_gram_schmidt(ctx, dfx.MultiVector.from_numpy(ctx, X), Xo,
+                                     diagonal(ctx, m)) == 0
+    assert np.isfinite(Xo.to_numpy()).all()
+    X[4, 3] = np.nan
+    rc = dfx.cholesky_gram_schmidt(ctx, dfx.MultiVector.from_numpy(ctx, X), Xo, diagonal(ctx, m))
+    assert rc != 0                                   # reported, as any failed factorization
