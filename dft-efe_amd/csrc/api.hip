@@ -116,6 +116,31 @@ namespace dfx
       k::c2p<T>(s, op->cons, Y);
   }
 
+  // Y = op X and the column dots X.Y (device) in one go where op is cell-wise
+  // on the slot path with no constraints but rows held at zero; false
+  // (nothing done) otherwise.  partials: DOT_PARTIALS X.B doubles
+  bool applyDot(dfx_op *op, View<double> X, View<double> Y, double *partials, double *out)
+  {
+    View<const double> Xc{X.p, X.N, X.B, X.ld};
+    if (op->kind != OP_CELLWISE || (op->cons && op->cons->nRows && !op->zeroRows) ||
+        op->profiling || X.N != op->nDofs || Y.N != op->nDofs || X.B != Y.B ||
+        !slotPath<double>(op, Xc))
+      return false;
+    if (op->yE.ensure((size_t)op->sumNe * X.B * sizeof(double)))
+      ++op->gen;
+    double *slots = op->yE.as<double>();
+    for (const Launch &l : op->slotLaunches64)
+      k::cellSlots<double>(op->ctx->stream, op, l, fragOf<double>(op), Xc, slots, nullptr, nullptr,
+                           op->zeroRows);
+    if (!k::slotSumDot(op->ctx->stream, op, slots, X, Y, partials, out))
+      {
+        k::slotSum<double>(op->ctx->stream, op, slots, X, Y, op->zeroRows, nullptr);
+        k::colDots<double>(op->ctx->stream, Xc, View<const double>{Y.p, Y.N, Y.B, Y.ld}, partials,
+                           out);
+      }
+    return true;
+  }
+
   template <class T>
   void applyCellwise(dfx_op *op, View<T> X, View<T> Y, const double *dsc = nullptr,
                      const T *xe = nullptr, bool skipP2C = false, T *yEOverride = nullptr,

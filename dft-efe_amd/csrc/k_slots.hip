@@ -5,6 +5,8 @@
 #include "kernels.hpp"
 #include "res_update.hpp"
 
+#include <algorithm>
+
 namespace dfx
 {
   namespace k
@@ -47,6 +49,36 @@ namespace dfx
       // interior) have no others.  Bound by memory: B values read per slot,
       // written per row (p = 4, 32^3 cells, FP32, 128 columns: 3.3 GB in 645 us;
       // p = 3, 16^3 cells, 40 columns, FP32: 68 MB in 14 us)
+      //
+      // The sum of one row's V columns from j on: the row's slots in order
+      template <class T, int V>
+      __device__ inline typename Vec<T, V>::type rowSum(RowHead h, const u32 *__restrict__ rest,
+                                                        const T *__restrict__ slots, u32 B, u32 j)
+      {
+        using vt      = typename Vec<T, V>::type;
+        const u32 cnt = h.rest >> ROW_COUNT_SHIFT;
+        vt        s{};
+        if (cnt)
+          s += *reinterpret_cast<const vt *>(slots + (u64)h.slot0 * B + j);
+        if (cnt > 1)
+          {
+            const u32 *q = rest + (h.rest & ((1u << ROW_COUNT_SHIFT) - 1));
+            for (u32 e = 0; e + 1 < cnt; e += 4)
+              {
+                vt v[4];
+#pragma unroll
+                for (u32 k = 0; k < 4; ++k)
+                  if (e + k + 1 < cnt)
+                    v[k] = *reinterpret_cast<const vt *>(slots + (u64)q[e + k] * B + j);
+#pragma unroll
+                for (u32 k = 0; k < 4; ++k)
+                  if (e + k + 1 < cnt)
+                    s += v[k];
+              }
+          }
+        return s;
+      }
+
       template <class T, int V, bool RES>
       __global__ __launch_bounds__(256) void slotSumK(
         const RowHead *__restrict__ heads, const u32 *__restrict__ rest,
@@ -104,25 +136,7 @@ namespace dfx
             rv = *reinterpret_cast<const vt *>(rf.res + o);
             zv = *reinterpret_cast<const vt *>(rf.r0 + o);
           }
-        vt s{};
-        if (cnt)
-          s += *reinterpret_cast<const vt *>(slots + (u64)h.slot0 * B + j);
-        if (cnt > 1)
-          {
-            const u32 *q = rest + (h.rest & ((1u << ROW_COUNT_SHIFT) - 1));
-            for (u32 e = 0; e + 1 < cnt; e += 4)
-              {
-                vt v[4];
-#pragma unroll
-                for (u32 k = 0; k < 4; ++k)
-                  if (e + k + 1 < cnt)
-                    v[k] = *reinterpret_cast<const vt *>(slots + (u64)q[e + k] * B + j);
-#pragma unroll
-                for (u32 k = 0; k < 4; ++k)
-                  if (e + k + 1 < cnt)
-                    s += v[k];
-              }
-          }
+        const vt s = rowSum<T, V>(h, rest, slots, B, j);
         if constexpr (RES)
           {
             const T a1 = (T)rf.coef[0], a2 = (T)rf.coef[1], c = (T)rf.coef[2];
@@ -136,7 +150,87 @@ namespace dfx
         else
           *reinterpret_cast<vt *>(y + (u64)row * ldy + j) = s;
       }
+      // The row sums with the column dots x.y of the same rows (PCG's p.w, FP64,
+      // V = 2 columns a thread, B even): a workgroup takes RB = 256 / (B / 2)
+      // rows at a time, every nBlocks-th such group; its sums per column go to
+      // partials[block] (fixed tree over the rows), an enriched dof's product
+      // to partials[nBlocks + dof].  Saves the separate dot a read of x and y
+      // and a launch (16^3 cells, p = 3, 8 columns: 7.9 + 6.3 us for the two)
+      __global__ __launch_bounds__(256) void slotSumDotK(
+        const RowHead *__restrict__ heads, const u32 *__restrict__ rest,
+        const u32 *__restrict__ enrOff, const u32 *__restrict__ enrSlots, u32 nC, u32 nE,
+        const double *__restrict__ slots, u32 B, double *x, double *y, u32 nBlocks,
+        double *__restrict__ partials)
+      {
+        using T  = double;
+        using vt = Vec<double, 2>::type;
+        __shared__ EnrReduce<T> red;
+        __shared__ vt           sum[256];
+        const u32 nb = (B + EnrReduce<T>::CB - 1) / EnrReduce<T>::CB;
+        if (blockIdx.x < nE * nb)
+          {
+            const u32 g = blockIdx.x / nb;
+            const u32 j = (blockIdx.x % nb) * EnrReduce<T>::CB + threadIdx.x % EnrReduce<T>::CB;
+            const T   s = red.sum(enrSlots, enrOff[g], enrOff[g + 1], slots, B, j);
+            if (threadIdx.x < EnrReduce<T>::CB && j < B)
+              {
+                const u64 o                           = (u64)(nC + g) * B + j;
+                y[o]                                  = s;
+                partials[(u64)(nBlocks + g) * B + j] = x[o] * s;
+              }
+            return;
+          }
+        const u32 blk = blockIdx.x - nE * nb, nv = B / 2, RB = 256 / nv;
+        const u32 r = threadIdx.x / nv, j = (threadIdx.x - r * nv) * 2;
+        vt        acc{};
+        if (r < RB)
+          for (u32 row = blk * RB + r; row < nC; row += nBlocks * RB)
+            {
+              const RowHead h = heads[row];
+              const u64     o = (u64)row * B + j;
+              if (h.rest >> ROW_COUNT_SHIFT == ROW_ZERO)
+                {
+                  *reinterpret_cast<vt *>(y + o) = vt{};
+                  *reinterpret_cast<vt *>(x + o) = vt{};
+                  continue;
+                }
+              const vt xv = *reinterpret_cast<const vt *>(x + o);
+              const vt s  = rowSum<T, 2>(h, rest, slots, B, j);
+              *reinterpret_cast<vt *>(y + o) = s;
+              acc[0] = fma(xv[0], s[0], acc[0]);
+              acc[1] = fma(xv[1], s[1], acc[1]);
+            }
+        sum[threadIdx.x] = acc;
+        __syncthreads();
+        for (u32 h = 128; h > 0; h >>= 1)
+          {
+            if (h < RB && r < h && r + h < RB)
+              sum[threadIdx.x] += sum[threadIdx.x + h * nv];
+            __syncthreads();
+          }
+        if (threadIdx.x < nv)
+          *reinterpret_cast<vt *>(partials + (u64)blk * B + j) = sum[threadIdx.x];
+      }
     } // namespace
+
+    bool slotSumDot(hipStream_t s, const dfx_op *op, const double *slots, View<double> x,
+                    View<double> y, double *partials, double *out)
+    {
+      const u32 nC = op->nClassical, nE = op->nDofs - nC, B = y.B;
+      auto aligned = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+      if (B < 2 || B % 2 || B > 128 || x.ld != B || y.ld != B || !aligned(slots) ||
+          !aligned(x.p) || !aligned(y.p) || !nC || nE > DOT_PARTIALS / 2)
+        return false;
+      const u32 RB      = 256 / (B / 2);
+      const u32 nBlocks = (u32)std::min<u64>(DOT_PARTIALS / 2, ((u64)nC + RB - 1) / RB);
+      const u32 nb      = (B + EnrReduce<double>::CB - 1) / EnrReduce<double>::CB;
+      slotSumDotK<<<nE * nb + nBlocks, 256, 0, s>>>(
+        op->rowHeads.as<RowHead>(), op->slotRest.as<u32>(), op->enrSlotOffsets.as<u32>(),
+        op->enrMapSlots.as<u32>(), nC, nE, slots, B, x.p, y.p, nBlocks, partials);
+      checkLaunch("slotSumDot");
+      colDotsFinal(s, partials, nBlocks + nE, B, out);
+      return true;
+    }
 
     template <class T>
     void slotSum(hipStream_t s, const dfx_op *op, const T *slots, View<T> x, View<T> y,

@@ -4,6 +4,7 @@
 // N x B views with a leading dimension (column blocks of a wider multivector
 // are addressed in place, without the reference's per-dof copy loops,
 // src/linearAlgebra/ChebyshevFilteredEigenSolver.t.cpp:246-333).
+#include <algorithm>
 #include <vector>
 
 #include "kernels.hpp"
@@ -123,20 +124,41 @@ namespace dfx
           }
       }
 
-      // PCG search direction p = z + beta p with beta = zrNew / zr per column
-      // (the division of the separate beta launch, then the blocked axpby's
-      // element with unit coefficients)
-      __global__ void cgDirectionK(double *p, const double *z, const double *zrNew,
-                                   const double *zr, u32 N, u32 B)
+      // PCG search direction p = d o r + beta p with beta = zrNew / zr per
+      // column (the division of the separate beta launch, the diagonal
+      // scaling's product, then the blocked axpby's element with unit
+      // coefficients); V columns per thread
+      template <int V>
+      __global__ void cgDirectionK(double *p, const double *r, const double *d,
+                                   const double *zrNew, const double *zr, u32 N, u32 B)
       {
-        const u64 n = (u64)N * B;
+        typedef double vt __attribute__((ext_vector_type(2)));
+        const u64 n = (u64)N * B / V;
         for (u64 t = blockIdx.x * (u64)blockDim.x + threadIdx.x; t < n;
              t += (u64)gridDim.x * blockDim.x)
           {
-            RC           r    = rc(t, B);
-            const double beta = zrNew[r.j] / zr[r.j];
-            const u64    o    = (u64)r.i * B + r.j;
-            p[o]              = axpbyOne<double>(1.0, 1.0, z[o], 1.0, beta, p[o]);
+            RC        c = rc(t, B / V);
+            const u64 o = (u64)c.i * B + c.j * V;
+            double    rv[V], pv[V];
+            if constexpr (V == 2)
+              {
+                const vt a = *reinterpret_cast<const vt *>(r + o);
+                const vt b = *reinterpret_cast<const vt *>(p + o);
+                rv[0] = a[0], rv[1] = a[1], pv[0] = b[0], pv[1] = b[1];
+              }
+            else
+              rv[0] = r[o], pv[0] = p[o];
+#pragma unroll
+            for (int e = 0; e < V; ++e)
+              {
+                const u32    j    = c.j * V + e;
+                const double beta = zrNew[j] / zr[j];
+                pv[e]             = axpbyOne<double>(1.0, 1.0, d[c.i] * rv[e], 1.0, beta, pv[e]);
+              }
+            if constexpr (V == 2)
+              *reinterpret_cast<vt *>(p + o) = vt{pv[0], pv[1]};
+            else
+              p[o] = pv[0];
           }
       }
 
@@ -225,18 +247,21 @@ namespace dfx
       }
 
       // The PCG update of one iteration with a Jacobi preconditioner, fused:
-      //   x += alpha p, r -= alpha w, z = d o r, and the partial sums of z.r
-      //   and r.r (alpha = zr / pw per column, formed here as cgAlphaK does).
+      //   xn = x + alpha p, r -= alpha w, and the partial sums of z.r and r.r
+      // with z = d o r (alpha = zr / pw per column, formed here as cgAlphaK
+      // does; z itself is formed again where it is used).
       // Rows, lanes and sums follow colDotsK exactly (same blocks of rows,
       // same lane order, same combine), and each element is the blocked
       // axpby's / the diagonal scaling's expression, so every value is the
       // separate launches' bit for bit.  partials: nBlocks x 2B (z.r in
-      // columns [0, B), r.r in [B, 2B)); N x B arrays with leading dimension B
+      // columns [0, B), r.r in [B, 2B)); N x B arrays with leading dimension B.
+      // Bound by memory: 4 reads and 2 writes per value (with z, a copy of x and
+      // 16 lanes for 8 columns it took 15.5 us at 117 649 x 8)
       template <int C>
-      __global__ void cgUpdateK(double *x, double *r, double *z, const double *p,
+      __global__ void cgUpdateK(const double *x, double *xn, double *r, const double *p,
                                 const double *w, const double *d, const double *zr,
                                 const double *pw, u32 N, u32 B, u32 rowsPerBlock,
-                                double *partials, double *xs)
+                                double *partials)
       {
         constexpr int R  = TPB / C;
         const int     tx = threadIdx.x % C, ty = threadIdx.x / C;
@@ -250,19 +275,29 @@ namespace dfx
             if (j < B)
               {
                 const double alpha = zr[j] / pw[j], nalpha = -zr[j] / pw[j];
-                for (u32 i = r0 + ty; i < r1; i += R)
+                // four rows of a lane in flight together, added in order
+                for (u32 i0 = r0 + ty; i0 < r1; i0 += 4 * R)
                   {
-                    const u64    o  = (u64)i * B + j;
-                    const double xn = axpbyOne<double>(1.0, 1.0, x[o], 1.0, alpha, p[o]);
-                    const double rn = axpbyOne<double>(1.0, 1.0, r[o], 1.0, nalpha, w[o]);
-                    const double zn = d[i] * rn;
-                    x[o]            = xn;
-                    if (xs) // a copy of the new x (launch-uniform)
-                      xs[o] = xn;
-                    r[o]            = rn;
-                    z[o]            = zn;
-                    accZ = fma(zn, rn, accZ);
-                    accR = fma(rn, rn, accR);
+                    double xv[4], pv[4], rv[4], wv[4], dv[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                      if (const u32 i = i0 + u * R; i < r1)
+                        {
+                          const u64 o = (u64)i * B + j;
+                          xv[u] = x[o], pv[u] = p[o], rv[u] = r[o], wv[u] = w[o], dv[u] = d[i];
+                        }
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                      if (const u32 i = i0 + u * R; i < r1)
+                        {
+                          const u64    o  = (u64)i * B + j;
+                          const double rn = axpbyOne<double>(1.0, 1.0, rv[u], 1.0, nalpha, wv[u]);
+                          const double zn = dv[u] * rn;
+                          xn[o] = axpbyOne<double>(1.0, 1.0, xv[u], 1.0, alpha, pv[u]);
+                          r[o]  = rn;
+                          accZ  = fma(zn, rn, accZ);
+                          accR  = fma(rn, rn, accR);
+                        }
                   }
               }
             red[0][threadIdx.x] = accZ;
@@ -711,6 +746,19 @@ namespace dfx
       checkLaunch("enrichedBlock");
     }
 
+    namespace
+    {
+      // row blocks of the column dots: 64 rows or more (enough workgroups for
+      // the GPU from small vectors on), at most 1024 blocks
+      u32 dotBlocks(u32 N) { return std::max(1u, std::min(1024u, (u32)(((u64)N + 63) / 64))); }
+    } // namespace
+
+    void colDotsFinal(hipStream_t s, const double *partials, u32 nBlocks, u32 B, double *out)
+    {
+      colDotsFinalK<<<B, 256, 0, s>>>(partials, nBlocks, B, out);
+      checkLaunch("colDotsFinal");
+    }
+
     template <class T>
     void colDots(hipStream_t s, View<const T> x, View<const T> y, double *partials,
                  double *out)
@@ -718,21 +766,18 @@ namespace dfx
       const u32 B = x.B;
       if (!B)
         return;
-      u32 nBlocks = (x.N + 255) / 256;
-      if (nBlocks > 1024)
-        nBlocks = 1024;
-      if (nBlocks == 0)
-        nBlocks = 1;
+      const u32 nBlocks = dotBlocks(x.N);
       const u32 rows = (x.N + nBlocks - 1) / nBlocks;
-      if (B <= 16)
+      if (B <= 8)
+        colDotsK<T, 8><<<nBlocks, TPB, 0, s>>>(x.p, x.ld, y.p, y.ld, x.N, B, rows, partials);
+      else if (B <= 16)
         colDotsK<T, 16><<<nBlocks, TPB, 0, s>>>(x.p, x.ld, y.p, y.ld, x.N, B, rows, partials);
       else if (B <= 32)
         colDotsK<T, 32><<<nBlocks, TPB, 0, s>>>(x.p, x.ld, y.p, y.ld, x.N, B, rows, partials);
       else
         colDotsK<T, 64><<<nBlocks, TPB, 0, s>>>(x.p, x.ld, y.p, y.ld, x.N, B, rows, partials);
       checkLaunch("colDots");
-      colDotsFinalK<<<B, 256, 0, s>>>(partials, nBlocks, B, out);
-      checkLaunch("colDotsFinal");
+      colDotsFinal(s, partials, nBlocks, B, out);
     }
 
     void combinationNorms(hipStream_t s, double a1, const double *a, View<const double> x,
@@ -744,63 +789,59 @@ namespace dfx
         return;
       DFX_REQUIRE(x.ld == B && y.ld == B && y.N == N && y.B == B,
                   "combination norms: contiguous multivectors of one shape expected");
-      u32 nBlocks = (N + 255) / 256;
-      if (nBlocks > 1024)
-        nBlocks = 1024;
-      if (nBlocks == 0)
-        nBlocks = 1;
+      const u32 nBlocks = dotBlocks(N);
       const u32 rows = (N + nBlocks - 1) / nBlocks;
-      if (B <= 16)
+      if (B <= 8)
+        combNormsK<8><<<nBlocks, TPB, 0, s>>>(a1, a, x.p, b1, b, y.p, N, B, rows, partials);
+      else if (B <= 16)
         combNormsK<16><<<nBlocks, TPB, 0, s>>>(a1, a, x.p, b1, b, y.p, N, B, rows, partials);
       else if (B <= 32)
         combNormsK<32><<<nBlocks, TPB, 0, s>>>(a1, a, x.p, b1, b, y.p, N, B, rows, partials);
       else
         combNormsK<64><<<nBlocks, TPB, 0, s>>>(a1, a, x.p, b1, b, y.p, N, B, rows, partials);
       checkLaunch("combNorms");
-      colDotsFinalK<<<B, 256, 0, s>>>(partials, nBlocks, B, out);
-      checkLaunch("colDotsFinal");
+      colDotsFinal(s, partials, nBlocks, B, out);
     }
 
-    void cgUpdate(hipStream_t s, View<double> x, View<double> r, View<double> z,
+    void cgUpdate(hipStream_t s, View<double> x, View<double> xn, View<double> r,
                   View<const double> p, View<const double> w, const double *d,
-                  const double *zr, const double *pw, double *partials, double *zrrr,
-                  double *xs)
+                  const double *zr, const double *pw, double *partials, double *zrrr)
     {
       const u32 B = x.B, N = x.N;
       if (!B)
         return;
-      DFX_REQUIRE(x.ld == B && r.ld == B && z.ld == B && p.ld == B && w.ld == B,
+      DFX_REQUIRE(x.ld == B && xn.ld == B && r.ld == B && p.ld == B && w.ld == B,
                   "CG update: contiguous multivectors expected");
       // the partition of colDots
-      u32 nBlocks = (N + 255) / 256;
-      if (nBlocks > 1024)
-        nBlocks = 1024;
-      if (nBlocks == 0)
-        nBlocks = 1;
+      const u32 nBlocks = dotBlocks(N);
       const u32 rows = (N + nBlocks - 1) / nBlocks;
-      if (B <= 16)
-        cgUpdateK<16><<<nBlocks, TPB, 0, s>>>(x.p, r.p, z.p, p.p, w.p, d, zr, pw, N, B, rows,
-                                              partials, xs);
+      auto go = [&](auto kern) {
+        kern<<<nBlocks, TPB, 0, s>>>(x.p, xn.p, r.p, p.p, w.p, d, zr, pw, N, B, rows, partials);
+      };
+      if (B <= 8)
+        go(cgUpdateK<8>);
+      else if (B <= 16)
+        go(cgUpdateK<16>);
       else if (B <= 32)
-        cgUpdateK<32><<<nBlocks, TPB, 0, s>>>(x.p, r.p, z.p, p.p, w.p, d, zr, pw, N, B, rows,
-                                              partials, xs);
+        go(cgUpdateK<32>);
       else
-        cgUpdateK<64><<<nBlocks, TPB, 0, s>>>(x.p, r.p, z.p, p.p, w.p, d, zr, pw, N, B, rows,
-                                              partials, xs);
+        go(cgUpdateK<64>);
       checkLaunch("cgUpdate");
-      colDotsFinalK<<<2 * B, 256, 0, s>>>(partials, nBlocks, 2 * B, zrrr);
-      checkLaunch("colDotsFinal");
+      colDotsFinal(s, partials, nBlocks, 2 * B, zrrr);
     }
 
-    void cgDirection(hipStream_t s, View<double> p, View<const double> z, const double *zrNew,
-                     const double *zr)
+    void cgDirection(hipStream_t s, View<double> p, View<const double> r, const double *d,
+                     const double *zrNew, const double *zr)
     {
       const u64 n = (u64)p.N * p.B;
       if (!n)
         return;
-      DFX_REQUIRE(p.ld == p.B && z.ld == z.B && z.N == p.N && z.B == p.B,
+      DFX_REQUIRE(p.ld == p.B && r.ld == r.B && r.N == p.N && r.B == p.B,
                   "CG direction: contiguous multivectors of one shape expected");
-      cgDirectionK<<<gridFor(n), TPB, 0, s>>>(p.p, z.p, zrNew, zr, p.N, p.B);
+      if (p.B % 2 == 0) // scratch vectors: 256-byte aligned
+        cgDirectionK<2><<<gridFor(n / 2), TPB, 0, s>>>(p.p, r.p, d, zrNew, zr, p.N, p.B);
+      else
+        cgDirectionK<1><<<gridFor(n), TPB, 0, s>>>(p.p, r.p, d, zrNew, zr, p.N, p.B);
       checkLaunch("cgDirection");
     }
 

@@ -37,6 +37,10 @@ namespace dfx
     void colDots(hipStream_t s, View<const T> x, View<const T> y, double *partials,
                  double *out);
 
+    // the second pass of the column dots: out[j] = sum of nBlocks partials
+    void colDotsFinal(hipStream_t s, const double *partials, u32 nBlocks, u32 B, double *out);
+    constexpr u32 DOT_PARTIALS = 2048; // rows of partial sums a CG work buffer holds
+
     // out[j] = sum_i (a1 a[j] x_ij + b1 b[j] y_ij)^2 without forming the
     // combination: the bits of the blocked axpby followed by colDots
     // (partials: 1024 B doubles; out on the device)
@@ -44,17 +48,16 @@ namespace dfx
                           double b1, const double *b, View<const double> y, double *partials,
                           double *out);
     // PCG iteration with a Jacobi (diagonal d) preconditioner, fused
-    // (CGLinearSolver.t.cpp:68-313): alpha = zr / pw per column; x += alpha
-    // p; r -= alpha w; z = d o r; zrrr[0, B) = z.r, zrrr[B, 2B) = r.r, the
-    // bits of the separate launches.  partials: 2048 B doubles; xs (may be
-    // null, contiguous like x) receives a copy of the new x
-    void cgUpdate(hipStream_t s, View<double> x, View<double> r, View<double> z,
+    // (CGLinearSolver.t.cpp:68-313): alpha = zr / pw per column; xn = x + alpha
+    // p; r -= alpha w; zrrr[0, B) = z.r, zrrr[B, 2B) = r.r with z = d o r, the
+    // bits of the separate launches.  partials: DOT_PARTIALS B doubles; xn may
+    // be x
+    void cgUpdate(hipStream_t s, View<double> x, View<double> xn, View<double> r,
                   View<const double> p, View<const double> w, const double *d,
-                  const double *zr, const double *pw, double *partials, double *zrrr,
-                  double *xs = nullptr);
-    // p = z + (zrNew / zr) p per column, one launch (contiguous p, z)
-    void cgDirection(hipStream_t s, View<double> p, View<const double> z, const double *zrNew,
-                     const double *zr);
+                  const double *zr, const double *pw, double *partials, double *zrrr);
+    // p = d o r + (zrNew / zr) p per column, one launch (contiguous p, r)
+    void cgDirection(hipStream_t s, View<double> p, View<const double> r, const double *d,
+                     const double *zrNew, const double *zr);
     // Plain Chebyshev degree step, fused (ChebyshevFilter.t.cpp:96-129):
     //   t  = Minv hx  (diag rows < nC: dinv o hx; enriched rows: given in tE)
     //   s1 = alpha t + beta xk;  xprev = s1 + gamma xprev
@@ -173,6 +176,11 @@ namespace dfx
     template <class T>
     void slotSum(hipStream_t s, const dfx_op *op, const T *slots, View<T> x, View<T> y,
                  bool zeroX, const ResFuse<T> *rf);
+    // slotSum (rows held at zero cleared in both) and the column dots x.y into
+    // out (device) in one pass; partials: DOT_PARTIALS B doubles.  False
+    // (nothing done) for shapes it does not take: odd or more than 128 columns
+    bool slotSumDot(hipStream_t s, const dfx_op *op, const double *slots, View<double> x,
+                    View<double> y, double *partials, double *out);
     // out[s] = d[map[s]] (map[s] < nC) else 1, for every slot of a cell->dof map
     void gatherDiag(hipStream_t s, const double *d, const u32 *map, u64 n, u32 nC,
                     double *out);

@@ -1295,11 +1295,11 @@ extern "C"
       double *coef = workDoubles(ctx, "cgs.coef", 4 * (size_t)B);
       // device dots: z.r (two, alternating), p.w, r.r; partial sums
       double *dots = workDoubles(ctx, "cgs.dots", 4 * (size_t)B);
-      double *part = workDoubles(ctx, "cgs.part", 2048 * (size_t)B);
+      double *part = workDoubles(ctx, "cgs.part", k::DOT_PARTIALS * (size_t)B);
       double *dZr = dots, *dZrNew = dots + B, *dPw = dots + 2 * B, *dRr = dots + 3 * B;
       // a Jacobi preconditioner (diagonal, no constraints, no enriched block)
-      // lets one launch do the updates of x, r, z and the dots z.r, r.r and
-      // one more form beta and the search direction (the same bits;
+      // lets one launch do the updates of x and r and the dots z.r, r.r and
+      // one more form beta, z and the search direction (the same bits;
       // DFX_FUSE_CG=0 keeps the separate launches); z.r and r.r of an
       // iteration land side by side in one of two 2B slots
       const char *fuseEnv = getenv("DFX_FUSE_CG");
@@ -1308,7 +1308,6 @@ extern "C"
       double *slots = fusedCG ? workDoubles(ctx, "cgs.zrrr", 4 * (size_t)B) : nullptr;
       if (fusedCG)
         dZr = slots;
-      k::convert<double, double>(s, x, cv(xo));
       std::vector<double> bNorm(B), rNorm(B);
       colDotsView<double>(ctx, cv(b), cv(b), bNorm.data());
       for (auto &v : bNorm)
@@ -1330,7 +1329,10 @@ extern "C"
         {
           xs[0] = workView<double>(ctx, "cgs.xs0", N, B);
           xs[1] = workView<double>(ctx, "cgs.xs1", N, B);
+          if (fusedCG) // iteration k's x is xs[k % 2]
+            x = xs[0];
         }
+      k::convert<double, double>(s, x, cv(xo));
       PinnedDoubles hr(2 * (size_t)B);
       EventPair     ev;
       auto check = [&](u32 k) {
@@ -1381,15 +1383,19 @@ extern "C"
           else
             {
               // z.r of this iteration is the previous iteration's z.r_new
-              applyOp<double>(A, pv, w);
-              k::colDots<double>(s, cv(pv), cv(w), part, dPw);
+              if (!applyDot(A, pv, w, part, dPw))
+                {
+                  applyOp<double>(A, pv, w);
+                  k::colDots<double>(s, cv(pv), cv(w), part, dPw);
+                }
             }
           if (iter > 0 && fusedCG)
             {
               double *next = dZr == slots ? slots + 2 * B : slots;
-              k::cgUpdate(s, x, r, z, cv(pv), cv(w), pc->diag.as<double>(), dZr, dPw, part,
-                          next, pipe ? xs[iter % 2].p : nullptr);
-              k::cgDirection(s, pv, cv(z), next, dZr);
+              View<double> xn   = pipe ? xs[iter % 2] : x;
+              k::cgUpdate(s, x, xn, r, cv(pv), cv(w), pc->diag.as<double>(), dZr, dPw, part, next);
+              k::cgDirection(s, pv, cv(r), pc->diag.as<double>(), next, dZr);
+              x = xn;
               dZr = next;
               dRr = next + B;
             }
@@ -1410,7 +1416,7 @@ extern "C"
             k::colDots<double>(s, cv(r), cv(r), part, dRr);
           // r.r of the iteration to pinned memory; pipelined, x as it stands
           // now is kept for the copy to the output
-          if (pipe && !(fusedCG && iter > 0)) // the fused update wrote it
+          if (pipe && !fusedCG) // the fused update writes there
             k::convert<double, double>(s, xs[iter % 2], cv(x));
           DFX_HIP(hipMemcpyAsync(hr.p + (size_t)(iter % 2) * B, dRr, B * sizeof(double),
                                  hipMemcpyDeviceToHost, s));
