@@ -234,8 +234,10 @@ namespace dfx
     u32 nc;      // classical dofs (rows scattered directly)
     u32 mapOff;  // offset into the cell->dof map
     u32 enrOff;  // first row of this cell's enriched partials in the yE buffer
-    u64 fragOff64; // offset (elements) of the cell's FP64 fragment-ordered matrix
-    u64 fragOff32; // offset (elements) of the cell's FP32 fragment-ordered matrix
+    // offsets (elements) of the cell's FP64 and FP32 fragment-ordered matrices;
+    // cells with the same matrix share them
+    u64 fragOff64;
+    u64 fragOff32;
     u32 rowLo;     // smallest classical dof of the cell (buffer base row)
     u32 pad_;
   };
@@ -306,6 +308,7 @@ struct dfx_op
   std::vector<dfx::u64> hMatOffset;             // raw (caller) layout offsets
   std::vector<dfx::u32> hOrder;                 // launch order -> caller cell
   std::vector<dfx::CellMeta> hMeta;             // launch order
+  std::vector<dfx::u32> hSlotPos;               // slot order -> launch position
   std::vector<dfx::Launch> launches64, launches32;
   dfx::u64 fragLen64 = 0, fragLen32 = 0;
   dfx::DevBuf map, meta, frag64, frag32;

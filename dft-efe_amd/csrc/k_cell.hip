@@ -24,13 +24,13 @@ namespace dfx
       }
 
       template <class T>
-      __global__ void repackK(const CellMeta *meta, const u32 *order,
+      __global__ void repackK(const CellMeta *meta, const u32 *pos, const u32 *order,
                               const double *raw, const u64 *rawOff, T *frag)
       {
         constexpr int G  = Mfma<T>::G;
         constexpr int KB = 4 * G;
-        const CellMeta cm = meta[blockIdx.x];
-        const u32      e  = order[blockIdx.x];
+        const CellMeta cm = meta[pos[blockIdx.x]];
+        const u32      e  = order[pos[blockIdx.x]];
         const int      n  = (int)cm.n;
         const int      mt = (n + 15) >> 4;
         const int      nkb  = (n + KB - 1) / KB;
@@ -49,6 +49,52 @@ namespace dfx
             const int kk   = kb * KB + G * (lane >> 4) + s;
             F[idx] = (j < n && kk < n) ? (T)A[(u64)kk + (u64)n * j] : (T)0;
           }
+      }
+
+
+      // content hash of every cell's matrix (words mixed with their place), one
+      // workgroup per cell
+      __global__ __launch_bounds__(256) void cellHashK(const u64 *__restrict__ raw,
+                                                       const u64 *__restrict__ off,
+                                                       u64 *__restrict__ out)
+      {
+        __shared__ u64 sm[256];
+        const u64      o = off[blockIdx.x], n = off[blockIdx.x + 1] - o;
+        u64            acc = 0;
+        for (u64 i = threadIdx.x; i < n; i += 256)
+          {
+            u64 z = raw[o + i] + (i + 1) * 0x9e3779b97f4a7c15ull; // splitmix64 finalizer
+            z     = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
+            z     = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
+            acc += z ^ (z >> 31);
+          }
+        sm[threadIdx.x] = acc;
+        __syncthreads();
+        for (int w = 128; w > 0; w >>= 1)
+          {
+            if ((int)threadIdx.x < w)
+              sm[threadIdx.x] += sm[threadIdx.x + w];
+            __syncthreads();
+          }
+        if (threadIdx.x == 0)
+          out[blockIdx.x] = sm[0];
+      }
+
+      // differs[b] = 1 when cells a[b] and c[b] (of one size) differ in any bit
+      __global__ __launch_bounds__(256) void cellDiffersK(const u64 *__restrict__ raw,
+                                                          const u64 *__restrict__ off,
+                                                          const u32 *__restrict__ a,
+                                                          const u32 *__restrict__ c,
+                                                          u32 *__restrict__ differs)
+      {
+        const u64 oa = off[a[blockIdx.x]], oc = off[c[blockIdx.x]],
+                  n  = off[a[blockIdx.x] + 1] - oa;
+        int diff = 0;
+        for (u64 i = threadIdx.x; i < n; i += 256)
+          diff |= raw[oa + i] != raw[oc + i];
+        diff = __syncthreads_or(diff);
+        if (threadIdx.x == 0)
+          differs[blockIdx.x] = diff ? 1u : 0u;
       }
 
     } // namespace
@@ -118,28 +164,44 @@ namespace dfx
     }
 
     template <class T>
-    void repackCells(hipStream_t s, const dfx_op *op, const double *raw,
-                     const u64 *rawOffsets, T *frag)
+    void repackCells(hipStream_t s, const dfx_op *op, const std::vector<u32> &pos,
+                     const double *raw, const u64 *rawOffsets, T *frag)
     {
-      if (!op->nCells)
+      if (pos.empty())
         return;
       // the meta array is in launch order; `order` maps back to caller cells
-      DevBuf order;
+      DevBuf order, dpos;
       upload(order, op->hOrder, s);
-      repackK<T><<<op->nCells, 256, 0, s>>>(op->meta.as<CellMeta>(), order.as<u32>(),
-                                            raw, rawOffsets, frag);
+      upload(dpos, pos, s);
+      repackK<T><<<(u32)pos.size(), 256, 0, s>>>(op->meta.as<CellMeta>(), dpos.as<u32>(),
+                                                 order.as<u32>(), raw, rawOffsets, frag);
       checkLaunch("repackCells");
       DFX_HIP(hipStreamSynchronize(s));
+    }
+
+    void cellHashes(hipStream_t s, u32 nCells, const double *raw, const u64 *rawOffsets,
+                    u64 *out)
+    {
+      cellHashK<<<nCells, 256, 0, s>>>(reinterpret_cast<const u64 *>(raw), rawOffsets, out);
+      checkLaunch("cellHashes");
+    }
+
+    void cellsDiffer(hipStream_t s, u32 n, const double *raw, const u64 *rawOffsets, const u32 *a,
+                     const u32 *b, u32 *differs)
+    {
+      cellDiffersK<<<n, 256, 0, s>>>(reinterpret_cast<const u64 *>(raw), rawOffsets, a, b,
+                                     differs);
+      checkLaunch("cellsDiffer");
     }
 
     template void enrichedReduce<double>(hipStream_t, const dfx_op *, const double *,
                                          View<double>);
     template void enrichedReduce<float>(hipStream_t, const dfx_op *, const float *,
                                         View<float>);
-    template void repackCells<double>(hipStream_t, const dfx_op *, const double *,
-                                      const u64 *, double *);
-    template void repackCells<float>(hipStream_t, const dfx_op *, const double *,
-                                     const u64 *, float *);
+    template void repackCells<double>(hipStream_t, const dfx_op *, const std::vector<u32> &,
+                                      const double *, const u64 *, double *);
+    template void repackCells<float>(hipStream_t, const dfx_op *, const std::vector<u32> &,
+                                     const double *, const u64 *, float *);
     DFX_INST_CELL(double)
   } // namespace k
 } // namespace dfx

@@ -193,10 +193,17 @@ namespace dfx
     // out[mapOff_e + i] = A_e(i, i) from the FP64 fragment-ordered matrices
     // (caller slot order)
     void cellDiag(hipStream_t s, const dfx_op *op, double *out);
-    // repack raw column-major cell matrices (device) into the fragment layout
+    // repack the raw column-major matrices (device) of the cells at launch
+    // positions `pos` into the fragment layout
     template <class T>
-    void repackCells(hipStream_t s, const dfx_op *op, const double *raw,
-                     const u64 *rawOffsets, T *frag);
+    void repackCells(hipStream_t s, const dfx_op *op, const std::vector<u32> &pos,
+                     const double *raw, const u64 *rawOffsets, T *frag);
+    // out[e]: content hash of cell e's raw matrix
+    void cellHashes(hipStream_t s, u32 nCells, const double *raw, const u64 *rawOffsets, u64 *out);
+    // differs[i]: whether the raw matrices of cells a[i] and b[i] (of one size)
+    // differ in any bit
+    void cellsDiffer(hipStream_t s, u32 n, const double *raw, const u64 *rawOffsets, const u32 *a,
+                     const u32 *b, u32 *differs);
 
     // --------------------------------------------------------- dense
     // S (n x n, column-major, FP64) = X^T Y over all N rows; deterministic

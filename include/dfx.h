@@ -215,8 +215,10 @@ typedef struct dfx_op_info
   uint32_t maxCellDofs;
   uint64_t sumNe;       /* sum_e n_e */
   uint64_t sumNe2;      /* sum_e n_e^2 */
-  uint64_t matBytesF64; /* device bytes of the FP64 cell-matrix store */
-  uint64_t matBytesF32; /* device bytes of the FP32 cell-matrix store (0 if none) */
+  /* device bytes of the FP64 and FP32 (0 if none) stores of the distinct cell
+   * matrices: cells with bitwise equal matrices share one */
+  uint64_t matBytesF64;
+  uint64_t matBytesF32;
 } dfx_op_info;
 int dfx_op_get_info(const dfx_op *op, dfx_op_info *info);
 /* Download the device-resident cell->dof map in the caller's cell order

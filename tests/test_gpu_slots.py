@@ -126,3 +126,57 @@ def test_rows_of_many_cells_and_of_none(ctx, cells):
         ref[cmap[e]] += A[e] @ X[cmap[e]]
     # sums of at most `cells` + 2 products per entry
     assert np.abs(Y.to_numpy() - ref).max() <= (cells + 2) * 2.0 ** -52 * cells
+
+
+@pytest.mark.parametrize("dtype", [dfx.F64, dfx.F32])
+def test_cells_with_the_same_matrix_share_it(ctx, probs, dtype):
+    """Cells of bitwise equal matrices share one stored copy; one that differs in
+    a single bit does not, and update_cells may turn either into the other;
+    against numpy's cell-by-cell sums and a freshly made operator."""
+    P = probs["c1"]
+    d = P.arrays()
+    ops = Ops(ctx, P)
+    n = int(d["cellNdofs"][0])
+    nc = len(d["cellNdofs"])
+    K0 = d["K"][:n * n]
+    uniform = np.tile(K0, nc)
+    one_bit = uniform.copy()
+    one_bit[n * n * (nc // 2) + 5] = np.nextafter(one_bit[n * n * (nc // 2) + 5], 10.0)
+    distinct = (uniform.reshape(nc, -1) * (1.0 + np.arange(nc)[:, None] / 64.0)).ravel()
+    npd = np.float64 if dtype == dfx.F64 else np.float32
+    X = guess(P, 10, seed=4).astype(npd)
+    off = np.concatenate([[0], np.cumsum(d["cellNdofs"])]).astype(int)
+    cons_rows = d["rows"]
+
+    def reference(mats):
+        Z, Y = X.astype(np.float64), np.zeros((P.nDofs, 10))
+        Z[cons_rows] = 0
+        for e in range(nc):
+            i = d["cellMap"][off[e]:off[e + 1]].astype(int)
+            np.add.at(Y, i, mats[e * n * n:(e + 1) * n * n].reshape(n, n) @ Z[i])
+        Y[cons_rows] = 0
+        return Y
+
+    def result(op):
+        Y = dfx.MultiVector(ctx, P.nDofs, 10, dtype)
+        op.apply(mv(ctx, X, dtype), Y)
+        Yc = dfx.MultiVector(ctx, P.nDofs, 10, dtype)
+        op.apply_noalloc(mv(ctx, X, dtype), Yc)
+        assert np.array_equal(Y.to_numpy(), Yc.to_numpy())
+        return Y.to_numpy()
+
+    def make(mats):
+        return dfx.CellOperator(ctx, d["cellNdofs"], d["cellMap"], mats, P.nDofs, P.nClassical,
+                                ops.cons, keep_fp32=True)
+
+    unit = make(uniform).info()["matBytesF64"]
+    assert make(one_bit).info()["matBytesF64"] == 2 * unit
+    assert make(distinct).info()["matBytesF64"] == nc * unit
+    op = make(uniform)
+    # n-term products and up to 8 cells added per row, each rounded in `dtype`
+    eps = np.finfo(npd).eps
+    for mats in (uniform, distinct, one_bit, uniform):
+        op.update_cells(mats)
+        got, ref = result(op), reference(mats)
+        assert np.abs(got - ref).max() <= (n + 10) * eps * np.abs(mats).max() * n
+        assert np.array_equal(got, result(make(mats)))
