@@ -219,6 +219,12 @@ namespace dfx
       const size_t m = (n + 15) / 16 * 16;
       return m * m;
     }
+    // Q = L^-T with L the Cholesky factor of S (n x n column-major, n <= 256, lower
+    // triangle read); L: scratch of cholScratch(n) doubles; *info (device)
+    // becomes 0, or 1 when a diagonal entry of the factor is below 1e-14 or not
+    // a number (Q is not usable then)
+    inline size_t cholScratch(u32 n) { return rotateScratch(n) + 16 * ((n + 15) / 16 * 16); }
+    void cholInverse(hipStream_t s, const double *S, u32 n, double *L, double *Q, int *info);
     // partial sums of gram (ld: the larger leading dimension)
     size_t gramPartialsNeeded(u32 N, u32 n, u32 ld);
   } // namespace k

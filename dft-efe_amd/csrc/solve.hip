@@ -539,7 +539,22 @@ namespace dfx
       double *S    = workDoubles(ctx, "cg.S", (size_t)n * n);
       double *part = workDoubles(ctx, "gram.part", k::gramPartialsNeeded(N, n, X.ld));
       k::gram(s, cv(X), cv(MX), part, k::gramPartialsNeeded(N, n, X.ld), S);
-      int *info = work(ctx, "info", 64).as<int>();
+      int    *info = work(ctx, "info", 64).as<int>();
+      double *qr   = workDoubles(ctx, "rot.qr", k::rotateScratch(n));
+      if (n <= 256)
+        {
+          // L, L^-1 and its transpose on the device; the factor's diagonal is
+          // checked before X is rotated (OrthonormalizationFunctions.t.cpp:274-306)
+          double *Q = workDoubles(ctx, "cg.Q", (size_t)n * n);
+          int     hinfo = 0;
+          k::cholInverse(s, S, n, workDoubles(ctx, "cg.L", k::cholScratch(n)), Q, info);
+          DFX_HIP(hipMemcpyAsync(&hinfo, info, sizeof(int), hipMemcpyDeviceToHost, s));
+          DFX_HIP(hipStreamSynchronize(s));
+          if (hinfo != 0)
+            return DFX_ORTHO_LAPACK_ERROR;
+          rotate64(ctx, cv(X), Q, Xo, qr);
+          return 0;
+        }
       rocblas_status st;
       {
         CaptureLock lk(captureMutex());
@@ -583,7 +598,6 @@ namespace dfx
         for (u32 i = j; i < n; ++i)
           hQ[j + (size_t)n * i] = hS[i + (size_t)n * j];
       toDevice(ctx, Q, hQ.data(), hQ.size());
-      double *qr = workDoubles(ctx, "rot.qr", k::rotateScratch(n));
       rotate64(ctx, cv(X), Q, Xo, qr);
       return 0;
     }

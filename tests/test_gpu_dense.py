@@ -64,3 +64,30 @@ def test_columns_past_the_block_do_not_enter(ctx):
     X[4, 3] = np.nan
     rc = dfx.cholesky_gram_schmidt(ctx, dfx.MultiVector.from_numpy(ctx, X), Xo, diagonal(ctx, m))
     assert rc != 0                                   # reported, as any failed factorization
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 40, 200, 256, 257])
+def test_rank_deficient_and_tiny_columns_are_reported(ctx, n):
+    """A zero column, a column below the factor's 1e-14 limit and (from two
+    columns on) equal columns fail; a column of norm 1e-13 does not."""
+    N = max(2 * n, 64)
+    rng = np.random.RandomState(n)
+    Q = np.linalg.qr(rng.uniform(-1, 1, (N, n)))[0]
+    M, Xo = diagonal(ctx, np.ones(N)), dfx.MultiVector(ctx, N, n)
+
+    def run(X):
+        return dfx.cholesky_gram_schmidt(ctx, dfx.MultiVector.from_numpy(ctx, X), Xo, M)
+
+    assert run(Q) == 0
+    for j in sorted({0, n // 2, n - 1}):
+        for scale, ok in ((0.0, False), (1e-15, False), (1e-13, True)):
+            X = Q.copy()
+            X[:, j] *= scale
+            assert (run(X) == 0) == ok, (n, j, scale)
+        if j:
+            X = Q.copy()
+            X[:, j] = 0.0
+            X[0, j] = -0.0
+            assert run(X) != 0
+    assert run(Q) == 0                       # a failure leaves nothing behind
+    assert np.abs(Xo.to_numpy() - Q).max() <= 50 * EPS * (n + np.sqrt(N))
