@@ -225,6 +225,13 @@ namespace dfx
     // a number (Q is not usable then)
     inline size_t cholScratch(u32 n) { return rotateScratch(n) + 16 * ((n + 15) / 16 * 16); }
     void cholInverse(hipStream_t s, const double *S, u32 n, double *L, double *Q, int *info);
+    // dsytrd (lower) of A (n x n column-major): reflectors below the diagonal,
+    // d, e and tau on the device
+    constexpr u32 TRIDIAG_MAX = 128;
+    void tridiagonalize(hipStream_t s, double *A, u32 n, double *d, double *e, double *tau);
+    // V = Q C with Q from the reflectors in A and tau (dormtr, lower, n <= 256)
+    void applyReflectors(hipStream_t s, const double *A, const double *tau, u32 n, const double *C,
+                         double *V);
     // partial sums of gram (ld: the larger leading dimension)
     size_t gramPartialsNeeded(u32 N, u32 n, u32 ld);
   } // namespace k

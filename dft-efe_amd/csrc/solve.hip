@@ -614,16 +614,37 @@ namespace dfx
       double *S    = workDoubles(ctx, "rr.S", (size_t)n * n);
       double *part = workDoubles(ctx, "gram.part", k::gramPartialsNeeded(N, n, X.ld));
       k::gram(s, cv(X), cv(HX), part, k::gramPartialsNeeded(N, n, X.ld), S);
-      double *D    = workDoubles(ctx, "rr.D", 2 * (size_t)n);
+      // eigenvectors in V: dsyevd, up to 256 columns with this library's
+      // reduction (up to 128) and return of the eigenvectors around the
+      // library's divide and conquer
+      double *D    = workDoubles(ctx, "rr.D", 3 * (size_t)n);
+      double *V    = workDoubles(ctx, "rr.V", (size_t)n * n);
       int    *info = work(ctx, "info", 64).as<int>();
-      rocblas_status st;
-      {
-        CaptureLock lk(captureMutex());
-        st = rocsolver_dsyevd(ctx->blas, rocblas_evect_original, rocblas_fill_lower,
-                           (rocblas_int)n, S, (rocblas_int)n, D, D + n, info);
-      }
-      if (st != rocblas_status_success)
-        throw Error(DFX_E_HIP, "rocsolver_dsyevd failed");
+      if (n >= 2 && n <= 256)
+        {
+          double *E = D + n, *tau = D + 2 * (size_t)n;
+          double *C = workDoubles(ctx, "rr.C", (size_t)n * n);
+          if (n <= k::TRIDIAG_MAX)
+            k::tridiagonalize(s, S, n, D, E, tau);
+          CaptureLock lk(captureMutex());
+          if (n > k::TRIDIAG_MAX &&
+              rocsolver_dsytrd(ctx->blas, rocblas_fill_lower, (rocblas_int)n, S, (rocblas_int)n, D,
+                               E, tau) != rocblas_status_success)
+            throw Error(DFX_E_HIP, "rocsolver_dsytrd failed");
+          if (rocsolver_dstedc(ctx->blas, rocblas_evect_tridiagonal, (rocblas_int)n, D, E, C,
+                               (rocblas_int)n, info) != rocblas_status_success)
+            throw Error(DFX_E_HIP, "rocsolver_dstedc failed");
+          k::applyReflectors(s, S, tau, n, C, V);
+        }
+      else
+        {
+          CaptureLock lk(captureMutex());
+          if (rocsolver_dsyevd(ctx->blas, rocblas_evect_original, rocblas_fill_lower,
+                               (rocblas_int)n, S, (rocblas_int)n, D, D + n, info) !=
+              rocblas_status_success)
+            throw Error(DFX_E_HIP, "rocsolver_dsyevd failed");
+          DFX_HIP(hipMemcpyAsync(V, S, (size_t)n * n * sizeof(double), hipMemcpyDeviceToDevice, s));
+        }
       int hinfo = 0;
       DFX_HIP(hipMemcpyAsync(&hinfo, info, sizeof(int), hipMemcpyDeviceToHost, s));
       DFX_HIP(hipMemcpyAsync(eig, D, n * sizeof(double), hipMemcpyDeviceToHost, s));
@@ -631,7 +652,7 @@ namespace dfx
       if (hinfo != 0)
         return DFX_EIG_LAPACK_ERROR;
       double *qr = workDoubles(ctx, "rot.qr", k::rotateScratch(n));
-      rotate64(ctx, cv(X), S, Xo, qr);
+      rotate64(ctx, cv(X), V, Xo, qr);
       return 0;
     }
 
@@ -836,7 +857,7 @@ namespace dfx
           // parent->child values that apply would give them)
           const u32    N    = XV.N;
           const size_t by   = (size_t)N * n * sizeof(double);
-          double      *S    = workDoubles(ctx, "rr.S", (size_t)n * n);
+          double      *S    = workDoubles(ctx, "rr.V", (size_t)n * n);
           double      *qr   = workDoubles(ctx, "rot.qr", k::rotateScratch(n));
           cs->kpHX.ensure(by);
           cs->kpMX.ensure(by);

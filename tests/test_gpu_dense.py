@@ -16,7 +16,7 @@ def diagonal(ctx, d):
     return dfx.DiagonalOperator(ctx, d)
 
 
-@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 33, 63, 64, 65, 101, 112, 113, 128, 129, 200,
+@pytest.mark.parametrize("n", [1, 2, 3, 15, 16, 17, 32, 33, 63, 64, 65, 66, 101, 112, 113, 128, 129, 200,
                                208, 255, 256, 257])
 def test_orthonormalization_and_ritz_at_every_width(ctx, n):
     for N in sorted({n, n + 1, 1031, 4099}):
@@ -91,3 +91,21 @@ def test_rank_deficient_and_tiny_columns_are_reported(ctx, n):
             assert run(X) != 0
     assert run(Q) == 0                       # a failure leaves nothing behind
     assert np.abs(Xo.to_numpy() - Q).max() <= 50 * EPS * (n + np.sqrt(N))
+
+
+@pytest.mark.parametrize("n", [2, 3, 17, 65, 100, 128, 150])
+def test_projected_problems_with_nothing_to_reflect(ctx, n):
+    """Diagonal and block-diagonal projected matrices (zero columns below the
+    diagonal: reflectors of zero length), repeated values and a wide range of
+    magnitudes: eigenvalues to the matrix norm, orthonormal vectors."""
+    N = n + 5
+    V = dfx.MultiVector(ctx, N, n)
+    for h in (np.arange(N) * 1.0, np.ones(N), 10.0 ** np.linspace(-9, 3, N),
+              np.where(np.arange(N) % 2, 1e-30, 2.0)):
+        for X in (np.eye(N, n), np.eye(N, n)[:, ::-1].copy()):
+            rc, ev = dfx.rayleigh_ritz(ctx, diagonal(ctx, h), dfx.MultiVector.from_numpy(ctx, X), V)
+            assert rc == 0
+            want = np.sort((X * (h[:, None] * X)).sum(axis=0))
+            assert np.abs(ev - want).max() <= 20 * n * EPS * max(np.abs(want).max(), 1e-300)
+            v = V.to_numpy()
+            assert np.abs(v.T @ v - np.eye(n)).max() <= 20 * n * EPS
