@@ -362,25 +362,45 @@ namespace dfx
       // one workgroup per column: thread t adds partials t, t + 256, ... in
       // order, then a fixed-shape tree over the 256 sums (deterministic; the
       // partial count depends on N only, so a column's result does not
-      // depend on how many columns share the call)
+      // depend on how many columns share the call).  Columns from hostFrom on
+      // also go to host (pinned memory).  All latency: eight loads are in
+      // flight together, the tree's last six levels stay in one wave
       __global__ __launch_bounds__(256) void colDotsFinalK(const double *partials, u32 nBlocks,
-                                                           u32 B, double *out)
+                                                           u32 B, double *out, double *host,
+                                                           u32 hostFrom)
       {
         __shared__ double red[256];
         const u32 j = blockIdx.x;
         double    s = 0.0;
-        for (u32 b = threadIdx.x; b < nBlocks; b += 256)
-          s += partials[(u64)b * B + j];
+        for (u32 b = threadIdx.x; b < nBlocks; b += 8 * 256)
+          {
+            double v[8];
+#pragma unroll
+            for (u32 k = 0; k < 8; ++k)
+              if (b + k * 256 < nBlocks)
+                v[k] = partials[(u64)(b + k * 256) * B + j];
+#pragma unroll
+            for (u32 k = 0; k < 8; ++k)
+              if (b + k * 256 < nBlocks)
+                s += v[k];
+          }
         red[threadIdx.x] = s;
         __syncthreads();
-        for (u32 w = 128; w > 0; w >>= 1)
-          {
-            if (threadIdx.x < w)
-              red[threadIdx.x] += red[threadIdx.x + w];
-            __syncthreads();
-          }
+        if (threadIdx.x >= 64)
+          return;
+        // the tree's levels 128 and 64, then within the wave
+        s = (red[threadIdx.x] + red[threadIdx.x + 128]) +
+            (red[threadIdx.x + 64] + red[threadIdx.x + 192]);
+#pragma unroll
+        for (int w = 32; w > 0; w >>= 1)
+          s += __shfl_down(s, w);
         if (threadIdx.x == 0)
-          out[j] = red[0];
+          {
+            out[j] = s;
+            if (host && j >= hostFrom)
+              __hip_atomic_store(host + (j - hostFrom), s, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_SYSTEM);
+          }
       }
 
       template <class T>
@@ -753,9 +773,10 @@ namespace dfx
       u32 dotBlocks(u32 N) { return std::max(1u, std::min(1024u, (u32)(((u64)N + 63) / 64))); }
     } // namespace
 
-    void colDotsFinal(hipStream_t s, const double *partials, u32 nBlocks, u32 B, double *out)
+    void colDotsFinal(hipStream_t s, const double *partials, u32 nBlocks, u32 B, double *out,
+                      double *host, u32 hostFrom)
     {
-      colDotsFinalK<<<B, 256, 0, s>>>(partials, nBlocks, B, out);
+      colDotsFinalK<<<B, 256, 0, s>>>(partials, nBlocks, B, out, host, hostFrom);
       checkLaunch("colDotsFinal");
     }
 
@@ -805,7 +826,8 @@ namespace dfx
 
     void cgUpdate(hipStream_t s, View<double> x, View<double> xn, View<double> r,
                   View<const double> p, View<const double> w, const double *d,
-                  const double *zr, const double *pw, double *partials, double *zrrr)
+                  const double *zr, const double *pw, double *partials, double *zrrr,
+                  double *rrHost)
     {
       const u32 B = x.B, N = x.N;
       if (!B)
@@ -827,7 +849,7 @@ namespace dfx
       else
         go(cgUpdateK<64>);
       checkLaunch("cgUpdate");
-      colDotsFinal(s, partials, nBlocks, 2 * B, zrrr);
+      colDotsFinal(s, partials, nBlocks, 2 * B, zrrr, rrHost, B);
     }
 
     void cgDirection(hipStream_t s, View<double> p, View<const double> r, const double *d,

@@ -37,8 +37,10 @@ namespace dfx
     void colDots(hipStream_t s, View<const T> x, View<const T> y, double *partials,
                  double *out);
 
-    // the second pass of the column dots: out[j] = sum of nBlocks partials
-    void colDotsFinal(hipStream_t s, const double *partials, u32 nBlocks, u32 B, double *out);
+    // the second pass of the column dots: out[j] = sum of nBlocks partials; the
+    // columns from hostFrom on also to host (pinned, coherent) where given
+    void colDotsFinal(hipStream_t s, const double *partials, u32 nBlocks, u32 B, double *out,
+                      double *host = nullptr, u32 hostFrom = 0);
     constexpr u32 DOT_PARTIALS = 2048; // rows of partial sums a CG work buffer holds
 
     // out[j] = sum_i (a1 a[j] x_ij + b1 b[j] y_ij)^2 without forming the
@@ -50,11 +52,12 @@ namespace dfx
     // PCG iteration with a Jacobi (diagonal d) preconditioner, fused
     // (CGLinearSolver.t.cpp:68-313): alpha = zr / pw per column; xn = x + alpha
     // p; r -= alpha w; zrrr[0, B) = z.r, zrrr[B, 2B) = r.r with z = d o r, the
-    // bits of the separate launches.  partials: DOT_PARTIALS B doubles; xn may
-    // be x
+    // bits of the separate launches, r.r also to rrHost (pinned, coherent).
+    // partials: DOT_PARTIALS B doubles; xn may be x
     void cgUpdate(hipStream_t s, View<double> x, View<double> xn, View<double> r,
                   View<const double> p, View<const double> w, const double *d,
-                  const double *zr, const double *pw, double *partials, double *zrrr);
+                  const double *zr, const double *pw, double *partials, double *zrrr,
+                  double *rrHost);
     // p = d o r + (zrNew / zr) p per column, one launch (contiguous p, r)
     void cgDirection(hipStream_t s, View<double> p, View<const double> r, const double *d,
                      const double *zrNew, const double *zr);

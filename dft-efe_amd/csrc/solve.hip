@@ -64,14 +64,15 @@ namespace dfx
 
     // small host -> device upload; completes before returning, so the host
     // buffer (often a temporary) may be released right after
-    // pinned host doubles (asynchronous device-to-host copies)
+    // pinned host doubles, coherent (asynchronous device-to-host copies and
+    // what kernels write themselves)
     struct PinnedDoubles
     {
       double *p = nullptr;
       explicit PinnedDoubles(size_t n)
       {
         DFX_HIP(hipHostMalloc(reinterpret_cast<void **>(&p), std::max<size_t>(n, 1) * sizeof(double),
-                              hipHostMallocDefault));
+                              hipHostMallocMapped | hipHostMallocCoherent));
       }
       ~PinnedDoubles()
       {
@@ -1428,7 +1429,8 @@ extern "C"
             {
               double *next = dZr == slots ? slots + 2 * B : slots;
               View<double> xn   = pipe ? xs[iter % 2] : x;
-              k::cgUpdate(s, x, xn, r, cv(pv), cv(w), pc->diag.as<double>(), dZr, dPw, part, next);
+              k::cgUpdate(s, x, xn, r, cv(pv), cv(w), pc->diag.as<double>(), dZr, dPw, part, next,
+                          hr.p + (size_t)(iter % 2) * B);
               k::cgDirection(s, pv, cv(r), pc->diag.as<double>(), next, dZr);
               x = xn;
               dZr = next;
@@ -1453,8 +1455,9 @@ extern "C"
           // now is kept for the copy to the output
           if (pipe && !fusedCG) // the fused update writes there
             k::convert<double, double>(s, xs[iter % 2], cv(x));
-          DFX_HIP(hipMemcpyAsync(hr.p + (size_t)(iter % 2) * B, dRr, B * sizeof(double),
-                                 hipMemcpyDeviceToHost, s));
+          if (!(fusedCG && iter > 0)) // the fused update writes there
+            DFX_HIP(hipMemcpyAsync(hr.p + (size_t)(iter % 2) * B, dRr, B * sizeof(double),
+                                   hipMemcpyDeviceToHost, s));
           DFX_HIP(hipEventRecord(ev.e[iter % 2], s));
           if (!pipe || iter > 0)
             {
