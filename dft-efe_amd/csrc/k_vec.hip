@@ -365,6 +365,7 @@ namespace dfx
       // depend on how many columns share the call).  Columns from hostFrom on
       // also go to host (pinned memory).  All latency: eight loads are in
       // flight together, the tree's last six levels stay in one wave
+      // (1024 partials, 16 columns: 4.7 -> 4.06 us)
       __global__ __launch_bounds__(256) void colDotsFinalK(const double *partials, u32 nBlocks,
                                                            u32 B, double *out, double *host,
                                                            u32 hostFrom)
