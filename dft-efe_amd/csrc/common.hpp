@@ -5,6 +5,7 @@
 
 #include <atomic>
 #include <cstdint>
+#include <cstdlib>
 #include <cstring>
 #include <map>
 #include <memory>
@@ -69,6 +70,14 @@ namespace dfx
   using CaptureLock = std::lock_guard<std::recursive_mutex>;
 
   // ------------------------------------------------------------ buffers
+  // DFX_MAX_ALLOC_BYTES (read on every allocation): a buffer of more bytes is
+  // refused as out of memory
+  inline size_t allocLimit()
+  {
+    const char *e = getenv("DFX_MAX_ALLOC_BYTES");
+    return e && *e ? (size_t)strtoull(e, nullptr, 10) : (size_t)-1;
+  }
+
   // Owning device allocation (hipMalloc / hipFree).
   struct DevBuf
   {
@@ -101,8 +110,17 @@ namespace dfx
       release();
       if (n)
         {
-          CaptureLock lk(captureMutex());
-          DFX_HIP(hipMalloc(&p, n));
+          if (n > allocLimit())
+            throw Error(DFX_E_OOM, "device allocation above DFX_MAX_ALLOC_BYTES");
+          CaptureLock      lk(captureMutex());
+          const hipError_t e = hipMalloc(&p, n);
+          if (e != hipSuccess)
+            {
+              p = nullptr;
+              (void)hipGetLastError(); // not reported again by the next launch's check
+              throw Error(e == hipErrorOutOfMemory ? DFX_E_OOM : DFX_E_HIP,
+                          std::string("hipMalloc: ") + hipGetErrorString(e));
+            }
         }
       bytes = n;
     }

@@ -164,19 +164,13 @@ namespace dfx
     }
 
     template <class T>
-    void repackCells(hipStream_t s, const dfx_op *op, const std::vector<u32> &pos,
+    void repackCells(hipStream_t s, const dfx_op *op, u32 nPos, const u32 *pos, const u32 *order,
                      const double *raw, const u64 *rawOffsets, T *frag)
     {
-      if (pos.empty())
+      if (!nPos)
         return;
-      // the meta array is in launch order; `order` maps back to caller cells
-      DevBuf order, dpos;
-      upload(order, op->hOrder, s);
-      upload(dpos, pos, s);
-      repackK<T><<<(u32)pos.size(), 256, 0, s>>>(op->meta.as<CellMeta>(), dpos.as<u32>(),
-                                                 order.as<u32>(), raw, rawOffsets, frag);
+      repackK<T><<<nPos, 256, 0, s>>>(op->meta.as<CellMeta>(), pos, order, raw, rawOffsets, frag);
       checkLaunch("repackCells");
-      DFX_HIP(hipStreamSynchronize(s));
     }
 
     void cellHashes(hipStream_t s, u32 nCells, const double *raw, const u64 *rawOffsets,
@@ -198,9 +192,9 @@ namespace dfx
                                          View<double>);
     template void enrichedReduce<float>(hipStream_t, const dfx_op *, const float *,
                                         View<float>);
-    template void repackCells<double>(hipStream_t, const dfx_op *, const std::vector<u32> &,
+    template void repackCells<double>(hipStream_t, const dfx_op *, u32, const u32 *, const u32 *,
                                       const double *, const u64 *, double *);
-    template void repackCells<float>(hipStream_t, const dfx_op *, const std::vector<u32> &,
+    template void repackCells<float>(hipStream_t, const dfx_op *, u32, const u32 *, const u32 *,
                                      const double *, const u64 *, float *);
     DFX_INST_CELL(double)
   } // namespace k

@@ -196,10 +196,11 @@ namespace dfx
     // out[mapOff_e + i] = A_e(i, i) from the FP64 fragment-ordered matrices
     // (caller slot order)
     void cellDiag(hipStream_t s, const dfx_op *op, double *out);
-    // repack the raw column-major matrices (device) of the cells at launch
-    // positions `pos` into the fragment layout
+    // repack the raw column-major matrices (device) of the nPos cells at launch
+    // positions `pos` (device) into the fragment layout; order (device): launch
+    // position -> caller cell.  Allocates nothing
     template <class T>
-    void repackCells(hipStream_t s, const dfx_op *op, const std::vector<u32> &pos,
+    void repackCells(hipStream_t s, const dfx_op *op, u32 nPos, const u32 *pos, const u32 *order,
                      const double *raw, const u64 *rawOffsets, T *frag);
     // out[e]: content hash of cell e's raw matrix
     void cellHashes(hipStream_t s, u32 nCells, const double *raw, const u64 *rawOffsets, u64 *out);

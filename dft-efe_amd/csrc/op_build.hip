@@ -447,14 +447,23 @@ namespace dfx
 
   namespace
   {
+    // Where the cell matrices of an upload go: per launch position the metadata
+    // with the fragment offsets, the launch positions whose matrices are stored
+    // (`stored`), and the stores' lengths
+    struct Placement
+    {
+      std::vector<CellMeta> meta;
+      std::vector<u32>      stored;
+      u64                   len64 = 0, len32 = 0;
+    };
+
     // Fragment offsets of the cell matrices, those of cells with the same
-    // matrix (bit for bit) shared, and the launch positions whose matrices are
-    // stored.  On a uniform mesh the mass and stiffness matrices of all
-    // unenriched cells are one matrix: their applies then read it from the L2
-    // instead of streaming a copy per cell (K apply of 16^3 cells at p = 3, 8
-    // columns FP64: cell kernel 29 -> 19 us; 134 MB of copies).  Candidates come
-    // from a content hash and are compared in full
-    std::vector<u32> placeCellMatrices(dfx_op *op, const double *raw, const u64 *rawOff)
+    // matrix (bit for bit) shared.  On a uniform mesh the mass and stiffness
+    // matrices of all unenriched cells are one matrix: their applies then read
+    // it from the L2 instead of streaming a copy per cell (K apply of 16^3 cells
+    // at p = 3, 8 columns FP64: cell kernel 29 -> 19 us; 134 MB of copies).
+    // Candidates come from a content hash and are compared in full
+    Placement placeCellMatrices(const dfx_op *op, const double *raw, const u64 *rawOff)
     {
       const u32   nCells = op->nCells;
       hipStream_t st     = op->ctx->stream;
@@ -491,45 +500,40 @@ namespace dfx
             if (!d[i])
               rep[a[i]] = b[i];
         }
-      std::vector<u32> stored, at(nCells, 0xffffffffu); // representative -> launch position
-      u64              f64 = 0, f32 = 0;
+      Placement P;
+      P.meta = op->hMeta;
+      std::vector<u32> at(nCells, 0xffffffffu); // representative -> launch position
       for (u32 q = 0; q < nCells; ++q)
         {
           u32 &r = at[rep[op->hOrder[q]]];
           if (r == 0xffffffffu)
             {
               r = q;
-              stored.push_back(q);
-              const u64 n = op->hMeta[q].n, mpad = 16 * ((n + 15) / 16);
-              op->hMeta[q].fragOff64 = f64;
-              op->hMeta[q].fragOff32 = f32;
-              f64 += mpad * (8 * ((n + 7) / 8));
-              f32 += mpad * (16 * ((n + 15) / 16));
+              P.stored.push_back(q);
+              const u64 n = P.meta[q].n, mpad = 16 * ((n + 15) / 16);
+              P.meta[q].fragOff64 = P.len64;
+              P.meta[q].fragOff32 = P.len32;
+              P.len64 += mpad * (8 * ((n + 7) / 8));
+              P.len32 += mpad * (16 * ((n + 15) / 16));
             }
           else
             {
-              op->hMeta[q].fragOff64 = op->hMeta[r].fragOff64;
-              op->hMeta[q].fragOff32 = op->hMeta[r].fragOff32;
+              P.meta[q].fragOff64 = P.meta[r].fragOff64;
+              P.meta[q].fragOff32 = P.meta[r].fragOff32;
             }
         }
-      op->fragLen64 = f64;
-      op->fragLen32 = f32;
-      upload(op->meta, op->hMeta, st);
-      if (op->slotsOk)
-        {
-          std::vector<CellMeta> meta(nCells);
-          for (u32 q = 0; q < nCells; ++q)
-            meta[q] = op->hMeta[op->hSlotPos[q]];
-          upload(op->metaSlots, meta, st);
-        }
-      return stored;
+      return P;
     }
   } // namespace
 
+  // Everything that can fail for want of memory comes first, into buffers of
+  // its own: a refused update leaves the operator as it was.  A store keeps its
+  // memory where its length stays the same (its old matrices are then
+  // overwritten by the last two launches)
   void uploadCellMatrices(dfx_op *op, const double *mats, bool device)
   {
     hipStream_t st = op->ctx->stream;
-    DevBuf      raw, rawOff;
+    DevBuf      raw, rawOff, order, stored, meta, metaSlots, new64, new32;
     const double *dmats = mats;
     if (!device)
       {
@@ -537,17 +541,38 @@ namespace dfx
         dmats = raw.as<double>();
       }
     upload(rawOff, op->hMatOffset, st);
-    ++op->gen;
-    const std::vector<u32> stored = placeCellMatrices(op, dmats, rawOff.as<u64>());
-    if (op->frag64.bytes != op->fragLen64 * sizeof(double))
-      op->frag64.alloc(op->fragLen64 * sizeof(double));
-    k::repackCells<double>(st, op, stored, dmats, rawOff.as<u64>(), op->frag64.as<double>());
-    if (op->hasF32)
+    Placement P = placeCellMatrices(op, dmats, rawOff.as<u64>());
+    upload(order, op->hOrder, st);
+    upload(stored, P.stored, st);
+    upload(meta, P.meta, st);
+    if (op->slotsOk)
       {
-        if (op->frag32.bytes != op->fragLen32 * sizeof(float))
-          op->frag32.alloc(op->fragLen32 * sizeof(float));
-        k::repackCells<float>(st, op, stored, dmats, rawOff.as<u64>(), op->frag32.as<float>());
+        std::vector<CellMeta> ms(op->nCells);
+        for (u32 q = 0; q < op->nCells; ++q)
+          ms[q] = P.meta[op->hSlotPos[q]];
+        upload(metaSlots, ms, st);
       }
+    if (op->frag64.bytes != P.len64 * sizeof(double))
+      new64.alloc(P.len64 * sizeof(double));
+    if (op->hasF32 && op->frag32.bytes != P.len32 * sizeof(float))
+      new32.alloc(P.len32 * sizeof(float));
+
+    ++op->gen;
+    op->hMeta     = std::move(P.meta);
+    op->fragLen64 = P.len64;
+    op->fragLen32 = P.len32;
+    op->meta      = std::move(meta);
+    op->metaSlots = std::move(metaSlots);
+    if (op->frag64.bytes != P.len64 * sizeof(double))
+      op->frag64 = std::move(new64);
+    if (op->hasF32 && op->frag32.bytes != P.len32 * sizeof(float))
+      op->frag32 = std::move(new32);
+    const u32 nStored = (u32)P.stored.size();
+    k::repackCells<double>(st, op, nStored, stored.as<u32>(), order.as<u32>(), dmats,
+                           rawOff.as<u64>(), op->frag64.as<double>());
+    if (op->hasF32)
+      k::repackCells<float>(st, op, nStored, stored.as<u32>(), order.as<u32>(), dmats,
+                            rawOff.as<u64>(), op->frag32.as<float>());
     DFX_HIP(hipStreamSynchronize(st));
   }
 } // namespace dfx

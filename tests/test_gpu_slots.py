@@ -180,3 +180,44 @@ def test_cells_with_the_same_matrix_share_it(ctx, probs, dtype):
         got, ref = result(op), reference(mats)
         assert np.abs(got - ref).max() <= (n + 10) * eps * np.abs(mats).max() * n
         assert np.array_equal(got, result(make(mats)))
+
+
+def test_a_refused_update_leaves_the_operator_as_it_was(ctx, monkeypatch):
+    """An update from equal to distinct cell matrices needs a larger store; where
+    that allocation is refused the operator keeps its matrices (FP64, FP32 and
+    the colour-by-colour path), and the same update works afterwards."""
+    P = c1_like(n=3, p=2)
+    d = P.arrays()
+    ops = Ops(ctx, P)
+    n, nc = int(d["cellNdofs"][0]), len(d["cellNdofs"])
+    uniform = np.tile(d["K"][:n * n], nc)
+    distinct = (uniform.reshape(nc, -1) * (1.0 + np.arange(nc)[:, None] / 64.0)).ravel()
+
+    def make(mats):
+        return dfx.CellOperator(ctx, d["cellNdofs"], d["cellMap"], mats, P.nDofs, P.nClassical,
+                                ops.cons, keep_fp32=True)
+
+    def results(op):
+        out = []
+        for dtype, npd in ((dfx.F64, np.float64), (dfx.F32, np.float32)):
+            X = guess(P, 6, seed=8).astype(npd)
+            for call in (op.apply, op.apply_noalloc):
+                Y = dfx.MultiVector(ctx, P.nDofs, 6, dtype)
+                call(mv(ctx, X, dtype), Y)
+                out.append(Y.to_numpy())
+        return out
+
+    op, fresh = make(uniform), make(distinct)
+    before, info = results(op), op.info()
+    store = fresh.info()["matBytesF64"]
+    assert distinct.nbytes < store      # the matrices themselves may be uploaded
+    monkeypatch.setenv("DFX_MAX_ALLOC_BYTES", str(store - 1))
+    with pytest.raises(dfx.DfxError, match="DFX_MAX_ALLOC_BYTES"):
+        op.update_cells(distinct)
+    monkeypatch.delenv("DFX_MAX_ALLOC_BYTES")
+    assert op.info() == info
+    for a, b in zip(results(op), before):
+        assert np.array_equal(a, b)
+    op.update_cells(distinct)
+    for a, b in zip(results(op), results(fresh)):
+        assert np.array_equal(a, b)
