@@ -34,19 +34,6 @@ namespace dfx
     return reinterpret_cast<const T *>(op->frag32.p);
   }
 
-  // Y = C^T (sum_e Q_e^T A_e Q_e) C X, KohnShamOperatorContextFE::apply
-  // (src/ksdft/KohnShamOperatorContextFE.t.cpp:1326-1415)
-  // dsc / xe: see applyInvThenCellwise (classical rows gathered as dsc o X,
-  // enriched rows from xe; X already constrained)
-  // skipP2C: X is used as given (the caller has applied the parent->child
-  // step of other constraints, as LaplaceOperatorContextFE::apply does with
-  // its X manager's constraints, LaplaceOperatorContextFE.t.cpp:433-436)
-  // yEOverride: caller-provided scratch for the enriched partial rows (at
-  // least nEnrSlots x B values of T): nothing is allocated and no profiling
-  // record is taken
-  // rf (with dsc): the residual Chebyshev step fused in; Y then holds
-  // partial sums on the rows the cells finish, and res is complete on
-  // return (the listed remaining rows by a separate step)
   // Whether an apply of B columns takes the slot path (all cells of a size
   // class in one launch, their products to map slots, then the row sums)
   // rather than one launch per colour and class.  The slot path writes and
@@ -68,9 +55,49 @@ namespace dfx
     return op->slotsOk && bytes <= SLOT_BYTES && k::slotAddressable<T>(op, X);
   }
 
+  // op's scratch of at least `bytes`.  The generation changes before the old
+  // buffer goes: a captured graph that holds its address is not replayed even
+  // where the new one is refused
+  void growScratch(dfx_op *op, size_t bytes)
+  {
+    if (bytes <= op->yE.bytes)
+      return;
+    ++op->gen;
+    op->yE.alloc(bytes);
+  }
+
+  // The slots of an apply to X where it takes the slot path and they can be
+  // had, else null: the apply then goes colour by colour, which gives the same
+  // bits without them.  Nothing is allocated while the stream is being captured
   template <class T>
-  void applySlots(dfx_op *op, View<T> X, View<T> Y, const double *dsc, const T *xe, bool skipP2C,
-                  const k::ResFuse<T> *rf)
+  T *slotBuffer(dfx_op *op, View<const T> X)
+  {
+    if (!slotPath<T>(op, X))
+      return nullptr;
+    const size_t bytes = (size_t)op->sumNe * X.B * sizeof(T);
+    if (bytes > op->yE.bytes)
+      {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        DFX_HIP(hipStreamIsCapturing(op->ctx->stream, &cap));
+        if (cap != hipStreamCaptureStatusNone)
+          return nullptr;
+        try
+          {
+            growScratch(op, bytes);
+          }
+        catch (const Error &e)
+          {
+            if (e.code != DFX_E_OOM)
+              throw;
+            return nullptr;
+          }
+      }
+    return op->yE.as<T>();
+  }
+
+  template <class T>
+  void applySlots(dfx_op *op, View<T> X, View<T> Y, T *slots, const double *dsc, const T *xe,
+                  bool skipP2C, const k::ResFuse<T> *rf)
   {
     hipStream_t s = op->ctx->stream;
     // rows held at zero are masked in the gather and cleared in X and Y by
@@ -78,10 +105,7 @@ namespace dfx
     const bool mask = op->zeroRows && !skipP2C;
     if (!dsc && !skipP2C && !op->zeroRows)
       k::p2c<T>(s, op->cons, X);
-    if (op->yE.ensure((size_t)op->sumNe * X.B * sizeof(T)))
-      ++op->gen;
-    T            *slots = op->yE.as<T>();
-    const T      *frag  = fragOf<T>(op);
+    const T      *frag = fragOf<T>(op);
     View<const T> Xc{X.p, X.N, X.B, X.ld};
     const bool    prof = op->profiling && (op->profMask & (sizeof(T) == 8 ? 1 : 2)) &&
                       (op->profApplies++ % op->profEvery) == 0;
@@ -123,12 +147,11 @@ namespace dfx
   {
     View<const double> Xc{X.p, X.N, X.B, X.ld};
     if (op->kind != OP_CELLWISE || (op->cons && op->cons->nRows && !op->zeroRows) ||
-        op->profiling || X.N != op->nDofs || Y.N != op->nDofs || X.B != Y.B ||
-        !slotPath<double>(op, Xc))
+        op->profiling || X.N != op->nDofs || Y.N != op->nDofs || X.B != Y.B)
       return false;
-    if (op->yE.ensure((size_t)op->sumNe * X.B * sizeof(double)))
-      ++op->gen;
-    double *slots = op->yE.as<double>();
+    double *slots = slotBuffer<double>(op, Xc);
+    if (!slots)
+      return false;
     for (const Launch &l : op->slotLaunches64)
       k::cellSlots<double>(op->ctx->stream, op, l, fragOf<double>(op), Xc, slots, nullptr, nullptr,
                            op->zeroRows);
@@ -141,13 +164,27 @@ namespace dfx
     return true;
   }
 
+  // Y = C^T (sum_e Q_e^T A_e Q_e) C X, KohnShamOperatorContextFE::apply
+  // (src/ksdft/KohnShamOperatorContextFE.t.cpp:1326-1415)
+  // dsc / xe: see applyInvThenCellwise (classical rows gathered as dsc o X,
+  // enriched rows from xe; X already constrained)
+  // skipP2C: X is used as given (the caller has applied the parent->child
+  // step of other constraints, as LaplaceOperatorContextFE::apply does with
+  // its X manager's constraints, LaplaceOperatorContextFE.t.cpp:433-436)
+  // yEOverride: caller-provided scratch for the enriched partial rows (at
+  // least nEnrSlots x B values of T): nothing is allocated and no profiling
+  // record is taken
+  // rf (with dsc): the residual Chebyshev step fused in; Y then holds
+  // partial sums on the rows the cells finish, and res is complete on
+  // return (the listed remaining rows by a separate step)
   template <class T>
   void applyCellwise(dfx_op *op, View<T> X, View<T> Y, const double *dsc = nullptr,
                      const T *xe = nullptr, bool skipP2C = false, T *yEOverride = nullptr,
                      const k::ResFuse<T> *rf = nullptr)
   {
-    if (!yEOverride && slotPath<T>(op, View<const T>{X.p, X.N, X.B, X.ld}))
-      return applySlots<T>(op, X, Y, dsc, xe, skipP2C, rf);
+    if (!yEOverride)
+      if (T *slots = slotBuffer<T>(op, View<const T>{X.p, X.N, X.B, X.ld}))
+        return applySlots<T>(op, X, Y, slots, dsc, xe, skipP2C, rf);
     hipStream_t s = op->ctx->stream;
     if (!dsc && !skipP2C)
       k::p2c<T>(s, op->cons, X);
@@ -161,8 +198,7 @@ namespace dfx
       yE = yEOverride;
     else if (op->nEnrSlots)
       {
-        if (op->yE.ensure((size_t)op->nEnrSlots * X.B * sizeof(double)))
-          ++op->gen;
+        growScratch(op, (size_t)op->nEnrSlots * X.B * sizeof(double));
         yE = op->yE.as<T>();
       }
     const T *frag = fragOf<T>(op);
@@ -278,15 +314,14 @@ namespace dfx
     View<const T> X{xb.as<T>(), N, B, B};
     View<T>       Y{yb.as<T>(), N, B, B};
     const bool    buf   = k::cellBufferPath<T>(op, X, View<const T>{Y.p, N, B, B});
-    const bool    slots = slotPath<T>(op, X);
+    const bool    slots = slotBuffer<T>(op, X) != nullptr;
     const auto   &L     = slots ? (sizeof(T) == 8 ? op->slotLaunches64 : op->slotLaunches32)
                                 : (sizeof(T) == 8 ? op->launches64 : op->launches32);
     T *yE = nullptr;
     if (op->nEnrSlots || slots)
       {
-        if (op->yE.ensure(slots ? (size_t)op->sumNe * B * sizeof(T)
-                                : (size_t)op->nEnrSlots * B * sizeof(double)))
-          ++op->gen;
+        if (!slots)
+          growScratch(op, (size_t)op->nEnrSlots * B * sizeof(double));
         yE = op->yE.as<T>();
       }
     std::vector<u32> classes;
@@ -389,7 +424,7 @@ namespace dfx
     if ((sizeof(T) == 4 && !A->hasF32) || X.N != A->nDofs || Y.N != A->nDofs ||
         S1.N != A->nDofs || S1.ld != X.ld || X.B != Y.B || S1.B != X.B)
       return false;
-    const bool slots = slotPath<T>(A, View<const T>{X.p, X.N, X.B, X.ld});
+    const bool slots = slotBuffer<T>(A, View<const T>{X.p, X.N, X.B, X.ld}) != nullptr;
     if (!slots && (!k::cellBufferPath<T>(A, View<const T>{X.p, X.N, X.B, X.ld},
                                          View<const T>{Y.p, Y.N, Y.B, Y.ld}) ||
                    (reinterpret_cast<uintptr_t>(S1.p) & 15) != 0))

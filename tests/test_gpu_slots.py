@@ -221,3 +221,93 @@ def test_a_refused_update_leaves_the_operator_as_it_was(ctx, monkeypatch):
     op.update_cells(distinct)
     for a, b in zip(results(op), results(fresh)):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("name", ["c1", "hang3", "wide"])
+@pytest.mark.parametrize("dtype", [dfx.F64, dfx.F32])
+def test_applies_run_where_the_slots_cannot_be_had(ctx, probs, name, dtype, monkeypatch):
+    """Operators whose slots are refused as out of memory apply colour by colour:
+    plain, with M^-1 folded in, and tuned; the bits of the slot path."""
+    P = probs[name]
+    npd = np.float64 if dtype == dfx.F64 else np.float32
+    size = np.dtype(npd).itemsize
+    rows = int(P.arrays()["cellNdofs"].sum())
+    for B in (8, 13, 40):
+        X = O.rng_uniform(B, -1, 1, P.nDofs * B).reshape(P.nDofs, B).astype(npd)
+        outs = []
+        for limit in (None, rows * B * size - 1):
+            ops = Ops(ctx, P)
+            Xa, Xb = mv(ctx, X, dtype), mv(ctx, X, dtype)
+            Ya, Yb, Yc = (dfx.MultiVector(ctx, P.nDofs, B, dtype) for _ in range(3))
+            if limit:
+                assert limit > P.nDofs * B * size        # vectors and work space are not
+                monkeypatch.setenv("DFX_MAX_ALLOC_BYTES", str(limit))
+            ops.H.apply(Xa, Ya)
+            ops.H.apply_after_inverse(ops.Minv, Xb, Yb)
+            ops.H.autotune(dtype, B, reps=1)
+            ops.H.apply(Xa, Yc)
+            monkeypatch.delenv("DFX_MAX_ALLOC_BYTES", raising=False)
+            outs.append([v.to_numpy() for v in (Xa, Xb, Ya, Yb, Yc)])
+        for a, b in zip(*outs):
+            assert np.array_equal(a, b), (name, B)
+
+
+@pytest.mark.parametrize("B", [8, 40, 72])
+@pytest.mark.parametrize("prec", [dfx.PREC_FP64, dfx.PREC_MIXED])
+def test_filter_runs_where_the_slots_cannot_be_had(ctx, probs, B, prec, monkeypatch):
+    """The filter with the residual step in the colour kernel's scatter, eager
+    and replayed, against the slot path: the same bits."""
+    P = probs["wide"]
+    lo, hi, beta = P.lanczos(O.rng_uniform(2, -1, 1, P.nDofs))
+    a, c = lo, hi + beta / 10
+    b = a + 0.05 * (c - a)
+    X = guess(P, B, seed=B)
+    size = 8 if prec == dfx.PREC_FP64 else 4
+    limit = int(P.arrays()["cellNdofs"].sum()) * B * size - 1
+    outs = []
+    for graph in (False, True):
+        G, V = mv(ctx, X), dfx.MultiVector(ctx, P.nDofs, B)
+        s = dfx.ChebyshevFilteredEigenSolver(ctx, a, b, c, 7, 1e-14, G, True, 0, prec, graph)
+        # with slots (this allocates the solver's work space), then fresh
+        # operators that get none; the second of their passes replays the loop
+        for ops, passes in ((Ops(ctx, P), 1), (Ops(ctx, P), 2)):
+            for _ in range(passes):
+                G.upload(X)
+                eig = np.linspace(a, b, B)
+                s.reinit(a, b, c, 7, 1e-14, G)
+                assert s.solve(ops.H, eig, V, True, ops.M, ops.Minv) == 0
+                outs.append((eig, V.to_numpy()))
+                monkeypatch.setenv("DFX_MAX_ALLOC_BYTES", str(limit))
+        monkeypatch.delenv("DFX_MAX_ALLOC_BYTES")
+    for o in outs[1:]:
+        assert np.array_equal(o[0], outs[0][0]) and np.array_equal(o[1], outs[0][1])
+
+
+def test_a_first_apply_is_captured_without_slots(ctx, probs):
+    """A classical operator's apply allocates nothing while its stream is being
+    captured, also the first one: it goes colour by colour there.  Replays give
+    the eager bits, with eager work between them."""
+    P = probs["c1"]
+    B = 8
+    warm, ops = Ops(ctx, P), Ops(ctx, P)
+    X, Y = dfx.MultiVector(ctx, P.nDofs, B), dfx.MultiVector(ctx, P.nDofs, B)
+    warm.H.apply_noalloc(X, Y)                       # the kernels are loaded
+    ctx.synchronize()
+    hip, stream, graph, run = dfx._lib, C.c_void_p(), C.c_void_p(), C.c_void_p()
+    assert hip.dfx_ctx_stream(ctx.h, C.byref(stream)) == 0
+    assert hip.hipStreamBeginCapture(stream, 0) == 0          # the strictest mode
+    try:
+        ops.H.apply(X, Y)
+    finally:
+        assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)) == 0
+    for seed in range(4):
+        X.upload(guess(P, B, seed=seed))
+        Y.set(0.0)
+        assert hip.hipGraphLaunch(run, stream) == 0
+        ctx.synchronize()
+        got = Y.to_numpy()
+        want = dfx.MultiVector(ctx, P.nDofs, B)
+        ops.H.apply(mv(ctx, guess(P, B, seed=seed)), want)     # eager: in slots
+        assert np.array_equal(got, want.to_numpy())
+    assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
