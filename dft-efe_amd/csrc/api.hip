@@ -300,8 +300,9 @@ namespace dfx
   // multivectors and keep the fastest.  Candidates: 1, 2, 4, 8 tiles of 16
   // columns up to twice the columns there are, 5 for FP32 with 65..80
   // columns, 3 for slot launches of 33..48, and only tiles that fit the LDS of
-  // a CU; the launches timed are those of the path such an apply takes.  Per-column results do
-  // not depend on the width (same K order per column), only the time does.
+  // a CU; the launches timed are those of the path such an apply takes, and
+  // the widths hold for that path.  Per-column results do not depend on the
+  // width (same K order per column), only the time does.
   template <class T>
   std::vector<std::pair<u32, int>> autotune(dfx_op *op, u32 B, u32 reps)
   {
@@ -330,9 +331,12 @@ namespace dfx
         classes.push_back(l.mtw);
     op->tuned.erase(std::remove_if(op->tuned.begin(), op->tuned.end(),
                                    [&](const dfx_op::Tuned &t) {
-                                     return t.s == sizeof(T) && t.B == B;
+                                     return t.s == sizeof(T) && t.B == B && t.slots == slots;
                                    }),
                     op->tuned.end());
+    // DFX_CELL_TUNE_NT: the only width tried (read on every call)
+    const char *onlyEnv = getenv("DFX_CELL_TUNE_NT");
+    const int   only    = onlyEnv ? atoi(onlyEnv) : 0;
     hipEvent_t a, b;
     DFX_HIP(hipEventCreate(&a));
     DFX_HIP(hipEventCreate(&b));
@@ -350,6 +354,8 @@ namespace dfx
             float     bestMs = 0.f;
             for (int nt : {1, 2, 3, 4, 5, 8})
               {
+                if (only && nt != only)
+                  continue;
                 if (nt == 5 && !(sizeof(T) == 4 && B > 64 && B <= 80))
                   continue;
                 // three tiles: slot launches of 33..48 columns; eight: colour launches
@@ -379,7 +385,7 @@ namespace dfx
               }
             if (!best)
               best = slots ? k::slotNT<T>(B, kpad) : k::builtinNT<T>(B, kpad);
-            op->tuned.push_back(dfx_op::Tuned{(u32)sizeof(T), B, c, best});
+            op->tuned.push_back(dfx_op::Tuned{(u32)sizeof(T), B, c, slots, best});
             out.emplace_back(c, best);
           }
       }

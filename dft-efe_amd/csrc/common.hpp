@@ -356,17 +356,19 @@ struct dfx_op
   dfx::DevBuf diag, diag32, enrBlock, enrFrag64, enrFrag32;
   dfx::u32 nEnriched = 0;
   // ----- column-chunk widths picked by dfx_op_autotune: for scalar size s
-  // and exactly B columns, launches of M-tile class mtw use 16 nt columns
+  // and exactly B columns, launches of M-tile class mtw on the slot or the
+  // colour path (whose kernels come in different widths) use 16 nt columns
   struct Tuned
   {
     dfx::u32 s, B, mtw;
+    bool     slots;
     int      nt;
   };
   std::vector<Tuned> tuned;
-  int tunedNT(dfx::u32 s, dfx::u32 B, dfx::u32 mtw) const
+  int tunedNT(dfx::u32 s, dfx::u32 B, dfx::u32 mtw, bool slots) const
   {
     for (const Tuned &t : tuned)
-      if (t.s == s && t.B == B && t.mtw == mtw)
+      if (t.s == s && t.B == B && t.mtw == mtw && t.slots == slots)
         return t.nt;
     return 0;
   }

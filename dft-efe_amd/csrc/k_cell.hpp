@@ -1212,7 +1212,7 @@ namespace dfx
       // explicit width, else the autotuner's for (scalar size, B, class) unless
       // the environment caps the width, else the built-in choice
       if (!nt && !ntOverride(sizeof(T) == 8))
-        nt = op->tunedNT(sizeof(T), x.B, L.mtw);
+        nt = op->tunedNT(sizeof(T), x.B, L.mtw, false);
       if (!nt)
         nt = chooseNT<T>(x.B, L.kpadMax);
       switch (nt)
@@ -1258,7 +1258,7 @@ namespace dfx
       if (L.end <= L.begin || !x.B)
         return;
       if (!nt && !ntOverride(sizeof(T) == 8))
-        nt = op->tunedNT(sizeof(T), x.B, L.mtw);
+        nt = op->tunedNT(sizeof(T), x.B, L.mtw, true);
       if (!nt)
         nt = slotNT<T>(x.B, L.kpadMax);
       switch (nt)

@@ -248,10 +248,11 @@ int dfx_op_get_profile(dfx_op *op, dfx_op_profile *out, int reset);
 /* Column-chunk autotuner.  No counterpart in the reference, whose cell-block
  * sizes are fixed defaults (KohnShamOperatorContextFE.t.cpp:1370-1371).
  * Times the candidate column-chunk widths of the fused cell-apply kernel
- * (16 NT columns per chunk, NT in {1, 2, 4, 5, 8}) for every size class of a
+ * (16 NT columns per chunk, NT in {1, 2, 3, 4, 5, 8}) for every size class of a
  * cell-wise operator, for dtype and exactly B columns, on scratch device
  * multivectors (reps passes per candidate), and keeps the fastest width per
- * class for later applies of that dtype with B columns.  Results of an apply
+ * class for later applies of that dtype with B columns that take the same
+ * path (through map slots or colour by colour).  Results of an apply
  * do not depend on the width (columns are independent, same K order).
  * classes / widths (room for maxOut entries; may be NULL when maxOut is 0):
  * the class (M tiles per wave) and the chosen NT, in launch order; *nOut

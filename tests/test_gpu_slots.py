@@ -311,3 +311,27 @@ def test_a_first_apply_is_captured_without_slots(ctx, probs):
         ops.H.apply(mv(ctx, guess(P, B, seed=seed)), want)     # eager: in slots
         assert np.array_equal(got, want.to_numpy())
     assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
+
+
+@pytest.mark.parametrize("dtype", [dfx.F64, dfx.F32])
+@pytest.mark.parametrize("B", [33, 40, 48])
+def test_widths_tuned_on_one_path_stay_there(ctx, probs, B, dtype, monkeypatch):
+    """Three tiles of 16 columns is a width of the slot kernels only: tuned to it,
+    an operator still applies colour by colour (without allocation, or where the
+    slots are refused), with the bits of the untuned operator."""
+    P = probs["wide"]
+    npd = np.float64 if dtype == dfx.F64 else np.float32
+    X = O.rng_uniform(B, -1, 1, P.nDofs * B).reshape(P.nDofs, B).astype(npd)
+    ops = Ops(ctx, P)
+
+    def run(call):
+        Y = dfx.MultiVector(ctx, P.nDofs, B, dtype)
+        call(mv(ctx, X, dtype), Y)
+        return Y.to_numpy()
+
+    before = run(ops.H.apply)
+    monkeypatch.setenv("DFX_CELL_TUNE_NT", "3")
+    assert set(ops.H.autotune(dtype, B, reps=1).values()) == {3}
+    monkeypatch.delenv("DFX_CELL_TUNE_NT")
+    assert np.array_equal(run(ops.H.apply), before)
+    assert np.array_equal(run(ops.H.apply_noalloc), before)
