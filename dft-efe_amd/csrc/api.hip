@@ -52,7 +52,8 @@ namespace dfx
   bool slotPath(const dfx_op *op, View<const T> X)
   {
     const u64 bytes = op->sumNe * X.B * sizeof(T);
-    return op->slotsOk && bytes <= SLOT_BYTES && k::slotAddressable<T>(op, X);
+    return op->slotsOk && op->ctx->useSlots && bytes <= SLOT_BYTES &&
+           k::slotAddressable<T>(op, X);
   }
 
   // op's scratch of at least `bytes`.  The generation changes before the old

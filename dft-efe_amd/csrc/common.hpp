@@ -189,6 +189,7 @@ struct dfx_ctx
   hipStream_t    stream2 = nullptr;
   hipEvent_t     forkEv = nullptr, joinEv = nullptr;
   bool           forkClasses = true; // false: every launch on `stream` (serving slots)
+  bool           useSlots = true;    // false: every apply colour by colour
   rocblas_handle blas   = nullptr;
   // hipBLASLt state of the FP64 subspace rotations (handle, workspace, one
   // plan per shape), owned here and released by ltFree

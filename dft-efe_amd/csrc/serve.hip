@@ -77,8 +77,10 @@ namespace dfx
 
     // device bytes a request holds at its peak: raw H, M, K (FP64), the three
     // operators' FP64 + FP32 fragment copies, setup tabulation batches (at
-    // most 6 GB), and about 16 N x states FP64 vectors of solver work space
-    u64 footprint(const dfx_request &r)
+    // most 6 GB), about 16 N x states FP64 vectors of solver work space and
+    // the slots of H's and M's applies, without which they go colour by colour
+    // (withSlots false)
+    u64 footprint(const dfx_request &r, bool withSlots)
     {
       u64 sumN, sumN2, nCells;
       u32 maxN;
@@ -101,8 +103,7 @@ namespace dfx
       // N x n FP64 arrays: subspaces, filter and CholGS / RR work, and the
       // H X, M X the solver keeps of its eigenvectors
       const u64 vecs  = 18 * N * (u64)r.numStates * 8;
-      // the slots of H's and M's applies
-      const u64 slots = 2 * std::min<u64>(SLOT_BYTES, sumN * r.numStates * 8);
+      const u64 slots = withSlots ? 2 * std::min<u64>(SLOT_BYTES, sumN * r.numStates * 8) : 0;
       return (mats + setup + vecs + slots) * 5 / 4 + (64ull << 20);
     }
 
@@ -230,7 +231,7 @@ extern "C"
       return DFX_E_ARG;
     try
       {
-        *bytes = footprint(*r);
+        *bytes = footprint(*r, true);
         return 0;
       }
     catch (...)
@@ -249,11 +250,18 @@ extern "C"
     std::stable_sort(order.begin(), order.end(), [&](u32 a, u32 b) {
       return reqs[a].arrivalSeconds < reqs[b].arrivalSeconds;
     });
-    std::vector<u64> energyOff(nRequests + 1, 0), fp(nRequests);
+    std::vector<u64>  energyOff(nRequests + 1, 0), fp(nRequests);
+    std::vector<char> slots(nRequests, 1);
     for (u32 i = 0; i < nRequests; ++i)
       {
         energyOff[i + 1] = energyOff[i] + reqs[i].numStates;
-        fp[i]            = footprint(reqs[i]);
+        fp[i]            = footprint(reqs[i], true);
+        // a request that fits the whole budget only without slots runs so
+        if (fp[i] > p->memoryBudgetBytes)
+          {
+            slots[i] = 0;
+            fp[i]    = footprint(reqs[i], false);
+          }
         if (fp[i] > p->memoryBudgetBytes)
           return DFX_E_OOM; // could never be admitted
       }
@@ -311,6 +319,7 @@ extern "C"
           else
             try
               {
+                ctx->useSlots = slots[idx] != 0;
                 out.status = runRequest(ctx, p->precision, p->useGraph != 0, reqs[idx],
                                         energies + energyOff[idx], out);
               }

@@ -613,7 +613,9 @@ int dfx_poisson_destroy(dfx_poisson *p);
  * arrival order when they have arrived, a slot is free and their estimated
  * device footprint fits in memoryBudgetBytes; each admitted request runs on
  * its own context / HIP stream, so the work of all admitted requests
- * overlaps on the device.  Results do not depend on the mix.
+ * overlaps on the device.  A request that the whole budget holds only without
+ * the scratch of the applies' map slots runs colour by colour; one that does
+ * not fit even so is refused (DFX_E_OOM).  Results do not depend on the mix.
  * ==================================================================== */
 typedef struct dfx_request
 {

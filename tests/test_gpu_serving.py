@@ -51,6 +51,22 @@ def test_admission_respects_the_memory_budget():
     assert all(spans[i + 1][0] >= spans[i][1] - 1e-6 for i in range(len(spans) - 1))
 
 
+def test_a_request_that_fits_only_without_slots_is_served():
+    """The footprint counts the scratch that applies send their products through.
+    A request that the whole budget holds only without it is served all the same,
+    colour by colour, with the same eigenvalues; one that does not fit even so is
+    refused."""
+    req = dict(small_stream(n=1, seed=14)[0], arrival=0.0)
+    full = dfx.request_footprint(req)
+    (want,), (free,) = dfx.serve([req], max_slots=1, memory_budget=full)
+    assert free["status"] == 0 and free["footprintBytes"] == full
+    (got,), (tight,) = dfx.serve([req], max_slots=1, memory_budget=full - 1)
+    assert tight["status"] == 0 and tight["footprintBytes"] < full
+    assert tight["passes"] == free["passes"] and np.array_equal(got, want)
+    with pytest.raises(dfx.DfxError):
+        dfx.serve([req], max_slots=1, memory_budget=tight["footprintBytes"] - 1)
+
+
 def test_graph_replay_gives_the_eager_results():
     """Requests replay their captured degree loop on every pass (the filter
     bounds change from pass to pass and are read from the device): the
