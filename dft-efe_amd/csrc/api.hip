@@ -141,30 +141,6 @@ namespace dfx
       k::c2p<T>(s, op->cons, Y);
   }
 
-  // Y = op X and the column dots X.Y (device) in one go where op is cell-wise
-  // on the slot path with no constraints but rows held at zero; false
-  // (nothing done) otherwise.  partials: DOT_PARTIALS X.B doubles
-  bool applyDot(dfx_op *op, View<double> X, View<double> Y, double *partials, double *out)
-  {
-    View<const double> Xc{X.p, X.N, X.B, X.ld};
-    if (op->kind != OP_CELLWISE || (op->cons && op->cons->nRows && !op->zeroRows) ||
-        op->profiling || X.N != op->nDofs || Y.N != op->nDofs || X.B != Y.B)
-      return false;
-    double *slots = slotBuffer<double>(op, Xc);
-    if (!slots)
-      return false;
-    for (const Launch &l : op->slotLaunches64)
-      k::cellSlots<double>(op->ctx->stream, op, l, fragOf<double>(op), Xc, slots, nullptr, nullptr,
-                           op->zeroRows);
-    if (!k::slotSumDot(op->ctx->stream, op, slots, X, Y, partials, out))
-      {
-        k::slotSum<double>(op->ctx->stream, op, slots, X, Y, op->zeroRows, nullptr);
-        k::colDots<double>(op->ctx->stream, Xc, View<const double>{Y.p, Y.N, Y.B, Y.ld}, partials,
-                           out);
-      }
-    return true;
-  }
-
   // Y = C^T (sum_e Q_e^T A_e Q_e) C X, KohnShamOperatorContextFE::apply
   // (src/ksdft/KohnShamOperatorContextFE.t.cpp:1326-1415)
   // dsc / xe: see applyInvThenCellwise (classical rows gathered as dsc o X,
@@ -470,6 +446,37 @@ namespace dfx
       applyCellwise<T>(op, X, Y);
     else
       applyDiagonal<T>(op, X, Y);
+  }
+
+  // Y = op X and the column dots X.Y (device; partials: DOT_PARTIALS X.B
+  // doubles).  In one pass over the slots where op is cell-wise on the slot
+  // path with no constraints but rows held at zero, else by an apply and the
+  // dots apart: the same bits, whatever the columns, the profiling and the path
+  void applyDot(dfx_op *op, View<double> X, View<double> Y, double *partials, double *out)
+  {
+    hipStream_t s  = op->ctx->stream;
+    const u32   nE = op->nDofs - op->nClassical;
+    View<const double> Xc{X.p, X.N, X.B, X.ld}, Yc{Y.p, Y.N, Y.B, Y.ld};
+    const bool         apart = op->kind == OP_CELLWISE && nE <= k::DOT_PARTIALS / 2;
+    if (apart && !(op->cons && op->cons->nRows && !op->zeroRows) && !op->profiling &&
+        X.N == op->nDofs && Y.N == op->nDofs && X.B == Y.B)
+      if (double *slots = slotBuffer<double>(op, Xc))
+        {
+          for (const Launch &l : op->slotLaunches64)
+            k::cellSlots<double>(s, op, l, fragOf<double>(op), Xc, slots, nullptr, nullptr,
+                                 op->zeroRows);
+          if (!k::slotSumDot(s, op, slots, X, Y, partials, out))
+            {
+              k::slotSum<double>(s, op, slots, X, Y, op->zeroRows, nullptr);
+              k::colDotsApart(s, Xc, Yc, op->nClassical, partials, out);
+            }
+          return;
+        }
+    applyOp<double>(op, X, Y);
+    if (apart)
+      k::colDotsApart(s, Xc, Yc, op->nClassical, partials, out);
+    else
+      k::colDots<double>(s, Xc, Yc, partials, out);
   }
 
   void ctxRelease(dfx_ctx *ctx)

@@ -74,7 +74,7 @@ namespace dfx
   View<T> view(dfx_mv *m);
   template <class T>
   void applyOp(dfx_op *op, View<T> X, View<T> Y);
-  bool applyDot(dfx_op *op, View<double> X, View<double> Y, double *partials, double *out);
+  void applyDot(dfx_op *op, View<double> X, View<double> Y, double *partials, double *out);
   template <class T>
   bool applyInvThenCellwise(dfx_op *Dinv, dfx_op *A, View<T> X, View<T> S1, View<T> Y,
                             const k::ResFuse<T> *rf = nullptr);

@@ -1,6 +1,7 @@
 // The row sums of the slot apply: every cell's product lies in its map slots'
 // rows (cellSlots), and each dof's row is the sum of its slots' rows in a
 // fixed order, with the step that follows the apply formed in the same launch.
+#include "dots.hpp"
 #include "enr_reduce.hpp"
 #include "kernels.hpp"
 #include "res_update.hpp"
@@ -151,19 +152,22 @@ namespace dfx
           *reinterpret_cast<vt *>(y + (u64)row * ldy + j) = s;
       }
       // The row sums with the column dots x.y of the same rows (PCG's p.w, FP64,
-      // V = 2 columns a thread, B even): a workgroup takes RB = 256 / (B / 2)
-      // rows at a time, every nBlocks-th such group; its sums per column go to
-      // partials[block] (fixed tree over the rows), an enriched dof's product
-      // to partials[nBlocks + dof].  Saves the separate dot a read of x and y
-      // and a launch (16^3 cells, p = 3, 8 columns: 7.9 + 6.3 us for the two)
+      // two columns a thread, B even), in the order of dots.hpp: a workgroup is
+      // a block of rows, R = 64 / U row threads of U lanes each (R the largest
+      // power of two that B / 2 column pairs leave room for); an enriched dof's
+      // product goes to partials[nBlocks + dof].  Saves the separate dot a read
+      // of x and y and a launch (16^3 cells, p = 3, 8 columns: 7.9 + 6.3 us for
+      // the two)
+      template <int U>
       __global__ __launch_bounds__(256) void slotSumDotK(
         const RowHead *__restrict__ heads, const u32 *__restrict__ rest,
         const u32 *__restrict__ enrOff, const u32 *__restrict__ enrSlots, u32 nC, u32 nE,
         const double *__restrict__ slots, u32 B, double *x, double *y, u32 nBlocks,
-        double *__restrict__ partials)
+        u32 rowsPerBlock, double *__restrict__ partials)
       {
-        using T  = double;
-        using vt = Vec<double, 2>::type;
+        using T         = double;
+        using vt        = Vec<double, 2>::type;
+        constexpr u32 R = DOT_LANES / U;
         __shared__ EnrReduce<T> red;
         __shared__ vt           sum[256];
         const u32 nb = (B + EnrReduce<T>::CB - 1) / EnrReduce<T>::CB;
@@ -180,31 +184,36 @@ namespace dfx
               }
             return;
           }
-        const u32 blk = blockIdx.x - nE * nb, nv = B / 2, RB = 256 / nv;
+        const u32 blk = blockIdx.x - nE * nb, nv = B / 2;
         const u32 r = threadIdx.x / nv, j = (threadIdx.x - r * nv) * 2;
-        vt        acc{};
-        if (r < RB)
-          for (u32 row = blk * RB + r; row < nC; row += nBlocks * RB)
-            {
-              const RowHead h = heads[row];
-              const u64     o = (u64)row * B + j;
-              if (h.rest >> ROW_COUNT_SHIFT == ROW_ZERO)
+        const u32 r0 = blk * rowsPerBlock, r1 = min(nC, r0 + rowsPerBlock);
+        vt        acc[U]{};
+        if (r < R)
+          for (u32 i0 = r0 + r; i0 < r1; i0 += DOT_LANES)
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+              if (const u32 row = i0 + u * R; row < r1)
                 {
-                  *reinterpret_cast<vt *>(y + o) = vt{};
-                  *reinterpret_cast<vt *>(x + o) = vt{};
-                  continue;
+                  const RowHead h = heads[row];
+                  const u64     o = (u64)row * B + j;
+                  if (h.rest >> ROW_COUNT_SHIFT == ROW_ZERO)
+                    {
+                      *reinterpret_cast<vt *>(y + o) = vt{};
+                      *reinterpret_cast<vt *>(x + o) = vt{};
+                      continue;
+                    }
+                  const vt xv = *reinterpret_cast<const vt *>(x + o);
+                  const vt s  = rowSum<T, 2>(h, rest, slots, B, j);
+                  *reinterpret_cast<vt *>(y + o) = s;
+                  acc[u][0] = fma(xv[0], s[0], acc[u][0]);
+                  acc[u][1] = fma(xv[1], s[1], acc[u][1]);
                 }
-              const vt xv = *reinterpret_cast<const vt *>(x + o);
-              const vt s  = rowSum<T, 2>(h, rest, slots, B, j);
-              *reinterpret_cast<vt *>(y + o) = s;
-              acc[0] = fma(xv[0], s[0], acc[0]);
-              acc[1] = fma(xv[1], s[1], acc[1]);
-            }
-        sum[threadIdx.x] = acc;
+        sum[threadIdx.x] = foldLanes(acc);
         __syncthreads();
-        for (u32 h = 128; h > 0; h >>= 1)
+#pragma unroll
+        for (u32 h = R / 2; h > 0; h >>= 1)
           {
-            if (h < RB && r < h && r + h < RB)
+            if (r < h)
               sum[threadIdx.x] += sum[threadIdx.x + h * nv];
             __syncthreads();
           }
@@ -221,12 +230,24 @@ namespace dfx
       if (B < 2 || B % 2 || B > 128 || x.ld != B || y.ld != B || !aligned(slots) ||
           !aligned(x.p) || !aligned(y.p) || !nC || nE > DOT_PARTIALS / 2)
         return false;
-      const u32 RB      = 256 / (B / 2);
-      const u32 nBlocks = (u32)std::min<u64>(DOT_PARTIALS / 2, ((u64)nC + RB - 1) / RB);
+      const u32 nBlocks = dotBlocks(nC), rows = dotRows(nC, nBlocks);
       const u32 nb      = (B + EnrReduce<double>::CB - 1) / EnrReduce<double>::CB;
-      slotSumDotK<<<nE * nb + nBlocks, 256, 0, s>>>(
-        op->rowHeads.as<RowHead>(), op->slotRest.as<u32>(), op->enrSlotOffsets.as<u32>(),
-        op->enrMapSlots.as<u32>(), nC, nE, slots, B, x.p, y.p, nBlocks, partials);
+      auto go = [&](auto kern) {
+        kern<<<nE * nb + nBlocks, 256, 0, s>>>(
+          op->rowHeads.as<RowHead>(), op->slotRest.as<u32>(), op->enrSlotOffsets.as<u32>(),
+          op->enrMapSlots.as<u32>(), nC, nE, slots, B, x.p, y.p, nBlocks, rows, partials);
+      };
+      // row threads: 256 / (B / 2), rounded down to a power of two, at most 64
+      if (B <= 8)
+        go(slotSumDotK<1>);
+      else if (B <= 16)
+        go(slotSumDotK<2>);
+      else if (B <= 32)
+        go(slotSumDotK<4>);
+      else if (B <= 64)
+        go(slotSumDotK<8>);
+      else
+        go(slotSumDotK<16>);
       checkLaunch("slotSumDot");
       colDotsFinal(s, partials, nBlocks + nE, B, out);
       return true;

@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "dots.hpp"
 #include "kernels.hpp"
 #include "res_update.hpp"
 
@@ -216,33 +217,79 @@ namespace dfx
       }
 
       // pass 1 of the column dots: block b owns rows [b*rows, (b+1)*rows);
-      // threads are C columns x R row-lanes
-      template <class T, int C>
-      __global__ void colDotsK(const T *x, u32 ldx, const T *y, u32 ldy, u32 N,
-                               u32 B, u32 rowsPerBlock, double *partials)
+      // threads are C columns x R row threads of U lanes each (dots.hpp)
+      template <int C>
+      struct DotShape
       {
-        constexpr int R  = TPB / C;
+        static constexpr int R = TPB / C, U = DOT_LANES / R;
+        // rows a thread takes per turn of its loop, in groups of four whose
+        // loads are in flight together; the t-th belongs to lane t % U
+        static constexpr int STEP = U > 4 ? U : 4;
+        static_assert(R <= DOT_LANES && STEP % U == 0, "whole lanes");
+      };
+      // a column's sum over the block, in the threads with ty == 0
+      template <int C>
+      __device__ inline double blockSum(double (&acc)[DotShape<C>::U], double *red)
+      {
+        constexpr int R  = DotShape<C>::R;
+        red[threadIdx.x] = foldLanes(acc);
+        __syncthreads();
+        if (threadIdx.x >= C)
+          return 0.0;
+        double v[R];
+#pragma unroll
+        for (int q = 0; q < R; ++q)
+          v[q] = red[q * C + threadIdx.x];
+        return foldLanes(v);
+      }
+
+      template <class T, int C>
+      __global__ __launch_bounds__(TPB) void colDotsK(const T *x, u32 ldx, const T *y, u32 ldy,
+                                                      u32 N, u32 B, u32 rowsPerBlock,
+                                                      double *partials)
+      {
+        using S          = DotShape<C>;
+        constexpr int R  = S::R, U = S::U;
         const int     tx = threadIdx.x % C, ty = threadIdx.x / C;
         __shared__ double red[TPB];
         const u32 r0 = blockIdx.x * rowsPerBlock;
         const u32 r1 = min(N, r0 + rowsPerBlock);
         for (u32 j0 = 0; j0 < B; j0 += C)
           {
-            const u32 j   = j0 + tx;
-            double    acc = 0.0;
+            const u32 j = j0 + tx;
+            double    acc[U]{};
             if (j < B)
-              for (u32 i = r0 + ty; i < r1; i += R)
-                acc = fma((double)x[(u64)i * ldx + j], (double)y[(u64)i * ldy + j], acc);
-            red[threadIdx.x] = acc;
-            __syncthreads();
+              for (u32 i0 = r0 + ty; i0 < r1; i0 += S::STEP * R)
+#pragma unroll
+                for (int g = 0; g < S::STEP; g += 4)
+                  {
+                    T xv[4], yv[4];
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+                      if (const u32 i = i0 + (g + t) * R; i < r1)
+                        xv[t] = x[(u64)i * ldx + j], yv[t] = y[(u64)i * ldy + j];
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+                      if (i0 + (g + t) * R < r1)
+                        acc[(g + t) % U] = fma((double)xv[t], (double)yv[t], acc[(g + t) % U]);
+                  }
+            const double s = blockSum<C>(acc, red);
             if (ty == 0 && j < B)
-              {
-                double s = 0.0;
-                for (int q = 0; q < R; ++q)
-                  s += red[q * C + tx];
-                partials[(u64)blockIdx.x * B + j] = s;
-              }
+              partials[(u64)blockIdx.x * B + j] = s;
             __syncthreads();
+          }
+      }
+
+      // partials[i, j] = x_ij y_ij: rows whose dot is a partial sum of its own
+      __global__ void rowProductsK(const double *x, u32 ldx, const double *y, u32 ldy, u32 N,
+                                   u32 B, double *partials)
+      {
+        const u64 n = (u64)N * B;
+        for (u64 t = blockIdx.x * (u64)blockDim.x + threadIdx.x; t < n;
+             t += (u64)gridDim.x * blockDim.x)
+          {
+            const RC r  = rc(t, B);
+            partials[t] = x[(u64)r.i * ldx + r.j] * y[(u64)r.i * ldy + r.j];
           }
       }
 
@@ -251,66 +298,62 @@ namespace dfx
       // with z = d o r (alpha = zr / pw per column, formed here as cgAlphaK
       // does; z itself is formed again where it is used).
       // Rows, lanes and sums follow colDotsK exactly (same blocks of rows,
-      // same lane order, same combine), and each element is the blocked
+      // same lane order, same folds), and each element is the blocked
       // axpby's / the diagonal scaling's expression, so every value is the
       // separate launches' bit for bit.  partials: nBlocks x 2B (z.r in
       // columns [0, B), r.r in [B, 2B)); N x B arrays with leading dimension B.
       // Bound by memory: 4 reads and 2 writes per value (with z, a copy of x and
       // 16 lanes for 8 columns it took 15.5 us at 117 649 x 8)
       template <int C>
-      __global__ void cgUpdateK(const double *x, double *xn, double *r, const double *p,
-                                const double *w, const double *d, const double *zr,
-                                const double *pw, u32 N, u32 B, u32 rowsPerBlock,
-                                double *partials)
+      __global__ __launch_bounds__(TPB) void cgUpdateK(const double *x, double *xn, double *r,
+                                                       const double *p, const double *w,
+                                                       const double *d, const double *zr,
+                                                       const double *pw, u32 N, u32 B,
+                                                       u32 rowsPerBlock, double *partials)
       {
-        constexpr int R  = TPB / C;
+        using S          = DotShape<C>;
+        constexpr int R  = S::R, U = S::U;
         const int     tx = threadIdx.x % C, ty = threadIdx.x / C;
         __shared__ double red[2][TPB];
         const u32 r0 = blockIdx.x * rowsPerBlock;
         const u32 r1 = min(N, r0 + rowsPerBlock);
         for (u32 j0 = 0; j0 < B; j0 += C)
           {
-            const u32 j     = j0 + tx;
-            double    accZ  = 0.0, accR = 0.0;
+            const u32 j = j0 + tx;
+            double    accZ[U]{}, accR[U]{};
             if (j < B)
               {
                 const double alpha = zr[j] / pw[j], nalpha = -zr[j] / pw[j];
-                // four rows of a lane in flight together, added in order
-                for (u32 i0 = r0 + ty; i0 < r1; i0 += 4 * R)
-                  {
-                    double xv[4], pv[4], rv[4], wv[4], dv[4];
+                for (u32 i0 = r0 + ty; i0 < r1; i0 += S::STEP * R)
 #pragma unroll
-                    for (int u = 0; u < 4; ++u)
-                      if (const u32 i = i0 + u * R; i < r1)
-                        {
-                          const u64 o = (u64)i * B + j;
-                          xv[u] = x[o], pv[u] = p[o], rv[u] = r[o], wv[u] = w[o], dv[u] = d[i];
-                        }
+                  for (int g = 0; g < S::STEP; g += 4)
+                    {
+                      double xv[4], pv[4], rv[4], wv[4], dv[4];
 #pragma unroll
-                    for (int u = 0; u < 4; ++u)
-                      if (const u32 i = i0 + u * R; i < r1)
-                        {
-                          const u64    o  = (u64)i * B + j;
-                          const double rn = axpbyOne<double>(1.0, 1.0, rv[u], 1.0, nalpha, wv[u]);
-                          const double zn = dv[u] * rn;
-                          xn[o] = axpbyOne<double>(1.0, 1.0, xv[u], 1.0, alpha, pv[u]);
-                          r[o]  = rn;
-                          accZ  = fma(zn, rn, accZ);
-                          accR  = fma(rn, rn, accR);
-                        }
-                  }
+                      for (int t = 0; t < 4; ++t)
+                        if (const u32 i = i0 + (g + t) * R; i < r1)
+                          {
+                            const u64 o = (u64)i * B + j;
+                            xv[t] = x[o], pv[t] = p[o], rv[t] = r[o], wv[t] = w[o], dv[t] = d[i];
+                          }
+#pragma unroll
+                      for (int t = 0; t < 4; ++t)
+                        if (const u32 i = i0 + (g + t) * R; i < r1)
+                          {
+                            const int     u  = (g + t) % U;
+                            const u64     o  = (u64)i * B + j;
+                            const double  rn = axpbyOne<double>(1.0, 1.0, rv[t], 1.0, nalpha, wv[t]);
+                            const double  zn = dv[t] * rn;
+                            xn[o]   = axpbyOne<double>(1.0, 1.0, xv[t], 1.0, alpha, pv[t]);
+                            r[o]    = rn;
+                            accZ[u] = fma(zn, rn, accZ[u]);
+                            accR[u] = fma(rn, rn, accR[u]);
+                          }
+                    }
               }
-            red[0][threadIdx.x] = accZ;
-            red[1][threadIdx.x] = accR;
-            __syncthreads();
+            const double sz = blockSum<C>(accZ, red[0]), sr = blockSum<C>(accR, red[1]);
             if (ty == 0 && j < B)
               {
-                double sz = 0.0, sr = 0.0;
-                for (int q = 0; q < R; ++q)
-                  {
-                    sz += red[0][q * C + tx];
-                    sr += red[1][q * C + tx];
-                  }
                 partials[(u64)blockIdx.x * 2 * B + j]     = sz;
                 partials[(u64)blockIdx.x * 2 * B + B + j] = sr;
               }
@@ -319,49 +362,60 @@ namespace dfx
       }
 
       // partial sums of |a1 a_j x_ij + b1 b_j y_ij|^2 per column without
-      // writing the combination: colDotsK's rows, lanes and combine and the
+      // writing the combination: colDotsK's rows, lanes and folds and the
       // blocked axpby's element, so the norms are those of the separate
       // launches bit for bit (N x B arrays with leading dimension B)
       template <int C>
-      __global__ void combNormsK(double a1, const double *a, const double *x, double b1,
-                                 const double *b, const double *y, u32 N, u32 B,
-                                 u32 rowsPerBlock, double *partials)
+      __global__ __launch_bounds__(TPB) void combNormsK(double a1, const double *a,
+                                                        const double *x, double b1,
+                                                        const double *b, const double *y, u32 N,
+                                                        u32 B, u32 rowsPerBlock, double *partials)
       {
-        constexpr int R  = TPB / C;
+        using S          = DotShape<C>;
+        constexpr int R  = S::R, U = S::U;
         const int     tx = threadIdx.x % C, ty = threadIdx.x / C;
         __shared__ double red[TPB];
         const u32 r0 = blockIdx.x * rowsPerBlock;
         const u32 r1 = min(N, r0 + rowsPerBlock);
         for (u32 j0 = 0; j0 < B; j0 += C)
           {
-            const u32 j   = j0 + tx;
-            double    acc = 0.0;
+            const u32 j = j0 + tx;
+            double    acc[U]{};
             if (j < B)
               {
                 const double aj = a[j], bj = b[j];
-                for (u32 i = r0 + ty; i < r1; i += R)
-                  {
-                    const u64    o = (u64)i * B + j;
-                    const double v = axpbyOne<double>(a1, aj, x[o], b1, bj, y[o]);
-                    acc            = fma(v, v, acc);
-                  }
+                for (u32 i0 = r0 + ty; i0 < r1; i0 += S::STEP * R)
+#pragma unroll
+                  for (int g = 0; g < S::STEP; g += 4)
+                    {
+                      double xv[4], yv[4];
+#pragma unroll
+                      for (int t = 0; t < 4; ++t)
+                        if (const u32 i = i0 + (g + t) * R; i < r1)
+                          {
+                            const u64 o = (u64)i * B + j;
+                            xv[t] = x[o], yv[t] = y[o];
+                          }
+#pragma unroll
+                      for (int t = 0; t < 4; ++t)
+                        if (i0 + (g + t) * R < r1)
+                          {
+                            const int    u = (g + t) % U;
+                            const double v = axpbyOne<double>(a1, aj, xv[t], b1, bj, yv[t]);
+                            acc[u]         = fma(v, v, acc[u]);
+                          }
+                    }
               }
-            red[threadIdx.x] = acc;
-            __syncthreads();
+            const double s = blockSum<C>(acc, red);
             if (ty == 0 && j < B)
-              {
-                double s = 0.0;
-                for (int q = 0; q < R; ++q)
-                  s += red[q * C + tx];
-                partials[(u64)blockIdx.x * B + j] = s;
-              }
+              partials[(u64)blockIdx.x * B + j] = s;
             __syncthreads();
           }
       }
 
       // one workgroup per column: thread t adds partials t, t + 256, ... in
       // order, then a fixed-shape tree over the 256 sums (deterministic; the
-      // partial count depends on N only, so a column's result does not
+      // partial count depends on the rows only, so a column's result does not
       // depend on how many columns share the call).  Columns from hostFrom on
       // also go to host (pinned memory).  All latency: eight loads are in
       // flight together, the tree's last six levels stay in one wave
@@ -767,13 +821,6 @@ namespace dfx
       checkLaunch("enrichedBlock");
     }
 
-    namespace
-    {
-      // row blocks of the column dots: 64 rows or more (enough workgroups for
-      // the GPU from small vectors on), at most 1024 blocks
-      u32 dotBlocks(u32 N) { return std::max(1u, std::min(1024u, (u32)(((u64)N + 63) / 64))); }
-    } // namespace
-
     void colDotsFinal(hipStream_t s, const double *partials, u32 nBlocks, u32 B, double *out,
                       double *host, u32 hostFrom)
     {
@@ -781,25 +828,52 @@ namespace dfx
       checkLaunch("colDotsFinal");
     }
 
+    namespace
+    {
+      // pass 1 over x's rows; the number of partial sums per column
+      template <class T>
+      u32 colDotsPartials(hipStream_t s, View<const T> x, View<const T> y, double *partials)
+      {
+        const u32 B = x.B, nBlocks = dotBlocks(x.N), rows = dotRows(x.N, nBlocks);
+        if (B <= 8)
+          colDotsK<T, 8><<<nBlocks, TPB, 0, s>>>(x.p, x.ld, y.p, y.ld, x.N, B, rows, partials);
+        else if (B <= 16)
+          colDotsK<T, 16><<<nBlocks, TPB, 0, s>>>(x.p, x.ld, y.p, y.ld, x.N, B, rows, partials);
+        else if (B <= 32)
+          colDotsK<T, 32><<<nBlocks, TPB, 0, s>>>(x.p, x.ld, y.p, y.ld, x.N, B, rows, partials);
+        else
+          colDotsK<T, 64><<<nBlocks, TPB, 0, s>>>(x.p, x.ld, y.p, y.ld, x.N, B, rows, partials);
+        checkLaunch("colDots");
+        return nBlocks;
+      }
+    } // namespace
+
     template <class T>
     void colDots(hipStream_t s, View<const T> x, View<const T> y, double *partials,
                  double *out)
     {
-      const u32 B = x.B;
+      if (!x.B)
+        return;
+      const u32 nBlocks = colDotsPartials<T>(s, x, y, partials);
+      colDotsFinal(s, partials, nBlocks, x.B, out);
+    }
+
+    void colDotsApart(hipStream_t s, View<const double> x, View<const double> y, u32 nC,
+                      double *partials, double *out)
+    {
+      const u32 B = x.B, nE = x.N - nC;
       if (!B)
         return;
-      const u32 nBlocks = dotBlocks(x.N);
-      const u32 rows = (x.N + nBlocks - 1) / nBlocks;
-      if (B <= 8)
-        colDotsK<T, 8><<<nBlocks, TPB, 0, s>>>(x.p, x.ld, y.p, y.ld, x.N, B, rows, partials);
-      else if (B <= 16)
-        colDotsK<T, 16><<<nBlocks, TPB, 0, s>>>(x.p, x.ld, y.p, y.ld, x.N, B, rows, partials);
-      else if (B <= 32)
-        colDotsK<T, 32><<<nBlocks, TPB, 0, s>>>(x.p, x.ld, y.p, y.ld, x.N, B, rows, partials);
-      else
-        colDotsK<T, 64><<<nBlocks, TPB, 0, s>>>(x.p, x.ld, y.p, y.ld, x.N, B, rows, partials);
-      checkLaunch("colDots");
-      colDotsFinal(s, partials, nBlocks, B, out);
+      const u32 nBlocks = colDotsPartials<double>(s, View<const double>{x.p, nC, B, x.ld},
+                                                  View<const double>{y.p, nC, B, y.ld}, partials);
+      if (nE)
+        {
+          rowProductsK<<<gridFor((u64)nE * B), TPB, 0, s>>>(
+            x.p + (u64)nC * x.ld, x.ld, y.p + (u64)nC * y.ld, y.ld, nE, B,
+            partials + (u64)nBlocks * B);
+          checkLaunch("rowProducts");
+        }
+      colDotsFinal(s, partials, nBlocks + nE, B, out);
     }
 
     void combinationNorms(hipStream_t s, double a1, const double *a, View<const double> x,
@@ -812,7 +886,7 @@ namespace dfx
       DFX_REQUIRE(x.ld == B && y.ld == B && y.N == N && y.B == B,
                   "combination norms: contiguous multivectors of one shape expected");
       const u32 nBlocks = dotBlocks(N);
-      const u32 rows = (N + nBlocks - 1) / nBlocks;
+      const u32 rows    = dotRows(N, nBlocks);
       if (B <= 8)
         combNormsK<8><<<nBlocks, TPB, 0, s>>>(a1, a, x.p, b1, b, y.p, N, B, rows, partials);
       else if (B <= 16)
@@ -837,7 +911,7 @@ namespace dfx
                   "CG update: contiguous multivectors expected");
       // the partition of colDots
       const u32 nBlocks = dotBlocks(N);
-      const u32 rows = (N + nBlocks - 1) / nBlocks;
+      const u32 rows    = dotRows(N, nBlocks);
       auto go = [&](auto kern) {
         kern<<<nBlocks, TPB, 0, s>>>(x.p, xn.p, r.p, p.p, w.p, d, zr, pw, N, B, rows, partials);
       };

@@ -42,6 +42,10 @@ namespace dfx
     void colDotsFinal(hipStream_t s, const double *partials, u32 nBlocks, u32 B, double *out,
                       double *host = nullptr, u32 hostFrom = 0);
     constexpr u32 DOT_PARTIALS = 2048; // rows of partial sums a CG work buffer holds
+    // the column dots with every row from nC on (at most DOT_PARTIALS / 2) a
+    // partial sum of its own: the bits of slotSumDot, any columns and strides
+    void colDotsApart(hipStream_t s, View<const double> x, View<const double> y, u32 nC,
+                      double *partials, double *out);
 
     // out[j] = sum_i (a1 a[j] x_ij + b1 b[j] y_ij)^2 without forming the
     // combination: the bits of the blocked axpby followed by colDots
@@ -180,8 +184,9 @@ namespace dfx
     void slotSum(hipStream_t s, const dfx_op *op, const T *slots, View<T> x, View<T> y,
                  bool zeroX, const ResFuse<T> *rf);
     // slotSum (rows held at zero cleared in both) and the column dots x.y into
-    // out (device) in one pass; partials: DOT_PARTIALS B doubles.  False
-    // (nothing done) for shapes it does not take: odd or more than 128 columns
+    // out (device) in one pass, the bits of colDotsApart; partials: DOT_PARTIALS
+    // B doubles.  False (nothing done) for shapes it does not take: odd or more
+    // than 128 columns
     bool slotSumDot(hipStream_t s, const dfx_op *op, const double *slots, View<double> x,
                     View<double> y, double *partials, double *out);
     // out[s] = d[map[s]] (map[s] < nC) else 1, for every slot of a cell->dof map

@@ -1419,11 +1419,7 @@ extern "C"
           else
             {
               // z.r of this iteration is the previous iteration's z.r_new
-              if (!applyDot(A, pv, w, part, dPw))
-                {
-                  applyOp<double>(A, pv, w);
-                  k::colDots<double>(s, cv(pv), cv(w), part, dPw);
-                }
+              applyDot(A, pv, w, part, dPw);
             }
           if (iter > 0 && fusedCG)
             {

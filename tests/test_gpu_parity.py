@@ -549,13 +549,14 @@ def test_cg_poisson(ctx, probs):
     assert rel(x.to_numpy(), xo) < 1e-8
 
 
-@pytest.mark.parametrize("B", [4, 20, 40])
+@pytest.mark.parametrize("B", [1, 4, 7, 12, 20, 40, 66])
 def test_cg_fused_update_is_bit_identical(ctx, probs, B, monkeypatch):
-    """With a Jacobi preconditioner one launch updates x, r and z and forms
-    the dots z.r and r.r of a PCG iteration, on the same rows, lanes and
-    combine as the separate launches (DFX_FUSE_CG=0): the iterations, the
-    residual norms and the solution are the same bits (16-, 32- and
-    64-column lane shapes).  The convergence test one iteration behind the
+    """With a Jacobi preconditioner one launch updates x and r and forms
+    the dots z.r and r.r of a PCG iteration and one more the search direction,
+    on the same rows, lanes and folds as the separate launches (DFX_FUSE_CG=0):
+    the iterations, the residual norms and the solution are the same bits
+    (8-, 16-, 32- and 64-column shapes, search directions of odd and even
+    counts).  The convergence test one iteration behind the
     device (DFX_CG_PIPELINE, default) gives the same bits as the test after
     every iteration, for a solve that converges (columns at different
     iterations) and for one stopped by the iteration limit."""
