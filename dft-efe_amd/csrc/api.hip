@@ -40,20 +40,33 @@ namespace dfx
   // reads every cell's product once through memory where the colour path adds
   // to Y in place; it pays for that by filling the GPU with one or two launches
   // instead of eight or more.  The line lies where the slots' traffic wins
-  // that back.  Measured, slot against colour path (us per apply): 12^3 cells
-  // at p = 3, FP64, 1 / 64 / 200 columns (1 / 64 / 201 MiB of slots) 34 / 79 /
-  // 273 against 89 / 133 / 311; 24^3 cells at p = 4, FP64, 64 / 128 / 200
-  // columns (0.9 / 1.7 / 2.7 GiB) 1071 / 2011 / 3486 against 1263 / 2075 / 3366;
-  // FP32, 64 / 128 / 200 columns (0.4 / 0.9 / 1.3 GiB) 548 / 995 / 1853 against
-  // 619 / 997 / 1799; per degree step of the residual filter 24^3 at p = 4
-  // FP32 72 / 128 columns 1071 / 1633 against 1216 / 1596.  Both paths give the
-  // same bits
+  // that back.  Both paths give the same bits.  Measured, colour against slot
+  // path (us per apply, enriched meshes of n^3 cells):
+  //   FP64, up to 1 GiB of slots: slots are ahead at every size.  12^3, p = 3,
+  //   1 / 64 / 200 columns (1 / 64 / 201 MiB) 89 / 133 / 311 against 34 / 79 /
+  //   273; 24^3, p = 4, 64 columns (861 MiB) 1181 against 1017; 20^3, p = 4, 128
+  //   columns (1012 MiB) 1310 against 1202; 32^3, p = 3, 64 columns (1042 MiB,
+  //   the line) 1040 against 1035.
+  //   FP32, up to 96 columns: slots are ahead (28^3, p = 4, 64 / 96 columns,
+  //   679 / 1018 MiB: 838 / 1286 against 806 / 1147).
+  //   FP32, more than 96 columns, cells of up to 192 dofs whose classes share a
+  //   colour's launch (p = 4): a chunk is 64 columns on both paths and the
+  //   colours fill the GPU, so the slots' traffic decides.  24^3, residual
+  //   step, 100 / 112 / 128 columns (673 / 754 / 861 MiB): colour 0.4 % behind,
+  //   1.4 and 3.8 % ahead; plain, 22^3, 128 columns (667 MiB) 2.2 % behind, 24^3
+  //   and 26^3, 112 columns (754, 953 MiB) 1.5 and 2.3 % ahead.  With more than
+  //   128 columns (three chunks) earlier: 19^3, 160 columns (545 MiB) 2.2 %
+  //   behind, 20^3, 160 / 176 columns (633 / 696 MiB) 4.0 and 2.7 % ahead.  Cells
+  //   of up to 128 dofs (p = 3) stay ahead in slots (28^3, 128 columns, 704 MiB:
+  //   12 %), larger ones as well (24^3, p = 4, 24 atoms, 128 columns: 23 %)
   template <class T>
   bool slotPath(const dfx_op *op, View<const T> X)
   {
     const u64 bytes = op->sumNe * X.B * sizeof(T);
-    return op->slotsOk && op->ctx->useSlots && bytes <= SLOT_BYTES &&
-           k::slotAddressable<T>(op, X);
+    u64       limit = SLOT_BYTES;
+    if (sizeof(T) == 4 && X.B > 96 && op->merged192 && k::cellBufferPath<T>(op, X, X))
+      limit = (X.B > 128 ? 608ull : 704ull) << 20;
+    return op->slotsOk && op->ctx->useSlots && bytes <= limit && k::slotAddressable<T>(op, X);
   }
 
   // op's scratch of at least `bytes`.  The generation changes before the old

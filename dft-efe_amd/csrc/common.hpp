@@ -286,7 +286,7 @@ namespace dfx
     u32 slot0, rest;
   };
   constexpr u32 ROW_ZERO = 31, ROW_COUNT_SHIFT = 27;
-  // slot bytes up to which an apply takes the slot path (see slotPath)
+  // slot bytes above which no apply takes the slot path (see slotPath)
   constexpr u64 SLOT_BYTES = 1ull << 30;
 
   // one profiled kernel launch
@@ -349,6 +349,7 @@ struct dfx_op
   // constraints are homogeneous Dirichlet ones on classical rows); per
   // classical row its slots in launch order; the enriched dofs' map slots
   bool slotsOk = false, zeroRows = false;
+  bool merged192 = false; // FP32: one launch a colour, the largest cells of 129..192 dofs
   std::vector<dfx::Launch> slotLaunches64, slotLaunches32;
   dfx::DevBuf metaSlots, slotMap, rowHeads, slotRest, enrMapSlots;
   // standalone gather / scatter (dof -> slots CSR, slots in cell order)

@@ -339,6 +339,7 @@ namespace dfx
     };
     buildLaunches(op->launches64, merge64, true);
     buildLaunches(op->launches32, merge32, false);
+    op->merged192 = merge32 && maxMtw == 3;
 
     // first-touch bits in launch order: the first cell to reach a classical
     // dof stores its contribution, later cells add to it

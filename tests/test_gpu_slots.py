@@ -335,3 +335,31 @@ def test_widths_tuned_on_one_path_stay_there(ctx, probs, B, dtype, monkeypatch):
     monkeypatch.delenv("DFX_CELL_TUNE_NT")
     assert np.array_equal(run(ops.H.apply), before)
     assert np.array_equal(run(ops.H.apply_noalloc), before)
+
+
+def test_applies_on_both_sides_of_the_slot_limits(ctx):
+    """1022 chained cells of 130 dofs: the widths next to the limits of the slot path
+    (FP64 1 GiB of products; FP32 608 MiB above 128 columns where the colour path has
+    its buffer kernel) take the path they should and give the same bits there."""
+    cells, n = 1022, 130
+    cmap = (120 * np.arange(cells)[:, None] + np.arange(n)).astype(np.uint32)
+    N = int(cmap.max()) + 1
+    A = O.rng_uniform(9, -1, 1, n * n)
+    op = dfx.CellOperator(ctx, np.full(cells, n), cmap.ravel(), np.tile(A, cells), N,
+                          keep_fp32=True)
+    rows, colours = cells * n, op.info()["nColors"]
+    assert colours > 1
+    for dtype, size, limit, widths in ((dfx.F64, 8, 1024, (1010, 1012)),
+                                       (dfx.F32, 4, 608, (1196, 1200, 1201))):
+        for B in widths:
+            slots = rows * B * size <= limit << 20 or B == 1201
+            X, Ya, Yb = (dfx.MultiVector(ctx, N, B, dtype) for _ in range(3))
+            X.fill_random(B, -1.0, 1.0)
+            op.set_profiling(True)
+            op.apply(X, Ya)
+            assert op.profile(reset=True)["launches"] == (1 if slots else colours), B
+            op.set_profiling(False)
+            op.apply_noalloc(X, Yb)
+            assert Ya.l2norms().min() > 0.0
+            Ya.axpby(1.0, Ya, -1.0, Yb)
+            assert not Ya.l2norms().any(), B
