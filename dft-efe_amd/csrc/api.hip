@@ -137,10 +137,10 @@ namespace dfx
       {
         k::cellSlots<T>(s, op, l, frag, Xc, slots, dsc, xe, mask);
         const double B = X.B, sz = sizeof(T);
-        // cell matrices and the map once, rows of X gathered, slots written
+        // distinct cell matrices and the map once, rows of X gathered, slots written
         // and read back, Y written
         r.flops += 2.0 * B * (double)l.sumN2;
-        r.bytes += sz * (double)l.sumN2 + 4.0 * (double)l.sumN + 3.0 * sz * B * (double)l.sumN +
+        r.bytes += sz * (double)l.distinctN2 + 4.0 * (double)l.sumN + 3.0 * sz * B * (double)l.sumN +
                    (dsc ? 8.0 * (double)l.sumNc : 0.0);
       }
     r.bytes += sizeof(T) * (double)X.B * op->nDofs;
@@ -245,9 +245,9 @@ namespace dfx
           {
             const double B = X.B, sz = sizeof(T);
             r.flops += 2.0 * B * (double)l.sumN2;
-            // cell matrices once, the map, gathered X rows, classical rows of
+            // distinct cell matrices once, the map, gathered X rows, classical rows of
             // Y written (and read unless first touched), enriched partials
-            r.bytes += sz * (double)l.sumN2 + 4.0 * (double)l.sumN + sz * B * (double)l.sumN +
+            r.bytes += sz * (double)l.distinctN2 + 4.0 * (double)l.sumN + sz * B * (double)l.sumN +
                        sz * B * (2.0 * (double)l.sumNc - (double)l.sumFirst) +
                        sz * B * (double)(l.sumN - l.sumNc) +
                        (dsc ? 8.0 * (double)l.sumNc : 0.0);

@@ -273,6 +273,7 @@ namespace dfx
     u64 sumNc;  // sum of classical rows
     u64 sumFirst = 0; // classical rows stored on first touch (not read)
     u32 color    = 0; // launches of one colour touch disjoint classical dofs
+    u64 distinctN2 = 0; // sum of n_e^2 over the launch's distinct matrices
   };
 
   // a row that a gather takes as 0 (never a dof: nDofs <= 2^32 - 2)

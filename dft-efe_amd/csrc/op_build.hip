@@ -527,6 +527,29 @@ namespace dfx
     }
   } // namespace
 
+  namespace
+  {
+    // per launch over `meta`, the n_e^2 of the matrices it reads, each once
+    std::vector<u64> distinctN2(const std::vector<Launch> &L, const std::vector<CellMeta> &meta)
+    {
+      std::vector<u64>                 out;
+      std::vector<std::pair<u64, u64>> m; // (offset, n^2)
+      for (const Launch &l : L)
+        {
+          m.clear();
+          for (u32 q = l.begin; q < l.end; ++q)
+            m.emplace_back(meta[q].fragOff64, (u64)meta[q].n * meta[q].n);
+          std::sort(m.begin(), m.end());
+          m.erase(std::unique(m.begin(), m.end()), m.end());
+          u64 s = 0;
+          for (const auto &x : m)
+            s += x.second;
+          out.push_back(s);
+        }
+      return out;
+    }
+  } // namespace
+
   // Everything that can fail for want of memory comes first, into buffers of
   // its own: a refused update leaves the operator as it was.  A store keeps its
   // memory where its length stays the same (its old matrices are then
@@ -546,19 +569,24 @@ namespace dfx
     upload(order, op->hOrder, st);
     upload(stored, P.stored, st);
     upload(meta, P.meta, st);
-    if (op->slotsOk)
-      {
-        std::vector<CellMeta> ms(op->nCells);
-        for (u32 q = 0; q < op->nCells; ++q)
-          ms[q] = P.meta[op->hSlotPos[q]];
-        upload(metaSlots, ms, st);
-      }
+    std::vector<CellMeta> ms(op->slotsOk ? op->nCells : 0); // slot order
+    for (u32 q = 0; q < ms.size(); ++q)
+      ms[q] = P.meta[op->hSlotPos[q]];
+    upload(metaSlots, ms, st);
+    std::vector<Launch> *const lists[] = {&op->launches64, &op->launches32, &op->slotLaunches64,
+                                          &op->slotLaunches32};
+    std::vector<u64> distinct[4];
+    for (int i = 0; i < 4; ++i)
+      distinct[i] = distinctN2(*lists[i], i < 2 ? P.meta : ms);
     if (op->frag64.bytes != P.len64 * sizeof(double))
       new64.alloc(P.len64 * sizeof(double));
     if (op->hasF32 && op->frag32.bytes != P.len32 * sizeof(float))
       new32.alloc(P.len32 * sizeof(float));
 
     ++op->gen;
+    for (int i = 0; i < 4; ++i)
+      for (size_t j = 0; j < lists[i]->size(); ++j)
+        (*lists[i])[j].distinctN2 = distinct[i][j];
     op->hMeta     = std::move(P.meta);
     op->fragLen64 = P.len64;
     op->fragLen32 = P.len32;

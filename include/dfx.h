@@ -229,8 +229,8 @@ int dfx_op_export_map(const dfx_op *op, uint32_t *cellNdofs, uint32_t *cellDofMa
  * context's two streams): with profiling on, every colour step is bracketed
  * by HIP events on the context's stream.  get_profile synchronizes, and
  * reports the colour steps ("launches"), their summed time, and the
- * algorithmic flops (2 B sum n_e^2) and bytes (matrices + map + gathered X +
- * scattered Y) of their cells.  An apply that sends its products through map
+ * algorithmic flops (2 B sum n_e^2) and bytes (distinct matrices + map +
+ * gathered X + scattered Y) of their cells.  An apply that sends its products through map
  * slots (small and middle sizes) is one "launch": its cell kernels and row
  * sums. */
 typedef struct dfx_op_profile

@@ -182,6 +182,37 @@ def test_cells_with_the_same_matrix_share_it(ctx, probs, dtype):
         assert np.array_equal(got, result(make(mats)))
 
 
+@pytest.mark.parametrize("dtype", [dfx.F64, dfx.F32])
+def test_profiled_bytes_count_a_shared_matrix_once(ctx, probs, dtype, monkeypatch):
+    """The bytes of a profile hold every distinct matrix of a launch once, on the
+    slot path (one launch here) and colour by colour (where the slots are refused);
+    the flops those of every cell; an update changes the bytes with the matrices."""
+    P = probs["c1"]
+    d = P.arrays()
+    n, nc, B = int(d["cellNdofs"][0]), len(d["cellNdofs"]), 8
+    size = 8 if dtype == dfx.F64 else 4
+    uniform = np.tile(d["K"][:n * n], nc)
+    distinct = (uniform.reshape(nc, -1) * (1.0 + np.arange(nc)[:, None] / 64.0)).ravel()
+    X, Y = (dfx.MultiVector(ctx, P.nDofs, B, dtype) for _ in range(2))
+    for limit in (None, int(d["cellNdofs"].sum()) * B * size - 1):
+        op = dfx.CellOperator(ctx, d["cellNdofs"], d["cellMap"], uniform, P.nDofs,
+                              P.nClassical, Ops(ctx, P).cons, keep_fp32=True)
+        got = []
+        for mats in (None, distinct):
+            if mats is not None:
+                op.update_cells(mats)
+            if limit:
+                monkeypatch.setenv("DFX_MAX_ALLOC_BYTES", str(limit))
+            op.set_profiling(True)
+            op.apply(X, Y)
+            got.append(op.profile(reset=True))
+            monkeypatch.delenv("DFX_MAX_ALLOC_BYTES", raising=False)
+        launches = op.info()["nColors"] if limit else 1
+        assert [g["launches"] for g in got] == [launches, launches]
+        assert got[0]["flops"] == got[1]["flops"] == 2.0 * B * nc * n * n
+        assert got[1]["bytes"] - got[0]["bytes"] == size * (nc - launches) * n * n
+
+
 def test_a_refused_update_leaves_the_operator_as_it_was(ctx, monkeypatch):
     """An update from equal to distinct cell matrices needs a larger store; where
     that allocation is refused the operator keeps its matrices (FP64, FP32 and
