@@ -1323,7 +1323,6 @@ extern "C"
       View<double> b = mvView(bmv), xo = mvView(xmv);
       DFX_REQUIRE(b.N == xo.N && b.B == xo.B, "b and x differ in shape");
       const u32 N = b.N, B = b.B;
-      View<double> x  = workView<double>(ctx, "cgs.x", N, B);
       View<double> r  = workView<double>(ctx, "cgs.r", N, B);
       View<double> w  = workView<double>(ctx, "cgs.w", N, B);
       View<double> z  = workView<double>(ctx, "cgs.z", N, B);
@@ -1365,9 +1364,9 @@ extern "C"
         {
           xs[0] = workView<double>(ctx, "cgs.xs0", N, B);
           xs[1] = workView<double>(ctx, "cgs.xs1", N, B);
-          if (fusedCG) // iteration k's x is xs[k % 2]
-            x = xs[0];
         }
+      // pipelined and fused, iteration k's x is xs[k % 2]
+      View<double> x = pipe && fusedCG ? xs[0] : workView<double>(ctx, "cgs.x", N, B);
       k::convert<double, double>(s, x, cv(xo));
       PinnedDoubles hr(2 * (size_t)B);
       EventPair     ev;

@@ -1,6 +1,8 @@
 """The PCG's dots: formed in the row sums of the apply or by a launch of their
 own, the bits of a column depend on its rows alone and not on the columns beside
 it, on profiling or on the path of the apply."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -118,3 +120,26 @@ def test_dots_of_a_column_in_any_batch(ctx, N, dtype):
             bound = EPS * (N + 2) * np.abs(X.astype(np.float64) * Y).sum(axis=0)
             assert (np.abs(got - ref) <= bound).all()
         assert np.array_equal(got, want[:B]), B
+
+
+def test_work_space_of_a_solve():
+    """r, w, z, p and two copies of x: the pipelined fused solve holds six arrays."""
+    own = dfx.Context(0)
+    N, B = 1 << 20, 8
+    one = dfx.DiagonalOperator(own, np.ones(N))
+    b, x = dfx.MultiVector(own, N, B), dfx.MultiVector(own, N, B)
+    b.fill_random(1, -1.0, 1.0)
+    one.apply(b, x)                      # the kernels are loaded
+    x.set(0.0)
+
+    def free():
+        own.synchronize()
+        f, t = C.c_size_t(), C.c_size_t()
+        assert dfx._lib.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+
+    before = free()
+    assert dfx.CGLinearSolver(own, 10, 1e-12, 1e-10, 1e10).solve(one, one, b, x) == 0
+    arrays = (before - free()) / (8.0 * N * B)
+    assert 6.0 <= arrays < 6.5
+    own.close()
