@@ -82,18 +82,23 @@ namespace dfx
 
   // The slots of an apply to X where it takes the slot path and they can be
   // had, else null: the apply then goes colour by colour, which gives the same
-  // bits without them.  Nothing is allocated while the stream is being captured
+  // bits without them.  Null also while a caller captures the stream: nothing
+  // may be allocated then, and a later, wider apply would move the buffer whose
+  // address the caller's graph holds
   template <class T>
   T *slotBuffer(dfx_op *op, View<const T> X)
   {
     if (!slotPath<T>(op, X))
       return nullptr;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (!op->ctx->ownCapture)
+      DFX_HIP(hipStreamIsCapturing(op->ctx->stream, &cap));
+    if (cap != hipStreamCaptureStatusNone)
+      return nullptr;
     const size_t bytes = (size_t)op->sumNe * X.B * sizeof(T);
     if (bytes > op->yE.bytes)
       {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        DFX_HIP(hipStreamIsCapturing(op->ctx->stream, &cap));
-        if (cap != hipStreamCaptureStatusNone)
+        if (op->ctx->ownCapture)
           return nullptr;
         try
           {

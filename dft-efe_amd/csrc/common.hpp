@@ -211,6 +211,9 @@ struct dfx_ctx
   };
   std::map<std::string, Graph> graphs;
   uint64_t graphCaptures = 0, graphReplays = 0;
+  // the stream is being captured for one of `graphs`, whose key holds the
+  // operators' buffer generations (a caller's own capture knows nothing of them)
+  bool ownCapture = false;
 };
 
 struct dfx_mv

@@ -230,13 +230,16 @@ namespace dfx
       hipGraph_t  graph = nullptr;
       CaptureLock lk(captureMutex());
       DFX_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed));
+      ctx->ownCapture = true;
       try
         {
           for (u32 d = first; d <= last; ++d)
             body(d);
+          ctx->ownCapture = false;
         }
       catch (...)
         {
+          ctx->ownCapture = false;
           (void)hipStreamEndCapture(s, &graph);
           if (graph)
             (void)hipGraphDestroy(graph);

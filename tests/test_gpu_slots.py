@@ -314,34 +314,45 @@ def test_filter_runs_where_the_slots_cannot_be_had(ctx, probs, B, prec, monkeypa
         assert np.array_equal(o[0], outs[0][0]) and np.array_equal(o[1], outs[0][1])
 
 
-def test_a_first_apply_is_captured_without_slots(ctx, probs):
-    """A classical operator's apply allocates nothing while its stream is being
-    captured, also the first one: it goes colour by colour there.  Replays give
-    the eager bits, with eager work between them."""
+def test_a_captured_apply_outlives_the_slots(ctx, probs):
+    """While a caller captures the stream an apply of a classical operator uses no
+    slots: the first one allocates nothing, and a later one does not put the slots'
+    address into the graph, which a wider apply moves.  Replays give the eager bits,
+    with eager work between them."""
     P = probs["c1"]
     B = 8
     warm, ops = Ops(ctx, P), Ops(ctx, P)
     X, Y = dfx.MultiVector(ctx, P.nDofs, B), dfx.MultiVector(ctx, P.nDofs, B)
     warm.H.apply_noalloc(X, Y)                       # the kernels are loaded
     ctx.synchronize()
-    hip, stream, graph, run = dfx._lib, C.c_void_p(), C.c_void_p(), C.c_void_p()
+    hip, stream = dfx._lib, C.c_void_p()
     assert hip.dfx_ctx_stream(ctx.h, C.byref(stream)) == 0
-    assert hip.hipStreamBeginCapture(stream, 0) == 0          # the strictest mode
-    try:
-        ops.H.apply(X, Y)
-    finally:
-        assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
-    assert hip.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)) == 0
-    for seed in range(4):
-        X.upload(guess(P, B, seed=seed))
-        Y.set(0.0)
-        assert hip.hipGraphLaunch(run, stream) == 0
-        ctx.synchronize()
-        got = Y.to_numpy()
-        want = dfx.MultiVector(ctx, P.nDofs, B)
-        ops.H.apply(mv(ctx, guess(P, B, seed=seed)), want)     # eager: in slots
-        assert np.array_equal(got, want.to_numpy())
-    assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
+    runs = []
+
+    def capture():
+        graph, run = C.c_void_p(), C.c_void_p()
+        assert hip.hipStreamBeginCapture(stream, 0) == 0          # the strictest mode
+        try:
+            ops.H.apply(X, Y)
+        finally:
+            assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+        assert hip.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)) == 0
+        runs.append((graph, run))
+
+    capture()
+    for seed, wide in enumerate((8, 8, 16, 40)):
+        Xw, want = guess(P, wide, seed=seed), dfx.MultiVector(ctx, P.nDofs, wide)
+        ops.H.apply(mv(ctx, Xw), want)                            # eager: in slots
+        if seed == 0:
+            capture()
+        X.upload(np.ascontiguousarray(Xw[:, :B]))
+        for _, run in runs:
+            Y.set(0.0)
+            assert hip.hipGraphLaunch(run, stream) == 0
+            ctx.synchronize()
+            assert np.array_equal(Y.to_numpy(), want.to_numpy()[:, :B])
+    for graph, run in runs:
+        assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
 
 
 @pytest.mark.parametrize("dtype", [dfx.F64, dfx.F32])
