@@ -333,7 +333,7 @@ struct dfx_op
   std::vector<dfx::CellMeta> hMeta;             // launch order
   std::vector<dfx::u32> hSlotPos;               // slot order -> launch position
   std::vector<dfx::Launch> launches64, launches32;
-  dfx::u64 fragLen64 = 0, fragLen32 = 0;
+  dfx::u64 fragLen64 = 0, fragLen32 = 0; // taken by the distinct matrices
   dfx::DevBuf map, meta, frag64, frag32;
   dfx::DevBuf first;     // per launch position, 8 words: first-touch bits of classical rows
   // per launch position, 8 words: last-touch bits of the unconstrained

@@ -448,9 +448,18 @@ namespace dfx
 
   namespace
   {
+    // elements of a cell matrix in fragment order: whole 16-row tiles and
+    // blocks of 4 G columns
+    template <class T>
+    u64 fragLength(u64 n)
+    {
+      constexpr u64 KB = 64 / sizeof(T);
+      return 16 * ((n + 15) / 16) * (KB * ((n + KB - 1) / KB));
+    }
+
     // Where the cell matrices of an upload go: per launch position the metadata
     // with the fragment offsets, the launch positions whose matrices are stored
-    // (`stored`), and the stores' lengths
+    // (`stored`), and the lengths that they take
     struct Placement
     {
       std::vector<CellMeta> meta;
@@ -511,11 +520,10 @@ namespace dfx
             {
               r = q;
               P.stored.push_back(q);
-              const u64 n = P.meta[q].n, mpad = 16 * ((n + 15) / 16);
               P.meta[q].fragOff64 = P.len64;
               P.meta[q].fragOff32 = P.len32;
-              P.len64 += mpad * (8 * ((n + 7) / 8));
-              P.len32 += mpad * (16 * ((n + 15) / 16));
+              P.len64 += fragLength<double>(P.meta[q].n);
+              P.len32 += fragLength<float>(P.meta[q].n);
             }
           else
             {
@@ -550,14 +558,15 @@ namespace dfx
     }
   } // namespace
 
-  // Everything that can fail for want of memory comes first, into buffers of
-  // its own: a refused update leaves the operator as it was.  A store keeps its
-  // memory where its length stays the same (its old matrices are then
-  // overwritten by the last two launches)
+  // The stores have room for a matrix per cell and, like the metadata, stay
+  // where they are from the operator's creation on: an update needs no memory
+  // for them however many matrices differ, and a graph that a caller captured
+  // an apply into stays valid.  What can fail for want of memory comes first: a
+  // refused update leaves the operator as it was
   void uploadCellMatrices(dfx_op *op, const double *mats, bool device)
   {
     hipStream_t st = op->ctx->stream;
-    DevBuf      raw, rawOff, order, stored, meta, metaSlots, new64, new32;
+    DevBuf      raw, rawOff, order, stored;
     const double *dmats = mats;
     if (!device)
       {
@@ -568,34 +577,41 @@ namespace dfx
     Placement P = placeCellMatrices(op, dmats, rawOff.as<u64>());
     upload(order, op->hOrder, st);
     upload(stored, P.stored, st);
-    upload(meta, P.meta, st);
     std::vector<CellMeta> ms(op->slotsOk ? op->nCells : 0); // slot order
     for (u32 q = 0; q < ms.size(); ++q)
       ms[q] = P.meta[op->hSlotPos[q]];
-    upload(metaSlots, ms, st);
     std::vector<Launch> *const lists[] = {&op->launches64, &op->launches32, &op->slotLaunches64,
                                           &op->slotLaunches32};
     std::vector<u64> distinct[4];
     for (int i = 0; i < 4; ++i)
       distinct[i] = distinctN2(*lists[i], i < 2 ? P.meta : ms);
-    if (op->frag64.bytes != P.len64 * sizeof(double))
-      new64.alloc(P.len64 * sizeof(double));
-    if (op->hasF32 && op->frag32.bytes != P.len32 * sizeof(float))
-      new32.alloc(P.len32 * sizeof(float));
+    const size_t metaBytes = P.meta.size() * sizeof(CellMeta), msBytes = ms.size() * sizeof(CellMeta);
+    if (!op->frag64.p) // the operator is being made
+      {
+        u64 cap64 = 0, cap32 = 0;
+        for (const CellMeta &m : P.meta)
+          {
+            cap64 += fragLength<double>(m.n);
+            cap32 += fragLength<float>(m.n);
+          }
+        op->meta.alloc(metaBytes);
+        op->metaSlots.alloc(msBytes);
+        op->frag64.alloc(cap64 * sizeof(double));
+        if (op->hasF32)
+          op->frag32.alloc(cap32 * sizeof(float));
+      }
 
     ++op->gen;
     for (int i = 0; i < 4; ++i)
       for (size_t j = 0; j < lists[i]->size(); ++j)
         (*lists[i])[j].distinctN2 = distinct[i][j];
-    op->hMeta     = std::move(P.meta);
+    op->hMeta.swap(P.meta);
     op->fragLen64 = P.len64;
     op->fragLen32 = P.len32;
-    op->meta      = std::move(meta);
-    op->metaSlots = std::move(metaSlots);
-    if (op->frag64.bytes != P.len64 * sizeof(double))
-      op->frag64 = std::move(new64);
-    if (op->hasF32 && op->frag32.bytes != P.len32 * sizeof(float))
-      op->frag32 = std::move(new32);
+    if (metaBytes)
+      DFX_HIP(hipMemcpyAsync(op->meta.p, op->hMeta.data(), metaBytes, hipMemcpyHostToDevice, st));
+    if (msBytes)
+      DFX_HIP(hipMemcpyAsync(op->metaSlots.p, ms.data(), msBytes, hipMemcpyHostToDevice, st));
     const u32 nStored = (u32)P.stored.size();
     k::repackCells<double>(st, op, nStored, stored.as<u32>(), order.as<u32>(), dmats,
                            rawOff.as<u64>(), op->frag64.as<double>());

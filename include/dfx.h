@@ -215,8 +215,9 @@ typedef struct dfx_op_info
   uint32_t maxCellDofs;
   uint64_t sumNe;       /* sum_e n_e */
   uint64_t sumNe2;      /* sum_e n_e^2 */
-  /* device bytes of the FP64 and FP32 (0 if none) stores of the distinct cell
-   * matrices: cells with bitwise equal matrices share one */
+  /* device bytes of the distinct cell matrices in the FP64 and FP32 (0 if none)
+   * stores: cells with bitwise equal matrices share one (the stores have room
+   * for a matrix per cell) */
   uint64_t matBytesF64;
   uint64_t matBytesF32;
 } dfx_op_info;

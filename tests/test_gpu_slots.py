@@ -214,9 +214,9 @@ def test_profiled_bytes_count_a_shared_matrix_once(ctx, probs, dtype, monkeypatc
 
 
 def test_a_refused_update_leaves_the_operator_as_it_was(ctx, monkeypatch):
-    """An update from equal to distinct cell matrices needs a larger store; where
-    that allocation is refused the operator keeps its matrices (FP64, FP32 and
-    the colour-by-colour path), and the same update works afterwards."""
+    """Where an update from equal to distinct cell matrices is refused for want of
+    memory the operator keeps its matrices (FP64, FP32 and the colour-by-colour
+    path); it needs no more than the copy of the caller's matrices."""
     P = c1_like(n=3, p=2)
     d = P.arrays()
     ops = Ops(ctx, P)
@@ -240,18 +240,58 @@ def test_a_refused_update_leaves_the_operator_as_it_was(ctx, monkeypatch):
 
     op, fresh = make(uniform), make(distinct)
     before, info = results(op), op.info()
-    store = fresh.info()["matBytesF64"]
-    assert distinct.nbytes < store      # the matrices themselves may be uploaded
-    monkeypatch.setenv("DFX_MAX_ALLOC_BYTES", str(store - 1))
+    assert fresh.info()["matBytesF64"] > distinct.nbytes
+    monkeypatch.setenv("DFX_MAX_ALLOC_BYTES", str(distinct.nbytes - 1))
     with pytest.raises(dfx.DfxError, match="DFX_MAX_ALLOC_BYTES"):
         op.update_cells(distinct)
-    monkeypatch.delenv("DFX_MAX_ALLOC_BYTES")
     assert op.info() == info
     for a, b in zip(results(op), before):
         assert np.array_equal(a, b)
+    # room for the matrices as the caller holds them is enough
+    monkeypatch.setenv("DFX_MAX_ALLOC_BYTES", str(distinct.nbytes))
     op.update_cells(distinct)
+    monkeypatch.delenv("DFX_MAX_ALLOC_BYTES")
     for a, b in zip(results(op), results(fresh)):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("call", ["apply", "apply_noalloc"])
+def test_a_captured_apply_outlives_an_update(ctx, probs, call):
+    """A caller's graph of an apply gives the new matrices' products after an update
+    that changes how many of them differ."""
+    P = probs["c1"]
+    d = P.arrays()
+    B, n, nc = 8, int(d["cellNdofs"][0]), len(d["cellNdofs"])
+    uniform = np.tile(d["K"][:n * n], nc)
+    distinct = (uniform.reshape(nc, -1) * (1.0 + np.arange(nc)[:, None] / 64.0)).ravel()
+    ops = Ops(ctx, P)
+
+    def make(mats):
+        return dfx.CellOperator(ctx, d["cellNdofs"], d["cellMap"], mats, P.nDofs, P.nClassical,
+                                ops.cons)
+
+    op = make(uniform)
+    X, Y = dfx.MultiVector(ctx, P.nDofs, B), dfx.MultiVector(ctx, P.nDofs, B)
+    ops.H.apply_noalloc(X, Y)                        # the kernels are loaded
+    ctx.synchronize()
+    hip, stream, graph, run = dfx._lib, C.c_void_p(), C.c_void_p(), C.c_void_p()
+    assert hip.dfx_ctx_stream(ctx.h, C.byref(stream)) == 0
+    assert hip.hipStreamBeginCapture(stream, 0) == 0
+    try:
+        getattr(op, call)(X, Y)
+    finally:
+        assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)) == 0
+    for seed, mats in enumerate((uniform, distinct, uniform)):
+        op.update_cells(mats)
+        Xs, want = guess(P, B, seed=seed), dfx.MultiVector(ctx, P.nDofs, B)
+        make(mats).apply(mv(ctx, Xs), want)
+        X.upload(Xs)
+        Y.set(0.0)
+        assert hip.hipGraphLaunch(run, stream) == 0
+        ctx.synchronize()
+        assert np.array_equal(Y.to_numpy(), want.to_numpy())
+    assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
 
 
 @pytest.mark.parametrize("name", ["c1", "hang3", "wide"])
