@@ -137,21 +137,23 @@ def test_cell_apply_narrow_tail_chunk_bitwise(ctx, probs, dtype, B):
     ops = Ops(ctx, P)
     npd = np.float64 if dtype == dfx.F64 else np.float32
     X = guess(P, B, seed=37).astype(npd)
-    outs = []
-    for cols in (slice(0, B), slice(0, B - 8), slice(B - 8, B)):
-        Xc = np.ascontiguousarray(X[:, cols])
-        Yg = dfx.MultiVector(ctx, P.nDofs, Xc.shape[1], dtype)
-        ops.H.apply(mv(ctx, Xc, dtype), Yg)
-        outs.append(Yg.to_numpy())
-    assert np.array_equal(outs[0], np.hstack(outs[1:]))
+    for call in (ops.H.apply, ops.H.apply_noalloc):     # in slots and colour by colour
+        outs = []
+        for cols in (slice(0, B), slice(0, B - 8), slice(B - 8, B)):
+            Xc = np.ascontiguousarray(X[:, cols])
+            Yg = dfx.MultiVector(ctx, P.nDofs, Xc.shape[1], dtype)
+            call(mv(ctx, Xc, dtype), Yg)
+            outs.append(Yg.to_numpy())
+        assert np.array_equal(outs[0], np.hstack(outs[1:]))
 
 
 @pytest.mark.parametrize("dtype", [dfx.F64, dfx.F32])
 def test_size_classes_merged_or_apart_give_the_same_bits(ctx, dtype, monkeypatch):
-    """Operators of few cells run each colour as one launch (the largest size
-    class's tile); large ones launch every size class of a colour apart, side
-    by side on two streams.  Both give the same bits: every cell computes the
-    same products and rows are completed in the same cell order."""
+    """Operators of few cells run each colour (in slots: all cells) as one launch
+    with the largest size class's tile; large ones launch every size class of a
+    colour apart, side by side on two streams (in slots: one after the other).
+    All give the same bits: every cell computes the same products and rows are
+    completed in the same cell order."""
     spec = dict(p=3, n=(4, 4, 4), lo=(-12.0,) * 3, hi=(12.0,) * 3,
                 atoms=[(0.5, -0.5, 0.25, 6)], enrich=True)
     npd = np.float64 if dtype == dfx.F64 else np.float32
@@ -161,11 +163,13 @@ def test_size_classes_merged_or_apart_give_the_same_bits(ctx, dtype, monkeypatch
         G = dfx.Problem(ctx, orthogonalize=True, **spec)
         H = G.operators(keep_fp32=True)[0]
         X = guess_like(G.nDofs, 24, seed=47).astype(npd)
-        Y = dfx.MultiVector(ctx, G.nDofs, 24, dtype)
-        H.apply(mv(ctx, X, dtype), Y)
-        outs.append(Y.to_numpy())
+        for call in (H.apply, H.apply_noalloc):
+            Y = dfx.MultiVector(ctx, G.nDofs, 24, dtype)
+            call(mv(ctx, X, dtype), Y)
+            outs.append(Y.to_numpy())
         classes.append(sorted(H.autotune(dtype, 24, reps=1)))
-    assert np.array_equal(outs[0], outs[1])
+    for o in outs[1:]:
+        assert np.array_equal(outs[0], o)
     assert classes[0] == [1, 2] and classes[1] == [2]   # apart: two classes; merged: one
 
 
@@ -194,18 +198,22 @@ def test_autotuned_widths_keep_the_bits(ctx, probs, dtype):
 
 @pytest.mark.parametrize("dtype", [dfx.F64, dfx.F32])
 def test_cell_apply_kernel_paths_agree_bitwise(ctx, probs, dtype):
-    """The buffer-addressed kernel (column count a multiple of the 16-byte
-    vector) and the pointer kernel (any other count) give the same bits per
-    column: columns are independent and both sum in the same K order."""
+    """The slot kernel (any column count) and, colour by colour (the apply without
+    allocation), the buffer-addressed kernel (column count a multiple of the
+    16-byte vector) and the pointer kernel (any other count) give the same bits per
+    column: columns are independent and all sum in the same K order."""
     P = probs["enr"]
     ops = Ops(ctx, P)
     npd = np.float64 if dtype == dfx.F64 else np.float32
     X = guess(P, 4, seed=31).astype(npd)
-    Y4 = dfx.MultiVector(ctx, P.nDofs, 4, dtype)
-    ops.H.apply(mv(ctx, X, dtype), Y4)
-    Y1 = dfx.MultiVector(ctx, P.nDofs, 1, dtype)
-    ops.H.apply(mv(ctx, np.ascontiguousarray(X[:, :1]), dtype), Y1)
-    assert np.array_equal(Y4.to_numpy()[:, :1], Y1.to_numpy())
+    outs = []
+    for call in (ops.H.apply, ops.H.apply_noalloc):
+        for n in (4, 1):
+            Y = dfx.MultiVector(ctx, P.nDofs, n, dtype)
+            call(mv(ctx, np.ascontiguousarray(X[:, :n]), dtype), Y)
+            outs.append(Y.to_numpy()[:, :1])
+    for o in outs[1:]:
+        assert np.array_equal(outs[0], o)
 
 
 def test_cell_apply_deterministic(ctx, probs):
@@ -213,11 +221,12 @@ def test_cell_apply_deterministic(ctx, probs):
     ops = Ops(ctx, P)
     X = guess(P, 40, seed=2)
     outs = []
-    for _ in range(3):
+    for call in 3 * [ops.H.apply] + 3 * [ops.H.apply_noalloc]:
         Xg, Yg = mv(ctx, X), dfx.MultiVector(ctx, P.nDofs, 40)
-        ops.H.apply(Xg, Yg)
+        call(Xg, Yg)
         outs.append(Yg.to_numpy())
-    assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])
+    for o in outs[1:]:
+        assert np.array_equal(outs[0], o)
 
 
 @pytest.mark.parametrize("name", ["hang3", "enr"])
