@@ -475,7 +475,7 @@ namespace dfx
     hipStream_t s  = op->ctx->stream;
     const u32   nE = op->nDofs - op->nClassical;
     View<const double> Xc{X.p, X.N, X.B, X.ld}, Yc{Y.p, Y.N, Y.B, Y.ld};
-    const bool         apart = op->kind == OP_CELLWISE && nE <= k::DOT_PARTIALS / 2;
+    const bool         apart = op->kind == OP_CELLWISE && nE <= DOT_BLOCKS;
     if (apart && !(op->cons && op->cons->nRows && !op->zeroRows) && !op->profiling &&
         X.N == op->nDofs && Y.N == op->nDofs && X.B == Y.B)
       if (double *slots = slotBuffer<double>(op, Xc))

@@ -279,6 +279,10 @@ namespace dfx
     u64 distinctN2 = 0; // sum of n_e^2 over the launch's distinct matrices
   };
 
+  // partial sums per column that a column dot leaves for its second pass
+  // (at most)
+  constexpr u32 DOT_BLOCKS = 4096;
+
   // a row that a gather takes as 0 (never a dof: nDofs <= 2^32 - 2)
   constexpr u32 ROW_NONE = 0xffffffffu;
 

@@ -42,16 +42,9 @@ namespace dfx
         v[e] = s;
       }
 
-      // Blocks below nE * ceil(B / 16): one enriched dof and 16 columns each
-      // (EnrReduce; first, as they run longest).  The others: one thread per
-      // classical row and V columns (V: one 16-byte vector where widths and
-      // addresses allow).  A row's first slot sits in its head, so that slot's
-      // load does not wait for the list of the others; most rows (a cell's
-      // interior) have no others.  Bound by memory: B values read per slot,
-      // written per row (p = 4, 32^3 cells, FP32, 128 columns: 3.3 GB in 645 us;
-      // p = 3, 16^3 cells, 40 columns, FP32: 68 MB in 14 us)
-      //
-      // The sum of one row's V columns from j on: the row's slots in order
+      // The sum of a row's slots in order, V columns from j on.  The first slot
+      // sits in the row's head, so that its load does not wait for the list of
+      // the others
       template <class T, int V>
       __device__ inline typename Vec<T, V>::type rowSum(RowHead h, const u32 *__restrict__ rest,
                                                         const T *__restrict__ slots, u32 B, u32 j)
@@ -80,6 +73,12 @@ namespace dfx
         return s;
       }
 
+      // Blocks below nE * ceil(B / 16): one enriched dof and 16 columns each
+      // (EnrReduce; first, as they run longest).  The others: one thread per
+      // classical row and V columns (V: one 16-byte vector where widths and
+      // addresses allow); most rows (a cell's interior) have one slot.  Bound by
+      // memory: B values read per slot, written per row (p = 3, 16^3 cells, 40
+      // columns: FP32 68 MB in 14.8 us, FP64 with the residual step 205 MB in 35.6)
       template <class T, int V, bool RES>
       __global__ __launch_bounds__(256) void slotSumK(
         const RowHead *__restrict__ heads, const u32 *__restrict__ rest,
@@ -152,25 +151,24 @@ namespace dfx
           *reinterpret_cast<vt *>(y + (u64)row * ldy + j) = s;
       }
       // The row sums with the column dots x.y of the same rows (PCG's p.w, FP64,
-      // two columns a thread, B even), in the order of dots.hpp: a workgroup is
-      // a block of rows, R = 64 / U row threads of U lanes each (R the largest
-      // power of two that B / 2 column pairs leave room for); an enriched dof's
-      // product goes to partials[nBlocks + dof].  Saves the separate dot a read
-      // of x and y and a launch (16^3 cells, p = 3, 8 columns: 7.9 + 6.3 us for
-      // the two)
+      // two columns a thread, B even), in the order of dots.hpp: a workgroup
+      // takes P column pairs of G blocks, 64 / U row threads of U lanes each; an
+      // enriched dof's product is a partial sum of its own, after the blocks'.
+      // Saves the separate dot a read of x and y and a launch (16^3 cells,
+      // p = 3, 8 columns: 7.9 + 6.3 us for the two)
       template <int U>
       __global__ __launch_bounds__(256) void slotSumDotK(
         const RowHead *__restrict__ heads, const u32 *__restrict__ rest,
         const u32 *__restrict__ enrOff, const u32 *__restrict__ enrSlots, u32 nC, u32 nE,
-        const double *__restrict__ slots, u32 B, double *x, double *y, u32 nBlocks,
-        u32 rowsPerBlock, double *__restrict__ partials)
+        const double *__restrict__ slots, u32 B, double *x, double *y, u32 nBlocks, u32 P, u32 G,
+        double *__restrict__ partials)
       {
         using T         = double;
         using vt        = Vec<double, 2>::type;
         constexpr u32 R = DOT_LANES / U;
         __shared__ EnrReduce<T> red;
         __shared__ vt           sum[256];
-        const u32 nb = (B + EnrReduce<T>::CB - 1) / EnrReduce<T>::CB;
+        const u32 nb = (B + EnrReduce<T>::CB - 1) / EnrReduce<T>::CB, nParts = nBlocks + nE;
         if (blockIdx.x < nE * nb)
           {
             const u32 g = blockIdx.x / nb;
@@ -178,21 +176,23 @@ namespace dfx
             const T   s = red.sum(enrSlots, enrOff[g], enrOff[g + 1], slots, B, j);
             if (threadIdx.x < EnrReduce<T>::CB && j < B)
               {
-                const u64 o                           = (u64)(nC + g) * B + j;
-                y[o]                                  = s;
-                partials[(u64)(nBlocks + g) * B + j] = x[o] * s;
+                const u64 o                               = (u64)(nC + g) * B + j;
+                y[o]                                      = s;
+                partials[(u64)j * nParts + nBlocks + g] = x[o] * s;
               }
             return;
           }
-        const u32 blk = blockIdx.x - nE * nb, nv = B / 2;
-        const u32 r = threadIdx.x / nv, j = (threadIdx.x - r * nv) * 2;
-        const u32 r0 = blk * rowsPerBlock, r1 = min(nC, r0 + rowsPerBlock);
-        vt        acc[U]{};
-        if (r < R)
-          for (u32 i0 = r0 + r; i0 < r1; i0 += DOT_LANES)
+        const u32  nCh = (B / 2 + P - 1) / P, wg = blockIdx.x - nE * nb;
+        const u32  sub = threadIdx.x / (R * P), q = threadIdx.x - sub * R * P, r = q / P;
+        const u32  blk = wg / nCh * G + sub, j = (wg % nCh * P + (q - r * P)) * 2;
+        const bool on  = sub < G && blk < nBlocks && j < B;
+        const u32  nGroups = (nC + DOT_LANES - 1) / DOT_LANES;
+        vt         acc[U]{};
+        if (on)
+          for (u32 g = blk; g < nGroups; g += nBlocks)
 #pragma unroll
             for (int u = 0; u < U; ++u)
-              if (const u32 row = i0 + u * R; row < r1)
+              if (const u32 row = g * DOT_LANES + r + u * R; row < nC)
                 {
                   const RowHead h = heads[row];
                   const u64     o = (u64)row * B + j;
@@ -213,12 +213,15 @@ namespace dfx
 #pragma unroll
         for (u32 h = R / 2; h > 0; h >>= 1)
           {
-            if (r < h)
-              sum[threadIdx.x] += sum[threadIdx.x + h * nv];
+            if (r < h && sub < G)
+              sum[threadIdx.x] += sum[threadIdx.x + h * P];
             __syncthreads();
           }
-        if (threadIdx.x < nv)
-          *reinterpret_cast<vt *>(partials + (u64)blk * B + j) = sum[threadIdx.x];
+        if (on && r == 0)
+          {
+            partials[(u64)j * nParts + blk]       = sum[threadIdx.x][0];
+            partials[(u64)(j + 1) * nParts + blk] = sum[threadIdx.x][1];
+          }
       }
     } // namespace
 
@@ -228,26 +231,33 @@ namespace dfx
       const u32 nC = op->nClassical, nE = op->nDofs - nC, B = y.B;
       auto aligned = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
       if (B < 2 || B % 2 || B > 128 || x.ld != B || y.ld != B || !aligned(slots) ||
-          !aligned(x.p) || !aligned(y.p) || !nC || nE > DOT_PARTIALS / 2)
+          !aligned(x.p) || !aligned(y.p) || !nC || nE > DOT_BLOCKS ||
+          nC > 0xffffff00u)
         return false;
-      const u32 nBlocks = dotBlocks(nC), rows = dotRows(nC, nBlocks);
+      const u32 nBlocks = dotBlocks(nC), nv = B / 2;
       const u32 nb      = (B + EnrReduce<double>::CB - 1) / EnrReduce<double>::CB;
+      // 4 U column pairs fit beside 64 / U row threads.  A thread's rows wait for
+      // each other's lists, so U stays at 4 or less (40 columns, 117 649 rows: U = 8
+      // took the solve 3 % longer) and lower where workgroups are few (20 columns,
+      // 35 937 rows: 9 %); the pairs spread evenly over the chunks; with one or
+      // two pairs a workgroup holds several blocks
+      u32 U = nv <= 4 ? 1 : nv <= 8 ? 2 : 4;
+      while (U > 1 && (u64)nBlocks * ((nv + 4 * U - 1) / (4 * U)) < 640)
+        U /= 2;
+      const u32 nCh = (nv + 4 * U - 1) / (4 * U), P = (nv + nCh - 1) / nCh;
+      const u32 G    = std::max(1u, 256 / (DOT_LANES / U * P));
+      const u32 grid = nE * nb + (nBlocks + G - 1) / G * nCh;
       auto go = [&](auto kern) {
-        kern<<<nE * nb + nBlocks, 256, 0, s>>>(
-          op->rowHeads.as<RowHead>(), op->slotRest.as<u32>(), op->enrSlotOffsets.as<u32>(),
-          op->enrMapSlots.as<u32>(), nC, nE, slots, B, x.p, y.p, nBlocks, rows, partials);
+        kern<<<grid, 256, 0, s>>>(op->rowHeads.as<RowHead>(), op->slotRest.as<u32>(),
+                                  op->enrSlotOffsets.as<u32>(), op->enrMapSlots.as<u32>(), nC, nE,
+                                  slots, B, x.p, y.p, nBlocks, P, G, partials);
       };
-      // row threads: 256 / (B / 2), rounded down to a power of two, at most 64
-      if (B <= 8)
-        go(slotSumDotK<1>);
-      else if (B <= 16)
-        go(slotSumDotK<2>);
-      else if (B <= 32)
-        go(slotSumDotK<4>);
-      else if (B <= 64)
-        go(slotSumDotK<8>);
-      else
-        go(slotSumDotK<16>);
+      switch (U)
+        {
+          case 1: go(slotSumDotK<1>); break;
+          case 2: go(slotSumDotK<2>); break;
+          default: go(slotSumDotK<4>); break;
+        }
       checkLaunch("slotSumDot");
       colDotsFinal(s, partials, nBlocks + nE, B, out);
       return true;

@@ -5,6 +5,7 @@
 // are addressed in place, without the reference's per-dof copy loops,
 // src/linearAlgebra/ChebyshevFilteredEigenSolver.t.cpp:246-333).
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "dots.hpp"
@@ -216,80 +217,129 @@ namespace dfx
           y[(u64)(nC + i) * ldy + j] = ((part[0][cj] + part[1][cj]) + part[2][cj]) + part[3][cj];
       }
 
-      // pass 1 of the column dots: block b owns rows [b*rows, (b+1)*rows);
-      // threads are C columns x R row threads of U lanes each (dots.hpp)
+      // pass 1 of the column dots in the order of dots.hpp.  A workgroup takes C
+      // columns of one block: C columns x R row threads of U lanes each
       template <int C>
       struct DotShape
       {
         static constexpr int R = TPB / C, U = DOT_LANES / R;
-        // rows a thread takes per turn of its loop, in groups of four whose
-        // loads are in flight together; the t-th belongs to lane t % U
+        // rows a thread takes per turn of its loop, in batches of four whose
+        // loads are in flight together: the f-th is lane f % U of group f / U
         static constexpr int STEP = U > 4 ? U : 4;
         static_assert(R <= DOT_LANES && STEP % U == 0, "whole lanes");
       };
-      // a column's sum over the block, in the threads with ty == 0
+      // the workgroup's block and first column; one row of the block's turn at
+      // group g
       template <int C>
-      __device__ inline double blockSum(double (&acc)[DotShape<C>::U], double *red)
+      struct DotPlace
       {
-        constexpr int R  = DotShape<C>::R;
-        red[threadIdx.x] = foldLanes(acc);
-        __syncthreads();
-        if (threadIdx.x >= C)
-          return 0.0;
-        double v[R];
+        using S = DotShape<C>;
+        u32 blk, j, nBlocks, nGroups, N;
+        int ty;
+        __device__ DotPlace(u32 N_, u32 B, u32 nBlocks_)
+          : nBlocks(nBlocks_), nGroups((u32)(((u64)N_ + DOT_LANES - 1) / DOT_LANES)), N(N_),
+            ty(threadIdx.x / C)
+        {
+          const u32 nCh = (B + C - 1) / C;
+          blk           = blockIdx.x / nCh;
+          j             = (blockIdx.x - blk * nCh) * C + threadIdx.x % C;
+        }
+        // calls load(t, row) for four rows, then use(t, lane, row)
+        template <class Load, class Use>
+        __device__ inline void rows(Load load, Use use) const
+        {
+          for (u32 g = blk; g < nGroups; g += S::STEP / S::U * nBlocks)
+#pragma unroll
+            for (int f = 0; f < S::STEP; f += 4)
+              {
+                u32  row[4];
+                bool ok[4];
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                  {
+                    const u32 gt = g + (f + t) / S::U * nBlocks;
+                    row[t]       = gt * DOT_LANES + ty + (f + t) % S::U * S::R;
+                    ok[t]        = gt < nGroups && row[t] < N;
+                  }
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                  if (ok[t])
+                    load(t, row[t]);
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                  if (ok[t])
+                    use(t, (f + t) % S::U, row[t]);
+              }
+        }
+      };
+      // a column's sum over the block from what the threads left in red, in the
+      // threads with ty == 0
+      template <int C>
+      __device__ inline double blockSum(const double *red)
+      {
+        constexpr int R = DotShape<C>::R;
+        double        v[R];
 #pragma unroll
         for (int q = 0; q < R; ++q)
           v[q] = red[q * C + threadIdx.x];
         return foldLanes(v);
       }
-
-      template <class T, int C>
-      __global__ __launch_bounds__(TPB) void colDotsK(const T *x, u32 ldx, const T *y, u32 ldy,
-                                                      u32 N, u32 B, u32 rowsPerBlock,
-                                                      double *partials)
+      // calls go(columns, workgroups) with the widest shape that leaves the GPU
+      // a workgroup per CU: wide ones read a row's lines whole, but a small vector
+      // has few blocks (N = 1331: 21).  16 columns at least: with 8 the update of
+      // 29 791 x 10 values took 8.4 us instead of 5.4
+      template <class Go>
+      void dotShape(u32 N, u32 B, Go go)
       {
-        using S          = DotShape<C>;
-        constexpr int R  = S::R, U = S::U;
-        const int     tx = threadIdx.x % C, ty = threadIdx.x / C;
-        __shared__ double red[TPB];
-        const u32 r0 = blockIdx.x * rowsPerBlock;
-        const u32 r1 = min(N, r0 + rowsPerBlock);
-        for (u32 j0 = 0; j0 < B; j0 += C)
+        const u32 nBlocks = dotBlocks(N);
+        u32       C       = B <= 8 ? 8 : B <= 16 ? 16 : B <= 32 ? 32 : 64;
+        while (C > 16 && (u64)nBlocks * ((B + C - 1) / C) < 256)
+          C /= 2;
+        const u64 grid = (u64)nBlocks * ((B + C - 1) / C);
+        DFX_REQUIRE(grid < (1ull << 31), "too many columns for the dots");
+        switch (C)
           {
-            const u32 j = j0 + tx;
-            double    acc[U]{};
-            if (j < B)
-              for (u32 i0 = r0 + ty; i0 < r1; i0 += S::STEP * R)
-#pragma unroll
-                for (int g = 0; g < S::STEP; g += 4)
-                  {
-                    T xv[4], yv[4];
-#pragma unroll
-                    for (int t = 0; t < 4; ++t)
-                      if (const u32 i = i0 + (g + t) * R; i < r1)
-                        xv[t] = x[(u64)i * ldx + j], yv[t] = y[(u64)i * ldy + j];
-#pragma unroll
-                    for (int t = 0; t < 4; ++t)
-                      if (i0 + (g + t) * R < r1)
-                        acc[(g + t) % U] = fma((double)xv[t], (double)yv[t], acc[(g + t) % U]);
-                  }
-            const double s = blockSum<C>(acc, red);
-            if (ty == 0 && j < B)
-              partials[(u64)blockIdx.x * B + j] = s;
-            __syncthreads();
+            case 8: return go(std::integral_constant<int, 8>{}, (unsigned)grid);
+            case 16: return go(std::integral_constant<int, 16>{}, (unsigned)grid);
+            case 32: return go(std::integral_constant<int, 32>{}, (unsigned)grid);
+            default: return go(std::integral_constant<int, 64>{}, (unsigned)grid);
           }
       }
 
-      // partials[i, j] = x_ij y_ij: rows whose dot is a partial sum of its own
+      // partials: column-major, nParts of them per column
+      template <class T, int C>
+      __global__ __launch_bounds__(TPB) void colDotsK(const T *x, u32 ldx, const T *y, u32 ldy,
+                                                      u32 N, u32 B, u32 nBlocks, u32 nParts,
+                                                      double *partials)
+      {
+        constexpr int U = DotShape<C>::U;
+        __shared__ double red[TPB];
+        const DotPlace<C> at(N, B, nBlocks);
+        const u32         j = at.j;
+        double            acc[U]{};
+        if (j < B)
+          {
+            T xv[4], yv[4];
+            at.rows([&](int t, u32 i) { xv[t] = x[(u64)i * ldx + j], yv[t] = y[(u64)i * ldy + j]; },
+                    [&](int t, int u, u32) { acc[u] = fma((double)xv[t], (double)yv[t], acc[u]); });
+          }
+        red[threadIdx.x] = foldLanes(acc);
+        __syncthreads();
+        if (at.ty == 0 && j < B)
+          partials[(u64)j * nParts + at.blk] = blockSum<C>(red);
+      }
+
+      // rows whose dot is a partial sum of its own, after `first` others
       __global__ void rowProductsK(const double *x, u32 ldx, const double *y, u32 ldy, u32 N,
-                                   u32 B, double *partials)
+                                   u32 B, u32 first, u32 nParts, double *partials)
       {
         const u64 n = (u64)N * B;
         for (u64 t = blockIdx.x * (u64)blockDim.x + threadIdx.x; t < n;
              t += (u64)gridDim.x * blockDim.x)
           {
-            const RC r  = rc(t, B);
-            partials[t] = x[(u64)r.i * ldx + r.j] * y[(u64)r.i * ldy + r.j];
+            const RC r = rc(t, B);
+            partials[(u64)r.j * nParts + first + r.i] =
+              x[(u64)r.i * ldx + r.j] * y[(u64)r.i * ldy + r.j];
           }
       }
 
@@ -297,68 +347,50 @@ namespace dfx
       //   xn = x + alpha p, r -= alpha w, and the partial sums of z.r and r.r
       // with z = d o r (alpha = zr / pw per column, formed here as cgAlphaK
       // does; z itself is formed again where it is used).
-      // Rows, lanes and sums follow colDotsK exactly (same blocks of rows,
-      // same lane order, same folds), and each element is the blocked
-      // axpby's / the diagonal scaling's expression, so every value is the
-      // separate launches' bit for bit.  partials: nBlocks x 2B (z.r in
-      // columns [0, B), r.r in [B, 2B)); N x B arrays with leading dimension B.
+      // Rows, lanes and sums follow colDotsK exactly, and each element is the
+      // blocked axpby's / the diagonal scaling's expression, so every value is the
+      // separate launches' bit for bit.  partials: those of z.r in columns
+      // [0, B), of r.r in [B, 2B); N x B arrays with leading dimension B.
       // Bound by memory: 4 reads and 2 writes per value (with z, a copy of x and
-      // 16 lanes for 8 columns it took 15.5 us at 117 649 x 8)
+      // 16 lanes for 8 columns it took 15.5 us at 117 649 x 8, now 9.1)
       template <int C>
       __global__ __launch_bounds__(TPB) void cgUpdateK(const double *x, double *xn, double *r,
                                                        const double *p, const double *w,
                                                        const double *d, const double *zr,
                                                        const double *pw, u32 N, u32 B,
-                                                       u32 rowsPerBlock, double *partials)
+                                                       u32 nBlocks, double *partials)
       {
-        using S          = DotShape<C>;
-        constexpr int R  = S::R, U = S::U;
-        const int     tx = threadIdx.x % C, ty = threadIdx.x / C;
+        constexpr int U = DotShape<C>::U;
         __shared__ double red[2][TPB];
-        const u32 r0 = blockIdx.x * rowsPerBlock;
-        const u32 r1 = min(N, r0 + rowsPerBlock);
-        for (u32 j0 = 0; j0 < B; j0 += C)
+        const DotPlace<C> at(N, B, nBlocks);
+        const u32         j = at.j;
+        double            accZ[U]{}, accR[U]{};
+        if (j < B)
           {
-            const u32 j = j0 + tx;
-            double    accZ[U]{}, accR[U]{};
-            if (j < B)
-              {
-                const double alpha = zr[j] / pw[j], nalpha = -zr[j] / pw[j];
-                for (u32 i0 = r0 + ty; i0 < r1; i0 += S::STEP * R)
-#pragma unroll
-                  for (int g = 0; g < S::STEP; g += 4)
-                    {
-                      double xv[4], pv[4], rv[4], wv[4], dv[4];
-#pragma unroll
-                      for (int t = 0; t < 4; ++t)
-                        if (const u32 i = i0 + (g + t) * R; i < r1)
-                          {
-                            const u64 o = (u64)i * B + j;
-                            xv[t] = x[o], pv[t] = p[o], rv[t] = r[o], wv[t] = w[o], dv[t] = d[i];
-                          }
-#pragma unroll
-                      for (int t = 0; t < 4; ++t)
-                        if (const u32 i = i0 + (g + t) * R; i < r1)
-                          {
-                            const int     u  = (g + t) % U;
-                            const u64     o  = (u64)i * B + j;
-                            const double  rn = axpbyOne<double>(1.0, 1.0, rv[t], 1.0, nalpha, wv[t]);
-                            const double  zn = dv[t] * rn;
-                            xn[o]   = axpbyOne<double>(1.0, 1.0, xv[t], 1.0, alpha, pv[t]);
-                            r[o]    = rn;
-                            accZ[u] = fma(zn, rn, accZ[u]);
-                            accR[u] = fma(rn, rn, accR[u]);
-                          }
-                    }
-              }
-            const double sz = blockSum<C>(accZ, red[0]), sr = blockSum<C>(accR, red[1]);
-            if (ty == 0 && j < B)
-              {
-                partials[(u64)blockIdx.x * 2 * B + j]     = sz;
-                partials[(u64)blockIdx.x * 2 * B + B + j] = sr;
-              }
-            __syncthreads();
+            const double alpha = zr[j] / pw[j], nalpha = -zr[j] / pw[j];
+            double       xv[4], pv[4], rv[4], wv[4], dv[4];
+            at.rows(
+              [&](int t, u32 i) {
+                const u64 o = (u64)i * B + j;
+                xv[t] = x[o], pv[t] = p[o], rv[t] = r[o], wv[t] = w[o], dv[t] = d[i];
+              },
+              [&](int t, int u, u32 i) {
+                const u64    o  = (u64)i * B + j;
+                const double rn = axpbyOne<double>(1.0, 1.0, rv[t], 1.0, nalpha, wv[t]);
+                const double zn = dv[t] * rn;
+                xn[o]   = axpbyOne<double>(1.0, 1.0, xv[t], 1.0, alpha, pv[t]);
+                r[o]    = rn;
+                accZ[u] = fma(zn, rn, accZ[u]);
+                accR[u] = fma(rn, rn, accR[u]);
+              });
           }
+        red[0][threadIdx.x] = foldLanes(accZ);
+        red[1][threadIdx.x] = foldLanes(accR);
+        __syncthreads();
+        // one sum by the first C threads, the other by the next C
+        if (const u32 jj = at.j; at.ty < 2 && jj < B)
+          partials[((u64)at.ty * B + jj) * nBlocks + at.blk] =
+            blockSum<C>(red[at.ty] - at.ty * C);
       }
 
       // partial sums of |a1 a_j x_ij + b1 b_j y_ij|^2 per column without
@@ -369,48 +401,27 @@ namespace dfx
       __global__ __launch_bounds__(TPB) void combNormsK(double a1, const double *a,
                                                         const double *x, double b1,
                                                         const double *b, const double *y, u32 N,
-                                                        u32 B, u32 rowsPerBlock, double *partials)
+                                                        u32 B, u32 nBlocks, double *partials)
       {
-        using S          = DotShape<C>;
-        constexpr int R  = S::R, U = S::U;
-        const int     tx = threadIdx.x % C, ty = threadIdx.x / C;
+        constexpr int U = DotShape<C>::U;
         __shared__ double red[TPB];
-        const u32 r0 = blockIdx.x * rowsPerBlock;
-        const u32 r1 = min(N, r0 + rowsPerBlock);
-        for (u32 j0 = 0; j0 < B; j0 += C)
+        const DotPlace<C> at(N, B, nBlocks);
+        const u32         j = at.j;
+        double            acc[U]{};
+        if (j < B)
           {
-            const u32 j = j0 + tx;
-            double    acc[U]{};
-            if (j < B)
-              {
-                const double aj = a[j], bj = b[j];
-                for (u32 i0 = r0 + ty; i0 < r1; i0 += S::STEP * R)
-#pragma unroll
-                  for (int g = 0; g < S::STEP; g += 4)
-                    {
-                      double xv[4], yv[4];
-#pragma unroll
-                      for (int t = 0; t < 4; ++t)
-                        if (const u32 i = i0 + (g + t) * R; i < r1)
-                          {
-                            const u64 o = (u64)i * B + j;
-                            xv[t] = x[o], yv[t] = y[o];
-                          }
-#pragma unroll
-                      for (int t = 0; t < 4; ++t)
-                        if (i0 + (g + t) * R < r1)
-                          {
-                            const int    u = (g + t) % U;
-                            const double v = axpbyOne<double>(a1, aj, xv[t], b1, bj, yv[t]);
-                            acc[u]         = fma(v, v, acc[u]);
-                          }
-                    }
-              }
-            const double s = blockSum<C>(acc, red);
-            if (ty == 0 && j < B)
-              partials[(u64)blockIdx.x * B + j] = s;
-            __syncthreads();
+            const double aj = a[j], bj = b[j];
+            double       xv[4], yv[4];
+            at.rows([&](int t, u32 i) { xv[t] = x[(u64)i * B + j], yv[t] = y[(u64)i * B + j]; },
+                    [&](int t, int u, u32) {
+                      const double v = axpbyOne<double>(a1, aj, xv[t], b1, bj, yv[t]);
+                      acc[u]         = fma(v, v, acc[u]);
+                    });
           }
+        red[threadIdx.x] = foldLanes(acc);
+        __syncthreads();
+        if (at.ty == 0 && j < B)
+          partials[(u64)j * nBlocks + at.blk] = blockSum<C>(red);
       }
 
       // one workgroup per column: thread t adds partials t, t + 256, ... in
@@ -418,10 +429,11 @@ namespace dfx
       // partial count depends on the rows only, so a column's result does not
       // depend on how many columns share the call).  Columns from hostFrom on
       // also go to host (pinned memory).  All latency: eight loads are in
-      // flight together, the tree's last six levels stay in one wave
-      // (1024 partials, 16 columns: 4.7 -> 4.06 us)
+      // flight together, the tree's last six levels stay in one wave, and a
+      // column's partials lie side by side (117 649 rows, 8 columns: the solve
+      // 5 % shorter than with a row of columns per block)
       __global__ __launch_bounds__(256) void colDotsFinalK(const double *partials, u32 nBlocks,
-                                                           u32 B, double *out, double *host,
+                                                           double *out, double *host,
                                                            u32 hostFrom)
       {
         __shared__ double red[256];
@@ -433,7 +445,7 @@ namespace dfx
 #pragma unroll
             for (u32 k = 0; k < 8; ++k)
               if (b + k * 256 < nBlocks)
-                v[k] = partials[(u64)(b + k * 256) * B + j];
+                v[k] = partials[(u64)j * nBlocks + b + k * 256];
 #pragma unroll
             for (u32 k = 0; k < 8; ++k)
               if (b + k * 256 < nBlocks)
@@ -824,27 +836,22 @@ namespace dfx
     void colDotsFinal(hipStream_t s, const double *partials, u32 nBlocks, u32 B, double *out,
                       double *host, u32 hostFrom)
     {
-      colDotsFinalK<<<B, 256, 0, s>>>(partials, nBlocks, B, out, host, hostFrom);
+      colDotsFinalK<<<B, 256, 0, s>>>(partials, nBlocks, out, host, hostFrom);
       checkLaunch("colDotsFinal");
     }
 
     namespace
     {
-      // pass 1 over x's rows; the number of partial sums per column
+      // pass 1 over the first N rows of x, the first of nParts partial sums
       template <class T>
-      u32 colDotsPartials(hipStream_t s, View<const T> x, View<const T> y, double *partials)
+      void colDotsPartials(hipStream_t s, View<const T> x, View<const T> y, u32 N, u32 nParts,
+                           double *partials)
       {
-        const u32 B = x.B, nBlocks = dotBlocks(x.N), rows = dotRows(x.N, nBlocks);
-        if (B <= 8)
-          colDotsK<T, 8><<<nBlocks, TPB, 0, s>>>(x.p, x.ld, y.p, y.ld, x.N, B, rows, partials);
-        else if (B <= 16)
-          colDotsK<T, 16><<<nBlocks, TPB, 0, s>>>(x.p, x.ld, y.p, y.ld, x.N, B, rows, partials);
-        else if (B <= 32)
-          colDotsK<T, 32><<<nBlocks, TPB, 0, s>>>(x.p, x.ld, y.p, y.ld, x.N, B, rows, partials);
-        else
-          colDotsK<T, 64><<<nBlocks, TPB, 0, s>>>(x.p, x.ld, y.p, y.ld, x.N, B, rows, partials);
+        dotShape(N, x.B, [&](auto c, unsigned grid) {
+          colDotsK<T, decltype(c)::value><<<grid, TPB, 0, s>>>(x.p, x.ld, y.p, y.ld, N, x.B,
+                                                               dotBlocks(N), nParts, partials);
+        });
         checkLaunch("colDots");
-        return nBlocks;
       }
     } // namespace
 
@@ -854,23 +861,23 @@ namespace dfx
     {
       if (!x.B)
         return;
-      const u32 nBlocks = colDotsPartials<T>(s, x, y, partials);
+      const u32 nBlocks = dotBlocks(x.N);
+      colDotsPartials<T>(s, x, y, x.N, nBlocks, partials);
       colDotsFinal(s, partials, nBlocks, x.B, out);
     }
 
     void colDotsApart(hipStream_t s, View<const double> x, View<const double> y, u32 nC,
                       double *partials, double *out)
     {
-      const u32 B = x.B, nE = x.N - nC;
+      const u32 B = x.B, nE = x.N - nC, nBlocks = dotBlocks(nC);
       if (!B)
         return;
-      const u32 nBlocks = colDotsPartials<double>(s, View<const double>{x.p, nC, B, x.ld},
-                                                  View<const double>{y.p, nC, B, y.ld}, partials);
+      colDotsPartials<double>(s, x, y, nC, nBlocks + nE, partials);
       if (nE)
         {
           rowProductsK<<<gridFor((u64)nE * B), TPB, 0, s>>>(
-            x.p + (u64)nC * x.ld, x.ld, y.p + (u64)nC * y.ld, y.ld, nE, B,
-            partials + (u64)nBlocks * B);
+            x.p + (u64)nC * x.ld, x.ld, y.p + (u64)nC * y.ld, y.ld, nE, B, nBlocks, nBlocks + nE,
+            partials);
           checkLaunch("rowProducts");
         }
       colDotsFinal(s, partials, nBlocks + nE, B, out);
@@ -886,15 +893,10 @@ namespace dfx
       DFX_REQUIRE(x.ld == B && y.ld == B && y.N == N && y.B == B,
                   "combination norms: contiguous multivectors of one shape expected");
       const u32 nBlocks = dotBlocks(N);
-      const u32 rows    = dotRows(N, nBlocks);
-      if (B <= 8)
-        combNormsK<8><<<nBlocks, TPB, 0, s>>>(a1, a, x.p, b1, b, y.p, N, B, rows, partials);
-      else if (B <= 16)
-        combNormsK<16><<<nBlocks, TPB, 0, s>>>(a1, a, x.p, b1, b, y.p, N, B, rows, partials);
-      else if (B <= 32)
-        combNormsK<32><<<nBlocks, TPB, 0, s>>>(a1, a, x.p, b1, b, y.p, N, B, rows, partials);
-      else
-        combNormsK<64><<<nBlocks, TPB, 0, s>>>(a1, a, x.p, b1, b, y.p, N, B, rows, partials);
+      dotShape(N, B, [&](auto c, unsigned grid) {
+        combNormsK<decltype(c)::value><<<grid, TPB, 0, s>>>(a1, a, x.p, b1, b, y.p, N, B, nBlocks,
+                                                            partials);
+      });
       checkLaunch("combNorms");
       colDotsFinal(s, partials, nBlocks, B, out);
     }
@@ -909,20 +911,11 @@ namespace dfx
         return;
       DFX_REQUIRE(x.ld == B && xn.ld == B && r.ld == B && p.ld == B && w.ld == B,
                   "CG update: contiguous multivectors expected");
-      // the partition of colDots
       const u32 nBlocks = dotBlocks(N);
-      const u32 rows    = dotRows(N, nBlocks);
-      auto go = [&](auto kern) {
-        kern<<<nBlocks, TPB, 0, s>>>(x.p, xn.p, r.p, p.p, w.p, d, zr, pw, N, B, rows, partials);
-      };
-      if (B <= 8)
-        go(cgUpdateK<8>);
-      else if (B <= 16)
-        go(cgUpdateK<16>);
-      else if (B <= 32)
-        go(cgUpdateK<32>);
-      else
-        go(cgUpdateK<64>);
+      dotShape(N, B, [&](auto c, unsigned grid) {
+        cgUpdateK<decltype(c)::value><<<grid, TPB, 0, s>>>(x.p, xn.p, r.p, p.p, w.p, d, zr, pw, N,
+                                                           B, nBlocks, partials);
+      });
       checkLaunch("cgUpdate");
       colDotsFinal(s, partials, nBlocks, 2 * B, zrrr, rrHost, B);
     }

@@ -32,24 +32,26 @@ namespace dfx
     void enrichedBlock(hipStream_t s, View<T> y, const double *E, View<const T> x,
                        u32 nC, u32 nE);
     // column dots (x_j . y_j) in FP64, deterministic two-pass; result to
-    // `out` (device, length B).  `partials` must hold >= 1024 * B doubles.
+    // `out` (device, length B).  `partials` must hold >= DOT_BLOCKS * B doubles.
     template <class T>
     void colDots(hipStream_t s, View<const T> x, View<const T> y, double *partials,
                  double *out);
 
-    // the second pass of the column dots: out[j] = sum of nBlocks partials; the
+    // the second pass of the column dots: out[j] = sum of column j's nBlocks
+    // partials (column-major); the
     // columns from hostFrom on also to host (pinned, coherent) where given
     void colDotsFinal(hipStream_t s, const double *partials, u32 nBlocks, u32 B, double *out,
                       double *host = nullptr, u32 hostFrom = 0);
-    constexpr u32 DOT_PARTIALS = 2048; // rows of partial sums a CG work buffer holds
-    // the column dots with every row from nC on (at most DOT_PARTIALS / 2) a
+    // partial sums per column that a CG work buffer holds
+    constexpr u32 DOT_PARTIALS = 2 * DOT_BLOCKS;
+    // the column dots with every row from nC on (at most DOT_BLOCKS) a
     // partial sum of its own: the bits of slotSumDot, any columns and strides
     void colDotsApart(hipStream_t s, View<const double> x, View<const double> y, u32 nC,
                       double *partials, double *out);
 
     // out[j] = sum_i (a1 a[j] x_ij + b1 b[j] y_ij)^2 without forming the
     // combination: the bits of the blocked axpby followed by colDots
-    // (partials: 1024 B doubles; out on the device)
+    // (partials: DOT_BLOCKS B doubles; out on the device)
     void combinationNorms(hipStream_t s, double a1, const double *a, View<const double> x,
                           double b1, const double *b, View<const double> y, double *partials,
                           double *out);

@@ -23,9 +23,9 @@ namespace dfx
   void colDotsView(dfx_ctx *ctx, View<const T> X, View<const T> Y, double *hostOut)
   {
     const u32 B = X.B;
-    ctx->reducePartials.ensure((size_t)1024 * B * sizeof(double) + B * sizeof(double));
+    ctx->reducePartials.ensure((size_t)DOT_BLOCKS * B * sizeof(double) + B * sizeof(double));
     double *part = ctx->reducePartials.as<double>();
-    double *out  = part + (size_t)1024 * B;
+    double *out  = part + (size_t)DOT_BLOCKS * B;
     k::colDots<T>(ctx->stream, X, Y, part, out);
     DFX_HIP(hipMemcpyAsync(hostOut, out, B * sizeof(double), hipMemcpyDeviceToHost,
                            ctx->stream));

@@ -714,9 +714,9 @@ namespace dfx
         }
       double *d = workDoubles(ctx, "rn.coef", 2 * (size_t)n);
       toDevice(ctx, d, h.data(), h.size());
-      ctx->reducePartials.ensure((size_t)1024 * n * sizeof(double) + n * sizeof(double));
+      ctx->reducePartials.ensure((size_t)DOT_BLOCKS * n * sizeof(double) + n * sizeof(double));
       double *part = ctx->reducePartials.as<double>();
-      double *out  = part + (size_t)1024 * n;
+      double *out  = part + (size_t)DOT_BLOCKS * n;
       k::combinationNorms(ctx->stream, 1.0, d, AX, 1.0, d + n, BX, part, out);
       DFX_HIP(hipMemcpyAsync(res, out, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
       DFX_HIP(hipStreamSynchronize(ctx->stream));
