@@ -210,11 +210,14 @@ namespace dfx
                 }
         sum[threadIdx.x] = foldLanes(acc);
         __syncthreads();
+        // the folds between the row threads, two at a time
 #pragma unroll
-        for (u32 h = R / 2; h > 0; h >>= 1)
+        for (u32 h = R / 2; h > 0; h /= 4)
           {
-            if (r < h && sub < G)
-              sum[threadIdx.x] += sum[threadIdx.x + h * P];
+            const u32 hh = h / 2;
+            vt       *v  = sum + threadIdx.x;
+            if (r < (hh ? hh : 1u) && sub < G)
+              v[0] = hh ? (v[0] + v[h * P]) + (v[hh * P] + v[(hh + h) * P]) : v[0] + v[h * P];
             __syncthreads();
           }
         if (on && r == 0)

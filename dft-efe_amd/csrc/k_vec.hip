@@ -218,72 +218,81 @@ namespace dfx
       }
 
       // pass 1 of the column dots in the order of dots.hpp.  A workgroup takes C
-      // columns of one block: C columns x R row threads of U lanes each
+      // columns of NB blocks: C columns x R row threads, each of U lanes of every
+      // block.  Two blocks for 8 columns, so that four rows of a thread are in
+      // flight together (117 649 rows, 1 column: update 9.1 -> 6.9 us)
       template <int C>
       struct DotShape
       {
-        static constexpr int R = TPB / C, U = DOT_LANES / R;
-        // rows a thread takes per turn of its loop, in batches of four whose
-        // loads are in flight together: the f-th is lane f % U of group f / U
-        static constexpr int STEP = U > 4 ? U : 4;
-        static_assert(R <= DOT_LANES && STEP % U == 0, "whole lanes");
+        static constexpr int R = TPB / C, U = DOT_LANES / R, NB = U < 4 ? 4 / U : 1;
+        static_assert(R <= DOT_LANES && NB * U % 4 == 0, "whole lanes, batches of four rows");
       };
-      // the workgroup's block and first column; one row of the block's turn at
-      // group g
       template <int C>
       struct DotPlace
       {
         using S = DotShape<C>;
-        u32 blk, j, nBlocks, nGroups, N;
+        u32 blk, j, nBlocks, nGroups, N; // the first block, this thread's column
         int ty;
         __device__ DotPlace(u32 N_, u32 B, u32 nBlocks_)
           : nBlocks(nBlocks_), nGroups((u32)(((u64)N_ + DOT_LANES - 1) / DOT_LANES)), N(N_),
             ty(threadIdx.x / C)
         {
-          const u32 nCh = (B + C - 1) / C;
-          blk           = blockIdx.x / nCh;
-          j             = (blockIdx.x - blk * nCh) * C + threadIdx.x % C;
+          const u32 nCh = (B + C - 1) / C, w = blockIdx.x / nCh;
+          blk           = w * S::NB;
+          j             = (blockIdx.x - w * nCh) * C + threadIdx.x % C;
         }
-        // calls load(t, row) for four rows, then use(t, lane, row)
+        // calls load(t, row) for four rows, then use(t, block, lane, row).  In
+        // place of a row that is not there the first one is loaded again, and not
+        // used: with a branch per load each waited for the one before
         template <class Load, class Use>
         __device__ inline void rows(Load load, Use use) const
         {
-          for (u32 g = blk; g < nGroups; g += S::STEP / S::U * nBlocks)
+          for (u32 g = blk; g < nGroups; g += nBlocks)
 #pragma unroll
-            for (int f = 0; f < S::STEP; f += 4)
+            for (int f = 0; f < S::NB * S::U; f += 4)
               {
                 u32  row[4];
                 bool ok[4];
 #pragma unroll
                 for (int t = 0; t < 4; ++t)
                   {
-                    const u32 gt = g + (f + t) / S::U * nBlocks;
-                    row[t]       = gt * DOT_LANES + ty + (f + t) % S::U * S::R;
-                    ok[t]        = gt < nGroups && row[t] < N;
+                    const u32 nb = (f + t) / S::U, u = (f + t) % S::U;
+                    row[t]       = (g + nb) * DOT_LANES + ty + u * S::R;
+                    ok[t]        = blk + nb < nBlocks && g + nb < nGroups && row[t] < N;
+                    row[t]       = ok[t] ? row[t] : t ? row[0] : N - 1;
                   }
 #pragma unroll
                 for (int t = 0; t < 4; ++t)
-                  if (ok[t])
-                    load(t, row[t]);
+                  load(t, row[t]);
 #pragma unroll
                 for (int t = 0; t < 4; ++t)
                   if (ok[t])
-                    use(t, (f + t) % S::U, row[t]);
+                    use(t, (f + t) / S::U, (f + t) % S::U, row[t]);
               }
         }
-      };
-      // a column's sum over the block from what the threads left in red, in the
-      // threads with ty == 0
-      template <int C>
-      __device__ inline double blockSum(const double *red)
-      {
-        constexpr int R = DotShape<C>::R;
-        double        v[R];
+        // the columns' sums over the blocks, M of them per column: every thread
+        // leaves its lanes' folds in LDS, the i-th set of C threads folds those of
+        // sum i / NB and block i % NB and calls put(sum, block, value)
+        template <int M, class Put>
+        __device__ inline void sums(double (&acc)[M][S::NB][S::U], u32 B, Put put) const
+        {
+          __shared__ double red[M][S::NB][TPB];
 #pragma unroll
-        for (int q = 0; q < R; ++q)
-          v[q] = red[q * C + threadIdx.x];
-        return foldLanes(v);
-      }
+          for (int m = 0; m < M; ++m)
+#pragma unroll
+            for (int nb = 0; nb < S::NB; ++nb)
+              red[m][nb][threadIdx.x] = foldLanes(acc[m][nb]);
+          __syncthreads();
+          const int m = ty / S::NB, nb = ty % S::NB;
+          if (m >= M || j >= B || blk + nb >= nBlocks)
+            return;
+          double v[S::R];
+#pragma unroll
+          for (int q = 0; q < S::R; ++q)
+            v[q] = red[m][nb][q * C + threadIdx.x % C];
+          put(m, blk + nb, foldLanes(v));
+        }
+      };
       // calls go(columns, workgroups) with the widest shape that leaves the GPU
       // a workgroup per CU: wide ones read a row's lines whole, but a small vector
       // has few blocks (N = 1331: 21).  16 columns at least: with 8 the update of
@@ -295,14 +304,18 @@ namespace dfx
         u32       C       = B <= 8 ? 8 : B <= 16 ? 16 : B <= 32 ? 32 : 64;
         while (C > 16 && (u64)nBlocks * ((B + C - 1) / C) < 256)
           C /= 2;
-        const u64 grid = (u64)nBlocks * ((B + C - 1) / C);
-        DFX_REQUIRE(grid < (1ull << 31), "too many columns for the dots");
+        auto launch = [&](auto c) {
+          constexpr u32 W = decltype(c)::value, NB = DotShape<W>::NB;
+          const u64     grid = (u64)((nBlocks + NB - 1) / NB) * ((B + W - 1) / W);
+          DFX_REQUIRE(grid < (1ull << 31), "too many columns for the dots");
+          go(c, (unsigned)grid);
+        };
         switch (C)
           {
-            case 8: return go(std::integral_constant<int, 8>{}, (unsigned)grid);
-            case 16: return go(std::integral_constant<int, 16>{}, (unsigned)grid);
-            case 32: return go(std::integral_constant<int, 32>{}, (unsigned)grid);
-            default: return go(std::integral_constant<int, 64>{}, (unsigned)grid);
+            case 8: return launch(std::integral_constant<int, 8>{});
+            case 16: return launch(std::integral_constant<int, 16>{});
+            case 32: return launch(std::integral_constant<int, 32>{});
+            default: return launch(std::integral_constant<int, 64>{});
           }
       }
 
@@ -312,21 +325,20 @@ namespace dfx
                                                       u32 N, u32 B, u32 nBlocks, u32 nParts,
                                                       double *partials)
       {
-        constexpr int U = DotShape<C>::U;
-        __shared__ double red[TPB];
+        using S = DotShape<C>;
         const DotPlace<C> at(N, B, nBlocks);
         const u32         j = at.j;
-        double            acc[U]{};
+        double            acc[1][S::NB][S::U]{};
         if (j < B)
           {
             T xv[4], yv[4];
             at.rows([&](int t, u32 i) { xv[t] = x[(u64)i * ldx + j], yv[t] = y[(u64)i * ldy + j]; },
-                    [&](int t, int u, u32) { acc[u] = fma((double)xv[t], (double)yv[t], acc[u]); });
+                    [&](int t, int nb, int u, u32) {
+                      acc[0][nb][u] = fma((double)xv[t], (double)yv[t], acc[0][nb][u]);
+                    });
           }
-        red[threadIdx.x] = foldLanes(acc);
-        __syncthreads();
-        if (at.ty == 0 && j < B)
-          partials[(u64)j * nParts + at.blk] = blockSum<C>(red);
+        at.sums(acc, B,
+                [&](int, u32 blk, double s) { partials[(u64)j * nParts + blk] = s; });
       }
 
       // rows whose dot is a partial sum of its own, after `first` others
@@ -360,11 +372,10 @@ namespace dfx
                                                        const double *pw, u32 N, u32 B,
                                                        u32 nBlocks, double *partials)
       {
-        constexpr int U = DotShape<C>::U;
-        __shared__ double red[2][TPB];
+        using S = DotShape<C>;
         const DotPlace<C> at(N, B, nBlocks);
         const u32         j = at.j;
-        double            accZ[U]{}, accR[U]{};
+        double            acc[2][S::NB][S::U]{}; // z.r, r.r
         if (j < B)
           {
             const double alpha = zr[j] / pw[j], nalpha = -zr[j] / pw[j];
@@ -374,23 +385,19 @@ namespace dfx
                 const u64 o = (u64)i * B + j;
                 xv[t] = x[o], pv[t] = p[o], rv[t] = r[o], wv[t] = w[o], dv[t] = d[i];
               },
-              [&](int t, int u, u32 i) {
+              [&](int t, int nb, int u, u32 i) {
                 const u64    o  = (u64)i * B + j;
                 const double rn = axpbyOne<double>(1.0, 1.0, rv[t], 1.0, nalpha, wv[t]);
                 const double zn = dv[t] * rn;
-                xn[o]   = axpbyOne<double>(1.0, 1.0, xv[t], 1.0, alpha, pv[t]);
-                r[o]    = rn;
-                accZ[u] = fma(zn, rn, accZ[u]);
-                accR[u] = fma(rn, rn, accR[u]);
+                xn[o]         = axpbyOne<double>(1.0, 1.0, xv[t], 1.0, alpha, pv[t]);
+                r[o]          = rn;
+                acc[0][nb][u] = fma(zn, rn, acc[0][nb][u]);
+                acc[1][nb][u] = fma(rn, rn, acc[1][nb][u]);
               });
           }
-        red[0][threadIdx.x] = foldLanes(accZ);
-        red[1][threadIdx.x] = foldLanes(accR);
-        __syncthreads();
-        // one sum by the first C threads, the other by the next C
-        if (const u32 jj = at.j; at.ty < 2 && jj < B)
-          partials[((u64)at.ty * B + jj) * nBlocks + at.blk] =
-            blockSum<C>(red[at.ty] - at.ty * C);
+        at.sums(acc, B, [&](int m, u32 blk, double s) {
+          partials[((u64)m * B + j) * nBlocks + blk] = s;
+        });
       }
 
       // partial sums of |a1 a_j x_ij + b1 b_j y_ij|^2 per column without
@@ -403,25 +410,22 @@ namespace dfx
                                                         const double *b, const double *y, u32 N,
                                                         u32 B, u32 nBlocks, double *partials)
       {
-        constexpr int U = DotShape<C>::U;
-        __shared__ double red[TPB];
+        using S = DotShape<C>;
         const DotPlace<C> at(N, B, nBlocks);
         const u32         j = at.j;
-        double            acc[U]{};
+        double            acc[1][S::NB][S::U]{};
         if (j < B)
           {
             const double aj = a[j], bj = b[j];
             double       xv[4], yv[4];
             at.rows([&](int t, u32 i) { xv[t] = x[(u64)i * B + j], yv[t] = y[(u64)i * B + j]; },
-                    [&](int t, int u, u32) {
+                    [&](int t, int nb, int u, u32) {
                       const double v = axpbyOne<double>(a1, aj, xv[t], b1, bj, yv[t]);
-                      acc[u]         = fma(v, v, acc[u]);
+                      acc[0][nb][u]  = fma(v, v, acc[0][nb][u]);
                     });
           }
-        red[threadIdx.x] = foldLanes(acc);
-        __syncthreads();
-        if (at.ty == 0 && j < B)
-          partials[(u64)j * nBlocks + at.blk] = blockSum<C>(red);
+        at.sums(acc, B,
+                [&](int, u32 blk, double s) { partials[(u64)j * nBlocks + blk] = s; });
       }
 
       // one workgroup per column: thread t adds partials t, t + 256, ... in
