@@ -78,7 +78,7 @@ namespace dfx
       // classical row and V columns (V: one 16-byte vector where widths and
       // addresses allow); most rows (a cell's interior) have one slot.  Bound by
       // memory: B values read per slot, written per row (p = 3, 16^3 cells, 40
-      // columns: FP32 68 MB in 14.8 us, FP64 with the residual step 205 MB in 35.6)
+      // columns: FP32 63 MB in 14.8 us, FP64 with the residual step 239 MB in 35.6)
       template <class T, int V, bool RES>
       __global__ __launch_bounds__(256) void slotSumK(
         const RowHead *__restrict__ heads, const u32 *__restrict__ rest,

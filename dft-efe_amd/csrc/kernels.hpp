@@ -38,8 +38,8 @@ namespace dfx
                  double *out);
 
     // the second pass of the column dots: out[j] = sum of column j's nBlocks
-    // partials (column-major); the
-    // columns from hostFrom on also to host (pinned, coherent) where given
+    // partials (column-major); the columns from hostFrom on also to host
+    // (pinned, coherent) where given
     void colDotsFinal(hipStream_t s, const double *partials, u32 nBlocks, u32 B, double *out,
                       double *host = nullptr, u32 hostFrom = 0);
     // partial sums per column that a CG work buffer holds

@@ -175,7 +175,9 @@ int dfx_op_create_cellwise(dfx_ctx *ctx, uint32_t nCells,
                            const double *cellMatrices, uint32_t nDofs,
                            uint32_t nClassical, dfx_constraints *cons,
                            uint32_t flags, dfx_op **op);
-/* replace the cell matrices (KohnShamOperatorContextFE::reinit, .t.cpp:1240-1310) */
+/* replace the cell matrices (KohnShamOperatorContextFE::reinit, .t.cpp:1240-1310).
+ * An update that fails for want of memory leaves the operator as it was; one
+ * that succeeds keeps the device addresses that a captured apply holds. */
 int dfx_op_update_cells(dfx_op *op, const double *cellMatrices);
 
 /* Diagonal (+ dense enriched block) operator
